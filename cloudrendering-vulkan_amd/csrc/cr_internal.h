@@ -59,7 +59,15 @@ struct PTArgs {
     float* records;         // record pass: [nFrames][H][W] records of 8 floats
     const float* points;    // continuation pass: records to continue
     float4* out;            // continuation pass: mean radiance per record
-    uint32_t spp;           // continuation pass: samples per record
+    uint32_t spp;           // continuation pass: samples per record (of this launch)
+    uint32_t nPoints;       // continuation pass: records
+    uint32_t sample0;       // continuation pass: index of the launch's first sample
+    // chunked passes: frames (or continuations) per work item, work items per
+    // pixel (or record), and where the samples go when there are several:
+    // [nFrames][H][W] (or [spp][nPoints])
+    uint32_t chunk, chunks;
+    float4* samples;
+    uint32_t blendBase;     // batched launch: first workgroup of this job in the blend kernel
     // scheduling (render pass): claim order of the tiles, and per-tile work of this launch
     const uint32_t* tileOrder;  // tile for each queue slot, or null (raster order)
     uint32_t* tileCost;         // lookups + brick visits per tile, accumulated, or null
@@ -76,12 +84,47 @@ struct BatchArgs {
     unsigned long long* counters;
 };
 
-// kern_pt.hip: a render of a.nFrames frames; launches of at most
-// PT_FEW_FRAMES frames use the instantiation with gated pixel claims
-// (kern_pt_few.hip), which is faster when each pixel carries little work.
+// kern_pt.hip: a render of a.nFrames frames; launches whose work items hold
+// at most PT_FEW_FRAMES frames use the instantiation with gated pixel claims
+// (kern_pt_few.hip), which is faster when an item carries little work.
 constexpr uint32_t PT_FEW_FRAMES = 16;
+// Work items of a chunked pass: at least this many per resident lane while
+// there are samples to make them of, each of at most PT_FEW_FRAMES samples.
+// Frames per work item of a chunked pass: at least PT_ITEMS_PER_LANE items per
+// resident lane while there are samples to make them of, each of at most
+// `most` samples.  Renders: chunks of 4 measured best where samples abound (a
+// 16-job batch: 125 ms with chunks of up to 16, 101 with 8, 85 with 4, 95 with
+// 1; 512x512 at 128 spp: 26.0, -, 20.6, 23.4), and 8 items per lane where they
+// do not (256x256 at 64 spp: 3.18 ms; with 4 items 3.47, with 32 3.32).
+// Record passes, whose samples are short, pay for the set-up of more items
+// (1080p at 32 spp, the whole learned render: 27.7 ms with 16, 29.0 with 4).
+constexpr uint64_t PT_ITEMS_PER_LANE = 8;
+constexpr uint32_t PT_CHUNK_RENDER = 4, PT_CHUNK_RECORD = 16;
+static_assert(PT_CHUNK_RENDER <= PT_FEW_FRAMES && PT_CHUNK_RECORD <= PT_FEW_FRAMES, "chunked items are few-frame items");
+inline uint32_t pt_chunk(uint64_t pixels, uint32_t samples, uint64_t lanes, uint32_t most)
+{
+    const uint64_t c = pixels * samples / (PT_ITEMS_PER_LANE * lanes);
+    return (uint32_t)(c < 1 ? 1 : (c > most ? most : c));
+}
+// Renders of several frames are chunked, except brick-DDA renders of images
+// with this many pixels or more per resident lane: their lanes have pixels
+// enough to balance, and the claims and stored samples cost more than they
+// bring (ms unchunked / chunked, 64 spp: 1 GiB grid at 256^2 45 / 5.8, 800x600
+// 44 / 24, 720p 54 / 43, 1080p with 256 bounces 334 / 360 at 256 spp; 128^3
+// grid at 1280x960 29 / 24.5, 1080p 83 / 77 at 64 spp and 302 / 300 at 256).
+// Global-majorant renders gain at every size (1080p 113 / 72, 4K 438 / 294).
+constexpr uint64_t PT_SPLIT_PIXELS_DDA = 6;
+// Samples stored by one chunked launch at most (4 GiB); more go in several
+// launches, each of which ends on its longest paths (16-job batch: 88.6 ms
+// with 1 GiB).
+constexpr uint64_t PT_SAMPLE_BUDGET = 1ull << 28;
 hipError_t launch_pt(const PTArgs& a, int dtype, int layout, int grid_blocks, hipStream_t s);
-int pt_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee, uint32_t n_frames);
+int pt_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee, uint32_t chunk);
+// The second half of a chunked launch: blend the stored samples into the
+// image(s), or sum the stored continuations (total: samples per record).
+hipError_t launch_pt_blend(const PTArgs& a, hipStream_t s);
+hipError_t launch_pt_blend_batch(const BatchArgs& b, uint32_t blocks, hipStream_t s);
+hipError_t launch_pt_sum(const PTArgs& a, uint32_t total, hipStream_t s);
 // kern_pt_few.hip
 hipError_t launch_pt_few(const PTArgs& a, int dtype, int layout, int grid_blocks, hipStream_t s);
 int pt_few_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee);

@@ -140,7 +140,7 @@ cr_status cr_destroy(cr_context* ctx)
     hipSetDevice(ctx->device);
     if (ctx->stream) hipStreamSynchronize(ctx->stream);
     void* bufs[] = {ctx->grid.data, ctx->grid.majorants, ctx->grid.skip, ctx->sv, ctx->image, ctx->dFrames, ctx->dQueue,
-                    ctx->tileCost, ctx->tileSort,
+                    ctx->tileCost, ctx->tileSort, ctx->ptSamples,
                     ctx->dCounters, ctx->dScalar};
     for (void* b : bufs)
         if (b) hipFree(b);
@@ -708,6 +708,36 @@ void fill_job_args(PTArgs& a, const DeviceGrid& g, const float* sv, const uint32
     const uint32_t tilesY = ((uint32_t)H + th - 1u) / th;
     a.totalIdx = a.tilesX * tilesY * 64u;
     a.base = 0;
+    a.chunk = n_frames;
+    a.chunks = 1;
+}
+
+// Work items of `chunk` frames instead of whole pixels, as long as their
+// number fits the queue's 32-bit counter (which idle lanes overrun a little).
+void set_chunk(PTArgs& a, uint32_t chunk)
+{
+    const uint32_t chunks = (a.nFrames + chunk - 1u) / chunk;
+    if (chunks <= 1 || (uint64_t)a.totalIdx * chunks >= (1ull << 31)) return;
+    a.chunk = chunk;
+    a.chunks = chunks;
+    a.totalIdx *= chunks;
+}
+
+// Scratch for `count` stored samples; false (and nothing allocated) when the
+// device has no room for it, where the caller renders without storing them.
+bool sample_buffer(float4** p, size_t* cap, uint64_t count)
+{
+    if (*p && *cap >= count) return true;
+    if (*p) hipFree(*p);
+    *p = nullptr;
+    *cap = 0;
+    if (hipMalloc((void**)p, count * sizeof(float4)) != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+        return false;
+    }
+    *cap = count;
+    return true;
 }
 
 cr_status fill_pt_args(cr_context* ctx, PTArgs& a, uint32_t n_frames)
@@ -738,36 +768,45 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
     PTArgs a;
     fill_pt_args(ctx, a, n_frames);
     const DeviceGrid& g = ctx->grid;
-    int per_cu = pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, n_frames);
-    int blocks = ctx->numCUs * per_cu;
-    uint32_t needed = (a.totalIdx + 255u) / 256u;
-    if ((uint32_t)blocks > needed) blocks = (int)needed;
-    if (ctx->ptBlocksOverride > 0) blocks = ctx->ptBlocksOverride;
+    // Work items of a few frames each, the samples stored and blended by a
+    // second kernel: whole pixels of a small image would leave lanes without
+    // work, and the last ones alone with a long pixel.
+    const uint64_t px = (uint64_t)ctx->W * (uint64_t)ctx->H;
+    const uint64_t lanes = (uint64_t)ctx->numCUs * 256u *
+                           (uint64_t)pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, 1);
+    uint32_t group = n_frames;  // frames per launch
+    if (n_frames > 1 && (ctx->ext.trackingMode != CR_TRACK_BRICK_DDA || px < PT_SPLIT_PIXELS_DDA * lanes)) {
+        group = (uint32_t)std::min<uint64_t>(n_frames, std::max<uint64_t>(1, PT_SAMPLE_BUDGET / px));
+        if (sample_buffer(&ctx->ptSamples, &ctx->ptSamplesCap, px * group)) a.samples = ctx->ptSamples;
+        else group = n_frames;
+    }
     CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
-    // Claim tiles in decreasing order of the previous render's per-tile work
-    // (same image shape), so the persistent grid drains on cheap tiles.  Only
-    // the schedule changes; every pixel's arithmetic is the same.
+    // Otherwise claim tiles in decreasing order of the previous render's
+    // per-tile work (same image shape), so the persistent grid drains on cheap
+    // tiles.  Only the schedule changes; every pixel's arithmetic is the same.
     const uint32_t nTiles = a.totalIdx / 64u;
-    if (ctx->tileN != nTiles || ctx->tileLog2W != a.tileLog2W || !ctx->tileCost) {
-        if (ctx->tileCost) hipFree(ctx->tileCost);
-        ctx->tileCost = nullptr;
-        ctx->tileCostValid = false;
-        CR_HIP(ctx, hipMalloc((void**)&ctx->tileCost, (size_t)nTiles * 4), "hipMalloc tile costs");
-        ctx->tileN = nTiles;
-        ctx->tileLog2W = a.tileLog2W;
+    if (!a.samples) {
+        if (ctx->tileN != nTiles || ctx->tileLog2W != a.tileLog2W || !ctx->tileCost) {
+            if (ctx->tileCost) hipFree(ctx->tileCost);
+            ctx->tileCost = nullptr;
+            ctx->tileCostValid = false;
+            CR_HIP(ctx, hipMalloc((void**)&ctx->tileCost, (size_t)nTiles * 4), "hipMalloc tile costs");
+            ctx->tileN = nTiles;
+            ctx->tileLog2W = a.tileLog2W;
+        }
+        if (ctx->tileCostValid) {
+            st = ensure_buffer(ctx, (void**)&ctx->tileSort, &ctx->tileSortCap,
+                               (size_t)nTiles * 16 + pt_order_counts(nTiles), "tile order");
+            if (st != CR_OK) return st;
+            uint32_t* k = ctx->tileSort;
+            CR_HIP(ctx, launch_tile_order(ctx->tileCost, nTiles, k, k + nTiles, k + 2 * (size_t)nTiles,
+                                          k + 3 * (size_t)nTiles, k + 4 * (size_t)nTiles, ctx->stream), "tile order");
+            a.tileOrder = k + nTiles;
+        }
+        CR_HIP(ctx, zero_async(ctx->tileCost, (size_t)nTiles * 4, ctx->stream), "zero tile costs");
+        a.tileCost = ctx->tileCost;
+        ctx->tileCostValid = true;
     }
-    if (ctx->tileCostValid) {
-        st = ensure_buffer(ctx, (void**)&ctx->tileSort, &ctx->tileSortCap,
-                           (size_t)nTiles * 16 + pt_order_counts(nTiles), "tile order");
-        if (st != CR_OK) return st;
-        uint32_t* k = ctx->tileSort;
-        CR_HIP(ctx, launch_tile_order(ctx->tileCost, nTiles, k, k + nTiles, k + 2 * (size_t)nTiles, k + 3 * (size_t)nTiles,
-                                      k + 4 * (size_t)nTiles, ctx->stream), "tile order");
-        a.tileOrder = k + nTiles;
-    }
-    CR_HIP(ctx, zero_async(ctx->tileCost, (size_t)nTiles * 4, ctx->stream), "zero tile costs");
-    a.tileCost = ctx->tileCost;
-    ctx->tileCostValid = true;
     if (ctx->ptEventsUsed >= 1024) {
         st = fold_pt_events(ctx);
         if (st != CR_OK) return st;
@@ -780,7 +819,20 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
     }
     const auto& ev = ctx->ptEvents[ctx->ptEventsUsed];
     CR_HIP(ctx, hipEventRecord(ev.first, ctx->stream), "event");
-    CR_HIP(ctx, launch_pt(a, g.dtype, g.layout, blocks, ctx->stream), "path tracer kernel");
+    for (uint32_t f0 = 0; f0 < n_frames; f0 += group) {
+        PTArgs b = a;
+        b.nFrames = std::min(group, n_frames - f0);
+        b.frames = a.frames + 2 * (size_t)f0;
+        b.chunk = b.nFrames;
+        if (a.samples) set_chunk(b, pt_chunk(px, b.nFrames, lanes, PT_CHUNK_RENDER));
+        int blocks = ctx->numCUs * pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, b.chunk);
+        const uint32_t needed = (b.totalIdx + 255u) / 256u;
+        if ((uint32_t)blocks > needed) blocks = (int)needed;
+        if (ctx->ptBlocksOverride > 0) blocks = ctx->ptBlocksOverride;
+        if (f0) CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
+        CR_HIP(ctx, launch_pt(b, g.dtype, g.layout, blocks, ctx->stream), "path tracer kernel");
+        if (b.samples) CR_HIP(ctx, launch_pt_blend(b, ctx->stream), "blend kernel");
+    }
     CR_HIP(ctx, hipEventRecord(ev.second, ctx->stream), "event");
     ctx->ptEventsUsed++;
     return CR_OK;

@@ -81,6 +81,9 @@ struct cr_context {
     size_t tileSortCap = 0;
     uint32_t tileN = 0, tileLog2W = 0;
     bool tileCostValid = false;
+    // samples of a chunked render or continuation pass (at most PT_SAMPLE_BUDGET)
+    float4* ptSamples = nullptr;
+    size_t ptSamplesCap = 0;
     uint32_t ptTileLog2W = 3;                  // 8x8 pixel tiles
 
     // bumped by every change to what a render reads (grid, uniforms, shadow volume)
@@ -111,6 +114,8 @@ void fill_job_args(PTArgs& a, const DeviceGrid& g, const float* sv, const uint32
                    const cr_camera_properties& cam, const cr_cloud_properties& cloud, const cr_parameters& params,
                    const cr_shadow_volume_properties& svp, const cr_render_ext& ext, const int32_t* frames,
                    uint32_t n_frames, float* image, int W, int H, uint32_t tileLog2W);
+void set_chunk(PTArgs& a, uint32_t chunk);
+bool sample_buffer(float4** p, size_t* cap, uint64_t count);
 cr_status fold_pt_events(cr_context* ctx);
 cr_status majorants_build(cr_context* ctx, DeviceGrid& g, int mb);
 void ppb_free(cr_context* ctx);

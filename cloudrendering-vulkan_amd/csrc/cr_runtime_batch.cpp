@@ -7,8 +7,14 @@
 // batch of 64 clouds never copies a grid.  The job table (one PTArgs per job,
 // ordered by decreasing frame count so the longest pixels start first) lives
 // in device memory and is copied to LDS by every workgroup of the launch; the
-// graph bakes in only the launch shape and the table's address, so frame lists
-// can change between replays without re-recording.
+// graph bakes in only the launch shapes and the tables' addresses, so frame
+// lists can change between replays without re-recording.
+//
+// A render is one or more launch groups.  Within a group every job's frames
+// are cut into chunks of a few frames per work item and the samples are stored;
+// a blend kernel then adds them to the images in frame order.  (With whole
+// pixels as work items the launch ended on a few lanes with 512-frame pixels
+// each.)  A group stores at most PT_SAMPLE_BUDGET samples.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,19 +49,33 @@ struct BatchJob {
     uint32_t nFrames = 0;
 };
 
+// One launch of a render or trial: its jobs' table entries [first, first + n).
+struct Group {
+    uint32_t first = 0, n = 0;
+    uint32_t total = 0;         // work items
+    uint32_t blendBlocks = 0;   // workgroups of the blend kernel
+    bool operator==(const Group& o) const
+    {
+        return first == o.first && n == o.n && total == o.total && blendBlocks == o.blendBlocks;
+    }
+};
+
 struct Batch {
     std::vector<BatchJob> jobs;
     cr_batch_tuning tuning;
     int dtype = 0, layout = 0;
     uint32_t tracking = 0, nee = 0;
     PTArgs* dTable = nullptr;       // render table
+    size_t tableCap = 0;
     PTArgs* dTuneTable = nullptr;   // autotuner trial table
+    size_t tuneTableCap = 0;
     uint32_t* dQueue = nullptr;     // [0] render queue, [16] trial queue
     unsigned long long* dCounters = nullptr;   // [0..7] render, [8..15] trials
     float* dScratch = nullptr;      // trial images
     size_t scratchCap = 0;
-    uint32_t total = 0;
-    int blocks = 0;
+    float4* dSamples = nullptr;     // a launch group's samples
+    size_t samplesCap = 0;
+    std::vector<Group> groups;
     bool tableDirty = true, graphDirty = true;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -90,9 +110,7 @@ cr_status ensure_batch(cr_context* ctx)
     if (ctx->batch) return CR_OK;
     Batch* b = new Batch();
     cr_batch_tuning_default(&b->tuning);
-    hipError_t e = hipMalloc((void**)&b->dTable, CR_BATCH_MAX_JOBS * sizeof(PTArgs));
-    if (e == hipSuccess) e = hipMalloc((void**)&b->dTuneTable, CR_BATCH_MAX_JOBS * sizeof(PTArgs));
-    if (e == hipSuccess) e = hipMalloc((void**)&b->dQueue, 32 * sizeof(uint32_t));
+    hipError_t e = hipMalloc((void**)&b->dQueue, 32 * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc((void**)&b->dCounters, 16 * sizeof(unsigned long long));
     if (e == hipSuccess) e = zero_async(b->dCounters, 16 * sizeof(unsigned long long), ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -116,40 +134,114 @@ std::vector<uint32_t> table_order(const Batch* b)
 
 uint32_t tile_log2(uint32_t tileWidth) { return tileWidth == 32 ? 5u : (tileWidth == 16 ? 4u : 3u); }
 
-// Job table for `which` jobs (table order); images at `images[k]` if given
-// (trial renders), each job's frame count divided by `frame_div` (at least 1
-// frame; 0 = all frames).
-std::vector<PTArgs> build_table(const Batch* b, const std::vector<uint32_t>& which, uint32_t tileWidth,
-                                const std::vector<float*>* images, uint32_t frame_div, uint32_t* total)
+int blocks_per_cu(const Batch* b, const cr_batch_tuning& t, uint32_t n_jobs)
 {
-    std::vector<PTArgs> t(which.size());
-    uint32_t base = 0;
-    for (size_t k = 0; k < which.size(); k++) {
-        const BatchJob& j = b->jobs[which[k]];
-        const uint32_t nf = frame_div ? std::max(1u, j.nFrames / frame_div) : j.nFrames;
-        fill_job_args(t[k], j.grid, j.sv, j.svDims, j.cam, j.cloud, j.params, j.svp, j.ext, j.dFrames, nf,
-                      images ? (*images)[k] : j.image, j.W, j.H, tile_log2(tileWidth));
-        t[k].base = base;
-        base += t[k].totalIdx;
-    }
-    *total = base;
-    return t;
+    if (t.blocksPerCU) return (int)t.blocksPerCU;
+    return pt_batch_blocks_per_cu(b->dtype, b->layout, b->tracking, b->nee, (int)t.blockThreads, n_jobs);
 }
 
-int launch_blocks(cr_context* ctx, const Batch* b, const cr_batch_tuning& t, uint32_t n_jobs, uint32_t total)
+// Job tables for `which` jobs (table order), group after group; images at
+// `images[k]` if given (trial renders), each job's frame count divided by
+// `frame_div` (at least 1 frame; 0 = all frames).  A job whose frames do not
+// fit the group's sample budget continues in the next group.  Without room
+// for the samples there is one group and lanes blend whole pixels.
+cr_status build_groups(cr_context* ctx, Batch* b, const std::vector<uint32_t>& which, const cr_batch_tuning& tuning,
+                       const std::vector<float*>* images, uint32_t frame_div, std::vector<PTArgs>* table,
+                       std::vector<Group>* groups)
 {
-    int per_cu = (int)t.blocksPerCU;
-    if (per_cu == 0)
-        per_cu = pt_batch_blocks_per_cu(b->dtype, b->layout, b->tracking, b->nee, (int)t.blockThreads, n_jobs);
-    int blocks = ctx->numCUs * per_cu;
-    const uint32_t needed = (total + t.blockThreads - 1u) / t.blockThreads;
+    table->clear();
+    groups->clear();
+    uint64_t all = 0;
+    auto frames_of = [&](size_t k) {
+        const uint32_t nf = b->jobs[which[k]].nFrames;
+        return frame_div ? std::max(1u, nf / frame_div) : nf;
+    };
+    for (size_t k = 0; k < which.size(); k++)
+        all += (uint64_t)b->jobs[which[k]].W * (uint64_t)b->jobs[which[k]].H * frames_of(k);
+    const uint64_t budget = std::min(all, PT_SAMPLE_BUDGET);
+    const bool store = sample_buffer(&b->dSamples, &b->samplesCap, budget);
+    const uint64_t lanes = (uint64_t)ctx->numCUs * tuning.blockThreads *
+                           (uint64_t)blocks_per_cu(b, tuning, (uint32_t)which.size());
+    Group g;
+    uint64_t used = 0;  // samples of the open group
+    auto close = [&]() {
+        if (g.n) groups->push_back(g);
+        g = Group();
+        g.first = (uint32_t)table->size();
+        used = 0;
+    };
+    for (size_t k = 0; k < which.size(); k++) {
+        const BatchJob& j = b->jobs[which[k]];
+        const uint64_t px = (uint64_t)j.W * (uint64_t)j.H;
+        const uint32_t nf = frames_of(k);
+        for (uint32_t f0 = 0; f0 < nf;) {
+            uint32_t take = nf - f0;
+            const bool fits = px <= budget;  // at least one frame of the job can be stored
+            if (store && fits) {
+                if (used + px > budget) close();
+                take = (uint32_t)std::min<uint64_t>(take, (budget - used) / px);
+            }
+            PTArgs a;
+            fill_job_args(a, j.grid, j.sv, j.svDims, j.cam, j.cloud, j.params, j.svp, j.ext, j.dFrames + 2 * (size_t)f0,
+                          take, images ? (*images)[k] : j.image, j.W, j.H, tile_log2(tuning.tileWidth));
+            if (store && fits && take > 1) set_chunk(a, pt_chunk(budget, 1, lanes, PT_CHUNK_RENDER));
+            if ((uint64_t)g.total + a.totalIdx >= (1ull << 31)) close();
+            a.base = g.total;
+            a.blendBase = g.blendBlocks;
+            if (a.chunks > 1) {
+                a.samples = b->dSamples + used;
+                used += px * take;
+                g.blendBlocks += (uint32_t)((px + 255) / 256);
+            }
+            g.total += a.totalIdx;
+            g.n++;
+            table->push_back(a);
+            f0 += take;
+            if (f0 < nf) close();  // a job's frames blend in order: one entry per group
+        }
+    }
+    close();
+    return CR_OK;
+}
+
+int launch_blocks(cr_context* ctx, const Batch* b, const cr_batch_tuning& t, const Group& g)
+{
+    int blocks = ctx->numCUs * blocks_per_cu(b, t, g.n);
+    const uint32_t needed = (g.total + t.blockThreads - 1u) / t.blockThreads;
     if ((uint32_t)blocks > needed) blocks = (int)needed;
     return blocks > 0 ? blocks : 1;
 }
 
-cr_status upload_table(cr_context* ctx, PTArgs* dst, const std::vector<PTArgs>& t)
+// The groups' launches: per group the queue reset, the path tracer, the blend.
+hipError_t enqueue_groups(cr_context* ctx, const Batch* b, const std::vector<Group>& groups, const PTArgs* table,
+                          const cr_batch_tuning& t, uint32_t* queue, unsigned long long* counters)
 {
-    CR_HIP(ctx, hipMemcpyAsync(dst, t.data(), t.size() * sizeof(PTArgs), hipMemcpyHostToDevice, ctx->stream),
+    hipError_t e = hipSuccess;
+    for (size_t k = 0; k < groups.size() && e == hipSuccess; k++) {
+        const Group& g = groups[k];
+        BatchArgs a;
+        a.jobs = table + g.first;
+        a.nJobs = g.n;
+        a.total = g.total;
+        a.queue = queue;
+        a.counters = counters;
+        e = zero_async(queue, 4, ctx->stream);
+        if (e == hipSuccess)
+            e = launch_pt_batch(a, b->dtype, b->layout, b->tracking, b->nee, launch_blocks(ctx, b, t, g), (int)t.blockThreads,
+                                ctx->stream);
+        if (e == hipSuccess) e = launch_pt_blend_batch(a, g.blendBlocks, ctx->stream);
+    }
+    return e;
+}
+
+// Copy a table to the device, growing its buffer; *moved: the buffer was replaced.
+cr_status upload_table(cr_context* ctx, PTArgs** dst, size_t* cap, const std::vector<PTArgs>& t, bool* moved)
+{
+    const PTArgs* before = *dst;
+    cr_status st = ensure_buffer(ctx, (void**)dst, cap, t.size() * sizeof(PTArgs), "job table");
+    if (st != CR_OK) return st;
+    if (moved) *moved = *dst != before;
+    CR_HIP(ctx, hipMemcpyAsync(*dst, t.data(), t.size() * sizeof(PTArgs), hipMemcpyHostToDevice, ctx->stream),
            "copy job table");
     CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync job table");
     return CR_OK;
@@ -169,17 +261,11 @@ cr_status trial(cr_context* ctx, Batch* b, const std::vector<uint32_t>& which, c
         images[k] = b->dScratch + off;
         off += (size_t)b->jobs[which[k]].W * b->jobs[which[k]].H * 4;
     }
-    uint32_t total = 0;
-    std::vector<PTArgs> table = build_table(b, which, t.tileWidth, &images, TRIAL_FRAME_DIV, &total);
-    cr_status st = upload_table(ctx, b->dTuneTable, table);
+    std::vector<PTArgs> table;
+    std::vector<Group> groups;
+    cr_status st = build_groups(ctx, b, which, t, &images, TRIAL_FRAME_DIV, &table, &groups);
+    if (st == CR_OK) st = upload_table(ctx, &b->dTuneTable, &b->tuneTableCap, table, nullptr);
     if (st != CR_OK) return st;
-    BatchArgs a;
-    a.jobs = b->dTuneTable;
-    a.nJobs = (uint32_t)which.size();
-    a.total = total;
-    a.queue = b->dQueue + 16;
-    a.counters = b->dCounters + 8;
-    const int blocks = launch_blocks(ctx, b, t, a.nJobs, total);
     hipEvent_t e0, e1;
     CR_HIP(ctx, hipEventCreate(&e0), "hipEventCreate");
     hipError_t e = hipEventCreate(&e1);
@@ -189,10 +275,8 @@ cr_status trial(cr_context* ctx, Batch* b, const std::vector<uint32_t>& which, c
     }
     float best = 1e30f;
     for (int r = 0; r <= reps && e == hipSuccess; r++) {
-        e = zero_async(a.queue, 4, ctx->stream);
-        if (e == hipSuccess) e = hipEventRecord(e0, ctx->stream);
-        if (e == hipSuccess)
-            e = launch_pt_batch(a, b->dtype, b->layout, b->tracking, b->nee, blocks, (int)t.blockThreads, ctx->stream);
+        e = hipEventRecord(e0, ctx->stream);
+        if (e == hipSuccess) e = enqueue_groups(ctx, b, groups, b->dTuneTable, t, b->dQueue + 16, b->dCounters + 8);
         if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
         float ms = 0.0f;
@@ -236,7 +320,7 @@ void batch_free(cr_context* ctx)
     if (!b) return;
     drop_graph(b);
     for (BatchJob& j : b->jobs) free_job(j);
-    void* bufs[] = {b->dTable, b->dTuneTable, b->dQueue, b->dCounters, b->dScratch};
+    void* bufs[] = {b->dTable, b->dTuneTable, b->dQueue, b->dCounters, b->dScratch, b->dSamples};
     for (void* p : bufs)
         if (p) hipFree(p);
     for (auto& ev : b->events) {
@@ -336,6 +420,9 @@ cr_status cr_batch_clear(cr_context* ctx)
     drop_graph(b);
     for (BatchJob& j : b->jobs) free_job(j);
     b->jobs.clear();
+    if (b->dSamples) hipFree(b->dSamples);
+    b->dSamples = nullptr;
+    b->samplesCap = 0;
     b->tableDirty = true;
     return CR_OK;
 }
@@ -419,29 +506,21 @@ cr_status cr_batch_render(cr_context* ctx)
     if (b->tableDirty) {
         // the graph may still be reading the table
         CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
-        const std::vector<uint32_t> order = table_order(b);
-        uint32_t total = 0;
-        std::vector<PTArgs> table = build_table(b, order, b->tuning.tileWidth, nullptr, 0, &total);
-        cr_status st = upload_table(ctx, b->dTable, table);
+        std::vector<PTArgs> table;
+        std::vector<Group> groups;
+        const float4* samples = b->dSamples;
+        bool moved = false;
+        cr_status st = build_groups(ctx, b, table_order(b), b->tuning, nullptr, 0, &table, &groups);
+        if (st == CR_OK) st = upload_table(ctx, &b->dTable, &b->tableCap, table, &moved);
         if (st != CR_OK) return st;
-        if (total != b->total) drop_graph(b);
-        b->total = total;
+        if (moved || samples != b->dSamples || groups != b->groups) drop_graph(b);
+        b->groups = groups;
         b->tableDirty = false;
     }
     if (b->graphDirty) {
         drop_graph(b);
-        BatchArgs a;
-        a.jobs = b->dTable;
-        a.nJobs = (uint32_t)b->jobs.size();
-        a.total = b->total;
-        a.queue = b->dQueue;
-        a.counters = b->dCounters;
-        b->blocks = launch_blocks(ctx, b, b->tuning, a.nJobs, a.total);
         CR_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed), "begin capture");
-        hipError_t e = zero_async(b->dQueue, 4, ctx->stream);
-        if (e == hipSuccess)
-            e = launch_pt_batch(a, b->dtype, b->layout, b->tracking, b->nee, b->blocks, (int)b->tuning.blockThreads,
-                                ctx->stream);
+        hipError_t e = enqueue_groups(ctx, b, b->groups, b->dTable, b->tuning, b->dQueue, b->dCounters);
         hipGraph_t g = nullptr;
         hipError_t e2 = hipStreamEndCapture(ctx->stream, &g);
         if (e == hipSuccess) e = e2;
@@ -532,6 +611,9 @@ cr_status cr_batch_autotune(cr_context* ctx, int tune_bricks, cr_batch_tuning* o
     if (!b || b->jobs.empty()) return fail(ctx, CR_ERR_STATE, "empty batch");
     hipSetDevice(ctx->device);
     CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
+    // trials share the render's sample buffer and may move it
+    b->tableDirty = true;
+    drop_graph(b);
     size_t px = 0;
     for (const BatchJob& j : b->jobs) px += (size_t)j.W * j.H;
     cr_status st = ensure_buffer(ctx, (void**)&b->dScratch, &b->scratchCap, px * 16, "autotune scratch images");

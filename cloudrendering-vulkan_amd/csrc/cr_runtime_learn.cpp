@@ -212,6 +212,7 @@ cr_status record_pass(cr_context* ctx, Learn* L, const cr_push_constants* frames
     CR_TRY(ensure_buffer(ctx, (void**)&L->records, &L->recordsCap, n * 32, "records"));
     PTArgs a;
     CR_TRY(fill_pt_args(ctx, a, n_frames));
+    set_chunk(a, pt_chunk((uint64_t)ctx->W * (uint64_t)ctx->H, n_frames, (uint64_t)pass_blocks(ctx, 0, ~0u) * 256u, PT_CHUNK_RECORD));
     a.records = L->records;
     a.counters = ctx->dCounters + 8;
     CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
@@ -221,7 +222,12 @@ cr_status record_pass(cr_context* ctx, Learn* L, const cr_push_constants* frames
     return CR_OK;
 }
 
-// Continuation pass over m device records into out (float4 per record).
+// Continuation pass over m device records into out (float4 per record).  The
+// samples of a record are independent until they are added, so a work item is
+// one sample, the samples are stored and a second kernel adds them in sample
+// order: 20 000 records filled 313 of the chip's 4096 waves and ran 256
+// samples each one after the other (c5-shaped collection of one cloud 110 ms,
+// now 9.2; chunks of two samples 10.2).
 cr_status continue_pass(cr_context* ctx, const float* pts, uint32_t m, uint32_t spp, float* out)
 {
     if (m == 0) return CR_OK;
@@ -229,12 +235,24 @@ cr_status continue_pass(cr_context* ctx, const float* pts, uint32_t m, uint32_t 
     CR_TRY(fill_pt_args(ctx, a, 0));
     a.points = pts;
     a.out = reinterpret_cast<float4*>(out);
-    a.spp = spp;
-    a.totalIdx = m;
+    a.nPoints = m;
     a.counters = ctx->dCounters + 8;
-    CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
-    CR_HIP(ctx, launch_pt_continue(a, ctx->grid.dtype, ctx->grid.layout, pass_blocks(ctx, 1, m), ctx->stream),
-           "continuation pass");
+    uint32_t group = spp;
+    if (spp > 1) {
+        group = (uint32_t)std::min<uint64_t>(spp, std::max<uint64_t>(1, PT_SAMPLE_BUDGET / m));
+        if (sample_buffer(&ctx->ptSamples, &ctx->ptSamplesCap, (uint64_t)m * group)) a.samples = ctx->ptSamples;
+        else group = spp;
+    }
+    for (uint32_t s0 = 0; s0 < spp; s0 += group) {
+        a.sample0 = s0;
+        a.spp = std::min(group, spp - s0);
+        a.chunk = a.samples ? 1u : a.spp;
+        a.totalIdx = m * ((a.spp + a.chunk - 1u) / a.chunk);
+        CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
+        CR_HIP(ctx, launch_pt_continue(a, ctx->grid.dtype, ctx->grid.layout, pass_blocks(ctx, 1, a.totalIdx), ctx->stream),
+               "continuation pass");
+        if (a.samples) CR_HIP(ctx, launch_pt_sum(a, spp, ctx->stream), "continuation sums");
+    }
     return CR_OK;
 }
 

@@ -11,10 +11,15 @@
 //    lanes, one lane advances the queue counter by the popcount, and each
 //    lane takes base + its rank among the idle lanes.  Claimed indices walk
 //    8x8 pixel tiles so neighbouring lanes trace neighbouring pixels.
-//  * Path regeneration: a lane renders all frames of its pixel back to back
-//    (frame f uses initializeRandom(seed_f * id) exactly as the reference),
-//    keeping the running mean in registers: 32 B of image traffic per pixel
-//    per launch.
+//  * Path regeneration: a lane renders the frames of its work item back to
+//    back (frame f uses initializeRandom(seed_f * id) exactly as the
+//    reference).  In a large render of many frames an item is a whole pixel,
+//    its running mean kept in registers: 32 B of image traffic per pixel per
+//    launch.  Otherwise it is a chunk of a few frames whose samples go to
+//    memory, and a blend kernel forms the mean in frame order (16 B written and
+//    read per sample, under 1% of the time of the paths): 256x256 pixels at 64
+//    spp on a 128^3 cloud went from 10.4 to 3.2 ms, as 65 536 lanes with 64
+//    frames each leave three quarters of the chip's wave slots empty.
 //  * Flattened state machine: every loop iteration performs at most one
 //    density lookup per lane (a delta-tracking step of the camera path, or a
 //    ratio-tracking step of a shadow ray); collisions, escapes, frame and
@@ -58,6 +63,7 @@ struct Lane {
     int32_t px, py;
     uint32_t id;
     uint32_t f;
+    uint32_t fEnd;  // chunked passes: end of the lane's frames (or continuations)
     // the pixel's camera ray, the same for every frame: its entry point into
     // the box (or the camera position when it misses the box) and direction
     f3 camPos, camDir;
@@ -354,15 +360,23 @@ enum { K_RENDER = 0, K_RECORD = 1, K_CONTINUE = 2, K_RENDER_FEW = 3 };
 
 constexpr bool renders(int kmode) { return kmode == K_RENDER || kmode == K_RENDER_FEW; }
 
-// Passes whose pixels carry little work (a few frames, camera paths cut at
-// their first collision, or the small jobs of a batched launch) claim pixels
-// only once CLAIM_MIN_LANES lanes of the wave (or all of its live ones) are
-// idle: lanes finish such pixels at scattered times, and the claim (queue
+// Passes whose work items carry little work (chunks of a few frames, camera
+// paths cut at their first collision, single continuations) claim items only
+// once CLAIM_MIN_LANES lanes of the wave (or all of its live ones) are
+// idle: lanes finish such items at scattered times, and the claim (queue
 // atomic, job lookup, pixel set-up, camera ray and box test) would otherwise
 // run for one or two lanes nearly every pass.  Single renders of many frames
 // per pixel claim as soon as one lane is idle.
-constexpr bool gated_claims(int kmode, bool batch) { return batch || kmode == K_RECORD || kmode == K_RENDER_FEW; }
+constexpr bool gated_claims(int kmode, bool batch) { return batch || kmode != K_RENDER; }
 constexpr uint32_t CLAIM_MIN_LANES = 16;
+
+// Passes whose work item is a chunk of a pixel's frames (or of a record's
+// continuations) rather than all of them: frames are independent until they
+// are blended, so a small image still fills the chip and no lane is left with
+// one long pixel at the end.  With a.samples set the pass stores every
+// sample's radiance and a second kernel adds them in the reference's order;
+// without it (one chunk per pixel) the lane blends as it goes.
+constexpr bool chunked(int kmode, bool batch) { return batch || kmode != K_RENDER; }
 
 __device__ __forceinline__ float* record_of(const cr::PTArgs& a, const Lane& L)
 {
@@ -379,10 +393,14 @@ __device__ __forceinline__ uint32_t continuation_seed(uint32_t s0, uint32_t s)
 }
 
 // End of a sample (frame or continuation).
-template <int KMODE>
+template <int KMODE, bool BATCH>
 __device__ __forceinline__ void finish_sample(const cr::PTArgs& a, Lane& L)
 {
-    if (renders(KMODE)) {
+    if (chunked(KMODE, BATCH) && KMODE != K_RECORD && a.samples) {
+        const size_t i = KMODE == K_CONTINUE ? (size_t)L.f * a.nPoints + (size_t)L.px
+                                             : ((size_t)L.f * (size_t)a.H + (size_t)L.py) * (size_t)a.W + (size_t)L.px;
+        a.samples[i] = make_float4(L.res.x, L.res.y, L.res.z, L.res.w);
+    } else if (renders(KMODE)) {
         blend(a, L);
     } else if (KMODE == K_CONTINUE) {
         L.acc.x = L.acc.x + L.res.x;
@@ -457,12 +475,14 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                 if (idx >= totalIdx) {
                     state = ST_DEAD;
                 } else if (KMODE == K_CONTINUE) {
-                    // one recorded collision; its samples start in the event loop
-                    L.px = (int32_t)idx;
+                    // a chunk of one recorded collision's samples, which start in the event loop
+                    const uint32_t ch = idx / a0.nPoints;
+                    L.px = (int32_t)(idx - ch * a0.nPoints);
                     L.py = 0;
                     L.id = 0;
                     L.acc.x = 0.0f; L.acc.y = 0.0f; L.acc.z = 0.0f; L.acc.w = 0.0f;
-                    L.f = 0;
+                    L.f = ch * a0.chunk;
+                    L.fEnd = min(a0.spp, L.f + a0.chunk);
                     state = ST_ACTIVE;
                     ev = EV_NONE;
                     L.mode = 0xFFu;
@@ -470,7 +490,13 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                     const uint32_t j = BATCH ? find_job(jobs, b.nJobs, idx) : 0u;
                     const cr::PTArgs& J = BATCH ? jobs[j] : a0;
                     const uint32_t local = BATCH ? idx - J.base : idx;
-                    const uint32_t slot = local >> 6, within = local & 63u;
+                    const uint32_t within = local & 63u;
+                    uint32_t slot = local >> 6, ch = 0;
+                    if (chunked(KMODE, BATCH)) {
+                        const uint32_t unit = slot;
+                        slot = unit / J.chunks;
+                        ch = unit - slot * J.chunks;
+                    }
                     // tiles in the order of the previous launch's cost, dearest first, so the
                     // queue ends on cheap tiles and the last lanes finish together
                     const uint32_t tile = J.tileOrder ? J.tileOrder[slot] : slot;
@@ -482,7 +508,7 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                         L.px = x;
                         L.py = y;
                         L.id = (uint32_t)x + (uint32_t)y * J.padded;
-                        if (renders(KMODE)) {
+                        if (renders(KMODE) && !(chunked(KMODE, BATCH) && J.samples)) {
                             float4 v = J.image[(size_t)y * J.W + x];
                             L.acc.x = v.x; L.acc.y = v.y; L.acc.z = v.z; L.acc.w = v.w;
                         }
@@ -495,11 +521,12 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                             L.camPos = L.camMiss ? cp : add(cp, mul(cd, tmax < tmin ? tmax : tmin));
                             L.camDir = cd;
                         }
+                        L.f = chunked(KMODE, BATCH) ? ch * J.chunk : 0u;
+                        if (chunked(KMODE, BATCH)) L.fEnd = min(J.nFrames, L.f + J.chunk);
                         if (J.nFrames > 0u) {
-                            L.seedNext = J.frames[0];
-                            L.countNext = J.frames[1];
+                            L.seedNext = J.frames[2 * L.f];
+                            L.countNext = J.frames[2 * L.f + 1];
                         }
-                        L.f = 0;
                         L.cost0 = c.lookups + c.brickVisits;
                         state = ST_ACTIVE;
                         ev = EV_NONE;
@@ -543,8 +570,10 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
             bool cam = false;  // batched: a camera ray, its box test after the shared reciprocal below
             if (needSample) {
                 needSample = false;
-                if (L.f >= (KMODE == K_CONTINUE ? a.spp : a.nFrames)) {
-                    if (renders(KMODE)) {
+                if (L.f >= (chunked(KMODE, BATCH) ? L.fEnd : a.nFrames)) {
+                    if (chunked(KMODE, BATCH) && KMODE != K_RECORD && a.samples) {
+                        // the samples are stored; the blend (or sum) kernel takes them in order
+                    } else if (renders(KMODE)) {
                         float4 o;
                         o.x = L.acc.x; o.y = L.acc.y; o.z = L.acc.z; o.w = L.acc.w;
                         a.image[(size_t)L.py * a.W + L.px] = o;
@@ -566,14 +595,16 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                     const float4 r0 = r[0], r1 = r[1];
                     if (!(r1.w > 0.5f)) {
                         // not a collision: the path escaped, nothing to continue
-                        a.out[L.px] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                        // (the sum kernel tests the flag itself)
+                        if (!a.samples) a.out[L.px] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                         state = ST_IDLE;
                         break;
                     }
                     L.pos = mk(r0.x, r0.y, r0.z);
                     L.dir = mk(r0.w, r1.x, r1.y);
                     const uint32_t s0 = __float_as_uint(r1.z);
-                    L.rng = L.f == 0 ? s0 : continuation_seed(s0, L.f);
+                    const uint32_t si = a.sample0 + L.f;
+                    L.rng = si == 0 ? s0 : continuation_seed(s0, si);
                     L.res.x = 0.0f; L.res.y = 0.0f; L.res.z = 0.0f; L.res.w = 0.0f;
                     L.thr = 1.0f;
                     L.bounces = 0;
@@ -692,7 +723,7 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                 fin = true;
             }
             if (fin) {
-                finish_sample<KMODE>(a, L);
+                finish_sample<KMODE, BATCH>(a, L);
                 L.f++;
                 ev = EV_NONE;
                 needSample = true;
