@@ -57,6 +57,14 @@ hipError_t launch_pack(uint32_t n, const uint4* meta, const float* lo, const flo
 hipError_t launch_treenodes(uint32_t n, const uint4* meta, const uint32_t* leafParent, const float* lo, const float* hi,
                             cr_tree_node* out, hipStream_t s);
 
+// What a photon path leaves of one interaction: the stretch of beam it starts
+// and its transmittance distances.
+struct BeamRecord {
+    float head[12];  // position, length, direction, path, data index and first segment on the path (as bits)
+    float tr[16];
+};
+static_assert(sizeof(BeamRecord) == 112, "BeamRecord is 112 B");
+
 // Beam producer: the scene a photon path sees.
 struct TraceArgs {
     const void* grid;
@@ -64,19 +72,22 @@ struct TraceArgs {
     cr_cloud_properties cloud;
     cr_parameters params;
     cr_beam_trace_params p;
-    // write pass only
+    uint32_t firstPath, nPaths;  // trace: the launch's paths; expand: paths that have offsets
+    BeamRecord* records;
+    unsigned long long* recordCount;  // records so far (may exceed recordCap; those past it are not stored)
+    uint64_t recordCap;
+    uint32_t* segCounts;         // trace: per path of the launch
+    uint32_t* dataCounts;
+    // expand
     const uint64_t* segOffsets;
     const uint64_t* dataOffsets;
     cr_photon_beam* beams;
     cr_photon_beam_data* data;
     uint64_t maxBeams;
     uint64_t maxData;
-    // count pass only
-    uint32_t* segCounts;
-    uint32_t* dataCounts;
 };
-hipError_t launch_trace_count(const TraceArgs& a, int dtype, int layout, hipStream_t s);
-hipError_t launch_trace_write(const TraceArgs& a, int dtype, int layout, hipStream_t s);
+hipError_t launch_trace(const TraceArgs& a, int dtype, int layout, hipStream_t s);
+hipError_t launch_trace_expand(const TraceArgs& a, uint64_t records, hipStream_t s);
 
 struct GatherArgs {
     const void* grid;

@@ -14,6 +14,16 @@ struct PpmGrid {
     int32_t nx, ny, nz, nbx, nby;
 };
 
+// A deposit as its path left it.
+struct PpmRecord {
+    float pos[3];
+    uint32_t path;
+    float dir[3];
+    uint32_t index;   // on its path
+    float power[4];
+};
+static_assert(sizeof(PpmRecord) == 48, "PpmRecord is three 16-B words");
+
 struct PpmTraceArgs {
     PpmGrid g;
     cr_cloud_properties cloud;
@@ -24,11 +34,14 @@ struct PpmTraceArgs {
     int32_t seed;
     float sunProbability;
     uint32_t maxCollisions;
-    uint32_t* counts;           // count pass: deposits per path
-    const uint32_t* offsets;    // write pass: first slot of each path
-    cr_photon* photons;         // write pass: deposits in emission order
-    uint32_t* cells;            //   their cells
-    uint32_t* order;            //   their slots (the sort's values)
+    uint32_t* counts;                 // trace: deposits per path
+    PpmRecord* records;
+    unsigned long long* recordCount;  // trace: records so far (may exceed recordCap; those past it are not stored)
+    uint64_t recordCap;
+    const uint32_t* offsets;          // place: first slot of each path
+    cr_photon* photons;               // place: deposits in emission order
+    uint32_t* cells;                  //   their cells
+    uint32_t* order;                  //   their slots (the sort's values)
 };
 
 struct PpmEstimateArgs {
@@ -53,7 +66,8 @@ struct PpmEstimateArgs {
     uint32_t padded;            // 32 * (W/32 + 1), the reference's pixel-id stride
 };
 
-hipError_t launch_ppm_trace(const PpmTraceArgs& a, bool write, int dtype, int layout, hipStream_t s);
+hipError_t launch_ppm_trace(const PpmTraceArgs& a, int dtype, int layout, hipStream_t s);
+hipError_t launch_ppm_place(const PpmTraceArgs& a, uint32_t records, hipStream_t s);
 hipError_t launch_ppm_runs(const uint32_t* keys, const uint32_t* vals, uint32_t n, uint32_t* start, uint32_t* arrivals,
                            const cr_photon* photons, cr_photon* sorted, float4* dirs, hipStream_t s);
 hipError_t launch_ppm_estimate(const PpmEstimateArgs& a, int dtype, int layout, hipStream_t s);

@@ -5,6 +5,7 @@
 // here capacities are explicit and exceeding one is an error.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -37,6 +38,12 @@ struct Ppb {
     size_t gcountersCap = 0;
     uint32_t* overflow = nullptr;
     size_t overflowCap = 0;
+    // beam producer: records of the last trace, per-path counts and offsets
+    BeamRecord* records = nullptr;
+    unsigned long long* recordCount = nullptr;
+    uint32_t* pathCounts = nullptr;
+    uint64_t* pathOffsets = nullptr;
+    size_t recordsCap = 0, recordCountCap = 0, pathCountsCap = 0, pathOffsetsCap = 0;
     bool built = false;
     uint32_t builtN = 0;
     hipEvent_t ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -51,7 +58,8 @@ void ppb_free(cr_context* ctx)
     Ppb* p = ctx->ppb;
     if (!p) return;
     void* bufs[] = {p->beams, p->data, p->sorted, p->sortedOff, p->keys, p->vals, p->keysTmp, p->valsTmp, p->counts, p->meta,
-                    p->leafParent, p->arrivals, p->exits, p->lo, p->hi, p->trav, p->gcounters, p->overflow};
+                    p->leafParent, p->arrivals, p->exits, p->lo, p->hi, p->trav, p->gcounters, p->overflow, p->records,
+                    p->recordCount, p->pathCounts, p->pathOffsets};
     for (void* b : bufs)
         if (b) hipFree(b);
     for (hipEvent_t e : p->ev)
@@ -87,6 +95,8 @@ static cr_status ppb_get(cr_context* ctx, Ppb** out)
     do { cr_status _s = (call); if (_s != CR_OK) return _s; } while (0)
 
 static const uint32_t MAX_BEAMS = 1u << 28;
+static const uint64_t TRACE_PATHS = 1u << 18;            // photon paths per launch of the producer at most
+static const size_t TRACE_KEEP = (size_t)1 << 30;        // bytes of beam records kept between traces at most
 
 // Sort, tree and traversal buffers for n beams (grown, never shrunk).
 static cr_status lbvh_buffers(cr_context* ctx, Ppb* p, uint32_t n)
@@ -178,42 +188,93 @@ cr_status cr_ppb_trace_beams(cr_context* ctx, const cr_beam_trace_params* prm, u
     a.cloud = ctx->cloud;
     a.params = ctx->params;
     a.p = *prm;
-    uint32_t* counts = nullptr;
-    CR_HIP(ctx, hipMalloc((void**)&counts, (size_t)P * 8), "hipMalloc counts");
-    a.segCounts = counts;
-    a.dataCounts = counts + P;
-    hipError_t e = launch_trace_count(a, g.dtype, g.layout, ctx->stream);
-    std::vector<uint32_t> hc(2 * (size_t)P);
-    if (e == hipSuccess) e = hipMemcpyAsync(hc.data(), counts, (size_t)P * 8, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    hipFree(counts);
-    if (e != hipSuccess) return hip_fail(ctx, e, "trace count");
-    std::vector<uint64_t> off(2 * (size_t)P);
+    // Paths are traced in order, in launches, until they fill max_beams: the
+    // beams of later paths would not be kept.  The first launch takes as many
+    // as fill it if each leaves one box side of beam (and at least one wave per
+    // SIMD), the next ones go by what the paths so far left.
+    const float side = ((ctx->cloud.bounds[1][0] - ctx->cloud.bounds[0][0]) + (ctx->cloud.bounds[1][1] - ctx->cloud.bounds[0][1]) +
+                        (ctx->cloud.bounds[1][2] - ctx->cloud.bounds[0][2])) / 3.0f;
+    const double guess = std::max(1.0, (double)side / (double)prm->radius);
+    const uint64_t least = (uint64_t)ctx->numCUs * 16u;
+    std::vector<uint64_t> segOff, dataOff;
+    std::vector<uint32_t> hc;
     uint64_t sb = 0, sd = 0;
-    for (uint32_t i = 0; i < P; i++) {
-        off[i] = sb;
-        off[P + i] = sd;
-        if (sb < max_beams) sd += hc[P + i];  // data of paths that keep at least one beam
-        sb += hc[i];
+    uint32_t done = 0;
+    unsigned long long records = 0;
+    CR_TRY(ensure_buffer(ctx, (void**)&p->recordCount, &p->recordCountCap, 8, "record count"));
+    a.recordCount = p->recordCount;
+    CR_HIP(ctx, zero_async(p->recordCount, 8, ctx->stream), "zero record count");
+    while (done < P && sb < max_beams) {
+        const double perPath = done && sb ? (double)sb / (double)done : guess;
+        const uint64_t want = std::max<uint64_t>(least, (uint64_t)(1.25 * (double)(max_beams - sb) / perPath) + 1u);
+        const uint32_t n = (uint32_t)std::min<uint64_t>({want, (uint64_t)(P - done), TRACE_PATHS, sb || !done ? want : (uint64_t)done});
+        CR_TRY(ensure_buffer(ctx, (void**)&p->pathCounts, &p->pathCountsCap, (size_t)n * 8, "path counts"));
+        if (!p->records)
+            CR_TRY(ensure_buffer(ctx, (void**)&p->records, &p->recordsCap, ((size_t)n * 8 + 1024) * sizeof(BeamRecord), "beam records"));
+        a.firstPath = done;
+        a.nPaths = n;
+        a.segCounts = p->pathCounts;
+        a.dataCounts = p->pathCounts + n;
+        a.records = p->records;
+        a.recordCap = p->recordsCap / sizeof(BeamRecord);
+        CR_HIP(ctx, launch_trace(a, g.dtype, g.layout, ctx->stream), "beam trace");
+        hc.resize(2 * (size_t)n);
+        unsigned long long total = 0;
+        CR_HIP(ctx, hipMemcpyAsync(hc.data(), p->pathCounts, (size_t)n * 8, hipMemcpyDeviceToHost, ctx->stream), "copy counts");
+        CR_HIP(ctx, hipMemcpyAsync(&total, p->recordCount, 8, hipMemcpyDeviceToHost, ctx->stream), "copy record count");
+        CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "beam trace");
+        if (total > a.recordCap) {
+            // more records than there is room for: make room, keep those of
+            // the earlier launches and trace these paths again
+            BeamRecord* more = nullptr;
+            const size_t bytes = (size_t)(total + total / 2) * sizeof(BeamRecord);
+            hipError_t e = hipMalloc((void**)&more, bytes);
+            if (e != hipSuccess) return fail(ctx, CR_ERR_OUT_OF_MEMORY, std::string("hipMalloc beam records: ") + hipGetErrorString(e));
+            if (records) e = hipMemcpyAsync(more, p->records, (size_t)records * sizeof(BeamRecord), hipMemcpyDeviceToDevice, ctx->stream);
+            if (e == hipSuccess) e = hipMemcpyAsync(p->recordCount, &records, 8, hipMemcpyHostToDevice, ctx->stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+            if (e != hipSuccess) {
+                hipFree(more);
+                return hip_fail(ctx, e, "grow beam records");
+            }
+            hipFree(p->records);
+            p->records = more;
+            p->recordsCap = bytes;
+            continue;
+        }
+        records = total;
+        for (uint32_t i = 0; i < n; i++) {
+            segOff.push_back(sb);
+            dataOff.push_back(sd);
+            if (sb < max_beams) sd += hc[n + i];  // data of paths that keep at least one beam
+            sb += hc[i];
+        }
+        done += n;
     }
     const uint64_t nb = sb < max_beams ? sb : max_beams;
     const uint64_t nd = sd;
     if (nd > MAX_BEAMS) return fail(ctx, CR_ERR_CAPACITY, "beam data exceeds 2^28 records");
     CR_TRY(ensure_buffer(ctx, (void**)&p->beams, &p->beamsCap, (size_t)nb * sizeof(cr_photon_beam), "beams"));
     CR_TRY(ensure_buffer(ctx, (void**)&p->data, &p->dataCap, (size_t)nd * sizeof(cr_photon_beam_data), "beam data"));
-    uint64_t* doff = nullptr;
-    CR_HIP(ctx, hipMalloc((void**)&doff, (size_t)P * 16), "hipMalloc offsets");
-    e = hipMemcpyAsync(doff, off.data(), (size_t)P * 16, hipMemcpyHostToDevice, ctx->stream);
-    a.segOffsets = doff;
-    a.dataOffsets = doff + P;
+    CR_TRY(ensure_buffer(ctx, (void**)&p->pathOffsets, &p->pathOffsetsCap, (size_t)done * 16, "path offsets"));
+    CR_HIP(ctx, hipMemcpyAsync(p->pathOffsets, segOff.data(), (size_t)done * 8, hipMemcpyHostToDevice, ctx->stream), "copy offsets");
+    CR_HIP(ctx, hipMemcpyAsync(p->pathOffsets + done, dataOff.data(), (size_t)done * 8, hipMemcpyHostToDevice, ctx->stream),
+           "copy offsets");
+    a.nPaths = done;
+    a.records = p->records;
+    a.segOffsets = p->pathOffsets;
+    a.dataOffsets = p->pathOffsets + done;
     a.beams = p->beams;
     a.data = p->data;
     a.maxBeams = nb;
     a.maxData = nd;
-    if (e == hipSuccess) e = launch_trace_write(a, g.dtype, g.layout, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    hipFree(doff);
-    if (e != hipSuccess) return hip_fail(ctx, e, "trace write");
+    CR_HIP(ctx, launch_trace_expand(a, records, ctx->stream), "beam expansion");
+    CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "beam expansion");
+    if (p->recordsCap > TRACE_KEEP) {
+        hipFree(p->records);
+        p->records = nullptr;
+        p->recordsCap = 0;
+    }
     p->n = (uint32_t)nb;
     p->nData = (uint32_t)nd;
     p->built = false;

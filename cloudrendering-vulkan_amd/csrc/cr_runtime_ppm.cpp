@@ -22,6 +22,9 @@ using namespace cr;
 struct Ppm {
     uint32_t *pathCounts = nullptr, *pathOffsets = nullptr;
     size_t pathCountsCap = 0, pathOffsetsCap = 0;
+    PpmRecord* records = nullptr;   // deposits as the paths left them
+    unsigned long long* recordCount = nullptr;
+    size_t recordsCap = 0, recordCountCap = 0;
     cr_photon *deposits = nullptr, *sorted = nullptr;
     size_t depositsCap = 0, sortedCap = 0;
     float4* dirs = nullptr;  // the sorted photons' unit directions
@@ -42,7 +45,7 @@ void ppm_free(cr_context* ctx)
 {
     Ppm* p = ctx->ppm;
     if (!p) return;
-    void* bufs[] = {p->pathCounts, p->pathOffsets, p->deposits, p->sorted, p->dirs, p->keys, p->vals, p->keysTmp,
+    void* bufs[] = {p->pathCounts, p->pathOffsets, p->records, p->recordCount, p->deposits, p->sorted, p->dirs, p->keys, p->vals, p->keysTmp,
                     p->valsTmp, p->sortCounts, p->arrivals, p->start, p->frames};
     for (void* b : bufs)
         if (b) hipFree(b);
@@ -59,6 +62,7 @@ static Ppm* ppm_get(cr_context* ctx)
 }
 
 static const uint32_t MAX_DEPOSITS = 1u << 28;
+static const size_t RECORDS_KEEP = (size_t)1 << 30;   // bytes of deposit records kept between traces at most
 static const uint64_t MAX_CELLS = 1ull << 27;
 
 extern "C" {
@@ -184,15 +188,30 @@ cr_status cr_ppm_trace(cr_context* ctx, int32_t seed, const cr_ppm_params* prm, 
     a.maxCollisions = prm->maxCollisions;
     a.counts = p->pathCounts;
     const DeviceGrid& g = ctx->grid;
-    CR_HIP(ctx, launch_ppm_trace(a, false, g.dtype, g.layout, s), "photon trace (count)");
     std::vector<uint32_t> counts(P), offsets(P);
-    CR_HIP(ctx, hipMemcpyAsync(counts.data(), p->pathCounts, (size_t)P * 4, hipMemcpyDeviceToHost, s), "copy counts");
-    CR_HIP(ctx, hipStreamSynchronize(s), "sync");
+    CR_TRY(ensure_buffer(ctx, (void**)&p->recordCount, &p->recordCountCap, 8, "record count"));
+    if (!p->records)
+        CR_TRY(ensure_buffer(ctx, (void**)&p->records, &p->recordsCap, ((size_t)P * 8 + 1024) * sizeof(PpmRecord), "deposit records"));
+    a.recordCount = p->recordCount;
+    unsigned long long total = 0;
+    for (;;) {
+        a.records = p->records;
+        a.recordCap = p->recordsCap / sizeof(PpmRecord);
+        CR_HIP(ctx, zero_async(p->recordCount, 8, s), "zero record count");
+        CR_HIP(ctx, launch_ppm_trace(a, g.dtype, g.layout, s), "photon trace");
+        CR_HIP(ctx, hipMemcpyAsync(counts.data(), p->pathCounts, (size_t)P * 4, hipMemcpyDeviceToHost, s), "copy counts");
+        CR_HIP(ctx, hipMemcpyAsync(&total, p->recordCount, 8, hipMemcpyDeviceToHost, s), "copy record count");
+        CR_HIP(ctx, hipStreamSynchronize(s), "sync");
+        if (total > MAX_DEPOSITS) return fail(ctx, CR_ERR_CAPACITY, "more than 2^28 photon deposits in one trace");
+        if (total <= a.recordCap) break;
+        // more deposits than there is room for: make room and trace again
+        CR_TRY(ensure_buffer(ctx, (void**)&p->records, &p->recordsCap, (size_t)(total + total / 4) * sizeof(PpmRecord),
+                             "deposit records"));
+    }
     uint64_t n = 0;
     for (uint32_t i = 0; i < P; i++) {
         offsets[i] = (uint32_t)n;
         n += counts[i];
-        if (n > MAX_DEPOSITS) return fail(ctx, CR_ERR_CAPACITY, "more than 2^28 photon deposits in one trace");
     }
     const uint32_t nd = (uint32_t)n;
     CR_TRY(ensure_buffer(ctx, (void**)&p->arrivals, &p->arrivalsCap, (size_t)nCells * 4, "cell arrivals"));
@@ -209,17 +228,21 @@ cr_status cr_ppm_trace(cr_context* ctx, int32_t seed, const cr_ppm_params* prm, 
         CR_TRY(ensure_buffer(ctx, (void**)&p->sortCounts, &p->sortCountsCap, (size_t)sort_counts_words(nd) * 4,
                              "sort histograms"));
         CR_HIP(ctx, hipMemcpyAsync(p->pathOffsets, offsets.data(), (size_t)P * 4, hipMemcpyHostToDevice, s), "copy offsets");
-        a.counts = nullptr;
         a.offsets = p->pathOffsets;
         a.photons = p->deposits;
         a.cells = p->keys;
         a.order = p->vals;
-        CR_HIP(ctx, launch_ppm_trace(a, true, g.dtype, g.layout, s), "photon trace (write)");
+        CR_HIP(ctx, launch_ppm_place(a, nd, s), "place deposits");
         CR_HIP(ctx, launch_radix_sort(p->keys, p->vals, p->keysTmp, p->valsTmp, p->sortCounts, nd, s), "sort by cell");
         CR_HIP(ctx, launch_ppm_runs(p->keys, p->vals, nd, p->start, p->arrivals, p->deposits, p->sorted, p->dirs, s),
                "cell runs");
     }
     CR_HIP(ctx, hipStreamSynchronize(s), "sync");
+    if (p->recordsCap > RECORDS_KEEP) {
+        hipFree(p->records);
+        p->records = nullptr;
+        p->recordsCap = 0;
+    }
     p->nDeposits = nd;
     p->nCells = (uint32_t)nCells;
     p->valid = true;

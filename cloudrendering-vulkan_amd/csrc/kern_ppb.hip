@@ -1,13 +1,14 @@
 // Photon-beam producer (shaders/PPB_PT.comp) and beam gather
 // (shaders/PPB_PE.comp) for gfx950.
 //
-// Producer: one lane per sun photon path.  The reference appends beams with
-// atomics (PPB_PT.comp:340, :381), so its output order depends on timing;
-// here a counting launch and a writing launch run the same path (same RNG
-// stream) and a scan between them gives every path its slots, so the beam
-// array is a pure function of the inputs.  Corrections: sun photons start on
-// the face the light enters and the face is chosen with if / else-if;
-// each segment keeps its offset along the parent beam in _padding_beam[0].
+// Producer: one row of 16 lanes per sun photon path (row_walk.h).  The
+// reference appends beams with atomics (PPB_PT.comp:340, :381), so its output
+// order depends on timing; here the paths leave records, a scan of their
+// counts gives every path its slots, and a second kernel writes beams and beam
+// data there, so the arrays are a pure function of the inputs.  Corrections:
+// sun photons start on the face the light enters and the face is chosen with
+// if / else-if; each segment keeps its offset along the parent beam in
+// _padding_beam[0].
 //
 // Gather: one lane per pixel; the traversal stack (64 entries, the
 // reference's depth, PPB_PE.comp:414) lives in LDS but for its deepest entries; nodes are 64-B records
@@ -19,6 +20,7 @@
 // full size to intersectBox, PPB_PE.comp:424-431).
 #include "cr_device.h"
 #include "cr_internal_ppb.h"
+#include "row_walk.h"
 
 using namespace crd;
 
@@ -66,18 +68,44 @@ __device__ __forceinline__ uint32_t morton30(f3 c, const float* b0, const float*
     return (expand_bits10(q[0]) << 2) + (expand_bits10(q[1]) << 1) + expand_bits10(q[2]);
 }
 
-template <typename T, int LAYOUT, bool WRITE>
+// generateSunRay's power of every photon — PPB_PT.comp:396-430 (corrected);
+// `total` is the box's area seen from the sun.
+__device__ __forceinline__ float photon_power(const cr::TraceArgs& a, float total)
+{
+    const float pdf = fdiv(1.0f, total);
+    return fdiv(1.0f * a.p.lightIntensity, (float)a.p.numPaths * pdf);
+}
+
+struct SunFaces { float ax, ay, az, total; };
+
+__device__ __forceinline__ SunFaces sun_faces(const cr::TraceArgs& a)
+{
+    const float* b0 = a.cloud.bounds[0];
+    const float* b1 = a.cloud.bounds[1];
+    const f3 L = ld3(a.p.lightDirection);
+    const float dx = b1[0] - b0[0], dy = b1[1] - b0[1], dz = b1[2] - b0[2];
+    SunFaces s;
+    s.ax = (dz * dy) * fabsf(L.x);
+    s.ay = (dx * dz) * fabsf(L.y);
+    s.az = (dy * dx) * fabsf(L.z);
+    s.total = (s.ax + s.ay) + s.az;
+    return s;
+}
+
+// Paths firstPath .. firstPath + nPaths - 1, one per row of 16 lanes.  Every
+// interaction (a stretch of beam between two collisions, or to the box's edge)
+// becomes a record in an arbitrary slot of a.records; segCounts and dataCounts
+// get the path's totals.  c3's trace: the paths that fill 2^22 beams took 25.6
+// ms when one lane walked each path, once to count and once more to write, and
+// every path of the call was counted.
+template <typename T, int LAYOUT>
 __global__ void __launch_bounds__(256) trace_kernel(cr::TraceArgs a)
 {
-    const uint32_t id = blockIdx.x * 256 + threadIdx.x;
-    if (id >= a.p.numPaths) return;
+    const uint32_t local = blockIdx.x * (256 / ROW) + threadIdx.x / ROW;
+    if (local >= a.nPaths) return;
+    const uint32_t id = a.firstPath + local;
+    const RowLane R;
     uint32_t segCount = 0, dataCount = 0;
-    uint64_t segBase = 0, dataBase = 0;
-    if (WRITE) {
-        segBase = a.segOffsets[id];
-        dataBase = a.dataOffsets[id];
-        if (segBase >= a.maxBeams) return;
-    }
     const cr_cloud_properties& cp = a.cloud;
     if (cp.densityScaling > 0.0f) {
         const float* b0 = cp.bounds[0];
@@ -85,100 +113,113 @@ __global__ void __launch_bounds__(256) trace_kernel(cr::TraceArgs a)
         uint32_t rng;
         xs_init(rng, (uint32_t)a.p.seed * id);
         const f3 L = ld3(a.p.lightDirection);
-        // generateSunRay — PPB_PT.comp:396-430 (corrected)
-        const float dx = b1[0] - b0[0], dy = b1[1] - b0[1], dz = b1[2] - b0[2];
-        const float ax = (dz * dy) * fabsf(L.x), ay = (dx * dz) * fabsf(L.y), az = (dy * dx) * fabsf(L.z);
-        const float total = (ax + ay) + az;
-        const float sel = xs_float(rng) * total;
+        const SunFaces F = sun_faces(a);
+        const float sel = xs_float(rng) * F.total;
         const f3 c1 = mk(L.x > 0.0f ? b0[0] : b1[0], L.y > 0.0f ? b0[1] : b1[1], L.z > 0.0f ? b0[2] : b1[2]);
         f3 pos;
         {
             const float u = xs_float(rng), v = xs_float(rng);
-            if (sel < ax) pos = mk(c1.x, b0[1] * (1.0f - u) + b1[1] * u, b0[2] * (1.0f - v) + b1[2] * v);
-            else if (sel < ax + ay) pos = mk(b0[0] * (1.0f - u) + b1[0] * u, c1.y, b0[2] * (1.0f - v) + b1[2] * v);
+            if (sel < F.ax) pos = mk(c1.x, b0[1] * (1.0f - u) + b1[1] * u, b0[2] * (1.0f - v) + b1[2] * v);
+            else if (sel < F.ax + F.ay) pos = mk(b0[0] * (1.0f - u) + b1[0] * u, c1.y, b0[2] * (1.0f - v) + b1[2] * v);
             else pos = mk(b0[0] * (1.0f - u) + b1[0] * u, b0[1] * (1.0f - v) + b1[1] * v, c1.z);
         }
-        const float pdf = fdiv(1.0f, total);
-        const float power = fdiv(1.0f * a.p.lightIntensity, (float)a.p.numPaths * pdf);
         f3 dir = L;
         const float r = a.p.radius;
         const float sigmaBar = fdiv(cp.maxExtinction * cp.densityScaling, cp.baseScaling);
         const float absorption = 1.0f - a.p.albedo;
-        for (uint32_t it = 0; it < a.p.maxInteractions; it++) {
+        bool alive = a.p.maxInteractions > 0u;
+        float len = 0.0f, tr = 0.0f, t = 0.0f;
+        uint32_t walk = 0, rounds = 0;  // walk 0..15: transmittance distances, 16: the next collision
+        if (alive) {
             float tmin = 0.0f, tmax = 0.0f;
-            if (!intersect_box(b0, b1, pos, dir, tmin, tmax)) break;
-            const f3 exitp = add(pos, mul(dir, tmax));
-            const float len = length(sub(pos, exitp));
-            const uint64_t di = dataBase + dataCount;
-            dataCount++;
-            // 16 transmittance distances — PPB_PT.comp:343-374
-            float tr[16];
-#pragma unroll 1
-            for (int s = 0; s < 16; s++) {
-                float t = 0.0f;
-                for (uint32_t step = 0; step < TRACK_CEILING; step++) {
-                    const float zeta = xs_float(rng);
-                    t = t + fdiv(-crd_logf(zeta), sigmaBar);
-                    if (!(t <= len)) break;
-                    const f3 cur = add(pos, mul(dir, t));
-                    const float e = cloud_at<T, LAYOUT>(a.grid, a.nx, a.ny, a.nz, a.nbx, a.nby, cp, cur);
-                    const float xi = xs_float(rng);
-                    if (xi < fdiv(e, cp.maxExtinction)) break;
-                }
-                if (WRITE) tr[s] = t;
-            }
-            if (WRITE && di < a.maxData) {
-                cr_photon_beam_data D;
-                D.power[0] = D.power[1] = D.power[2] = D.power[3] = power;
+            alive = intersect_box(b0, b1, pos, dir, tmin, tmax);
+            len = length(sub(pos, add(pos, mul(dir, tmax))));
+        }
+        while (alive) {
+            bool hit = false;
+            bool end = row_walk(R, sigmaBar, cp.maxExtinction, len, t, rng, hit, [&](float d) {
+                return cloud_at<T, LAYOUT>(a.grid, a.nx, a.ny, a.nz, a.nbx, a.nby, cp, add(pos, mul(dir, d)));
+            });
+            if (++rounds == TRACK_CEILING / ROW) end = true;
+            if (!end) continue;
+            rounds = 0;
+            if (walk < 16u) {
+                // 16 transmittance distances — PPB_PT.comp:343-374
+                if (R.i == walk) tr = t;
+                t = 0.0f;
+                if (++walk < 16u) continue;
+                const uint32_t segs = (uint32_t)fdiv(len, r) + 1u;
+                const unsigned long long slot = row_slot(R, a.recordCount);
+                if (slot < a.recordCap) {
+                    cr::BeamRecord& rec = a.records[slot];
+                    rec.tr[R.i] = tr;
+                    const float w[ROW] = {pos.x, pos.y, pos.z, len, dir.x, dir.y, dir.z, __uint_as_float(id),
+                                          __uint_as_float(dataCount), __uint_as_float(segCount)};
+                    float mine = w[0];
 #pragma unroll
-                for (int s = 0; s < 16; s++) D.trDistances[s] = tr[s];
-                a.data[di] = D;
-            }
-            const uint32_t segs = (uint32_t)fdiv(len, r) + 1u;
-            const float segSize = fdiv(len, (float)segs);
-            if (WRITE) {
-                for (uint32_t i = 0; i < segs; i++) {
-                    const uint64_t bi = segBase + segCount + i;
-                    if (bi >= a.maxBeams) break;
-                    const float off = (float)i * segSize;
-                    const f3 st = add(pos, mul(dir, off));
-                    const f3 en = add(st, mul(dir, segSize));
-                    cr_photon_beam B;
-                    B.startPos[0] = st.x; B.startPos[1] = st.y; B.startPos[2] = st.z;
-                    B.endPos[0] = en.x; B.endPos[1] = en.y; B.endPos[2] = en.z;
-                    B.radius = r;
-                    B.mortonCode = morton30(mk(fdiv(st.x + en.x, 2.0f), fdiv(st.y + en.y, 2.0f), fdiv(st.z + en.z, 2.0f)), b0, b1);
-                    B.dataIdx = (uint32_t)di;
-                    B._padding_beam[0] = __float_as_uint(off);
-                    B._padding_beam[1] = 0u;
-                    B._padding_beam[2] = 0u;
-                    a.beams[bi] = B;
+                    for (int k = 1; k < 10; k++) mine = R.i == (uint32_t)k ? w[k] : mine;
+                    if (R.i < 10u) rec.head[R.i] = mine;
                 }
+                dataCount++;
+                segCount += segs;
+                continue;
             }
-            segCount += segs;
             // next real collision — PPB_PT.comp:473-494
-            float t = 0.0f;
-            f3 cur = pos;
-            bool left = true;
-            for (uint32_t step = 0; step < TRACK_CEILING; step++) {
-                const float zeta = xs_float(rng);
-                t = t + fdiv(-crd_logf(zeta), sigmaBar);
-                if (!(t <= len)) { left = true; break; }
-                cur = add(pos, mul(dir, t));
-                const float e = cloud_at<T, LAYOUT>(a.grid, a.nx, a.ny, a.nz, a.nbx, a.nby, cp, cur);
-                const float xi = xs_float(rng);
-                if (xi < fdiv(e, cp.maxExtinction)) { left = false; break; }
-            }
-            if (left) break;
-            pos = cur;
+            if (!hit) break;
+            pos = add(pos, mul(dir, t));
+            t = 0.0f;
+            walk = 0;
             const float xi = xs_float(rng);
             if (!(xi > absorption)) break;
             dir = scatter_norm(a.params, dir, rng);
+            if (dataCount >= a.p.maxInteractions) break;
+            float tmin = 0.0f, tmax = 0.0f;
+            if (!intersect_box(b0, b1, pos, dir, tmin, tmax)) break;
+            len = length(sub(pos, add(pos, mul(dir, tmax))));
         }
     }
-    if (!WRITE) {
-        a.segCounts[id] = segCount;
-        a.dataCounts[id] = dataCount;
+    if (R.i == 0u) {
+        a.segCounts[local] = segCount;
+        a.dataCounts[local] = dataCount;
+    }
+}
+
+// One wave per record: its beam data and its segments, in the slots its path
+// and its place on the path give it.
+__global__ void __launch_bounds__(256) expand_kernel(cr::TraceArgs a, uint64_t nRecords)
+{
+    const uint64_t ri = (uint64_t)blockIdx.x * 4 + threadIdx.x / 64;
+    const uint32_t lane = threadIdx.x & 63u;
+    if (ri >= nRecords) return;
+    const cr::BeamRecord& rec = a.records[ri];
+    const uint32_t id = __float_as_uint(rec.head[7]);
+    if (id >= a.nPaths) return;
+    const uint64_t segBase = a.segOffsets[id];
+    if (segBase >= a.maxBeams) return;
+    const uint64_t di = a.dataOffsets[id] + __float_as_uint(rec.head[8]);
+    const f3 pos = mk(rec.head[0], rec.head[1], rec.head[2]), dir = mk(rec.head[4], rec.head[5], rec.head[6]);
+    const float len = rec.head[3], r = a.p.radius;
+    if (di < a.maxData) {
+        const float power = photon_power(a, sun_faces(a).total);
+        float* D = reinterpret_cast<float*>(a.data + di);
+        if (lane < 20u) D[lane] = lane < 4u ? power : rec.tr[lane - 4u];
+    }
+    const float* b0 = a.cloud.bounds[0];
+    const float* b1 = a.cloud.bounds[1];
+    const uint32_t segs = (uint32_t)fdiv(len, r) + 1u;
+    const float segSize = fdiv(len, (float)segs);
+    const uint64_t first = segBase + __float_as_uint(rec.head[9]);
+    for (uint32_t i = lane; i < segs; i += 64u) {
+        const uint64_t bi = first + i;
+        if (bi >= a.maxBeams) break;
+        const float off = (float)i * segSize;
+        const f3 st = add(pos, mul(dir, off));
+        const f3 en = add(st, mul(dir, segSize));
+        const uint32_t code = morton30(mk(fdiv(st.x + en.x, 2.0f), fdiv(st.y + en.y, 2.0f), fdiv(st.z + en.z, 2.0f)), b0, b1);
+        uint4* B = reinterpret_cast<uint4*>(a.beams + bi);
+        B[0] = make_uint4(__float_as_uint(st.x), __float_as_uint(st.y), __float_as_uint(st.z), code);
+        B[1] = make_uint4(__float_as_uint(en.x), __float_as_uint(en.y), __float_as_uint(en.z), __float_as_uint(r));
+        B[2] = make_uint4((uint32_t)di, __float_as_uint(off), 0u, 0u);
     }
 }
 
@@ -468,29 +509,24 @@ __global__ void __launch_bounds__(GATHER_THREADS, 4) gather_kernel(cr::GatherArg
 
 namespace cr {
 
-hipError_t launch_trace_count(const TraceArgs& a, int dtype, int layout, hipStream_t s)
+hipError_t launch_trace(const TraceArgs& a, int dtype, int layout, hipStream_t s)
 {
-    dim3 g((a.p.numPaths + 255) / 256);
+    if (a.nPaths == 0) return hipSuccess;
+    const dim3 g((a.nPaths + 256 / ROW - 1) / (256 / ROW));
     if (dtype == CR_DTYPE_F16) {
-        if (layout == LAYOUT_BRICK4) hipLaunchKernelGGL((trace_kernel<__half, LAYOUT_BRICK4, false>), g, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((trace_kernel<__half, LAYOUT_DENSE, false>), g, dim3(256), 0, s, a);
+        if (layout == LAYOUT_BRICK4) hipLaunchKernelGGL((trace_kernel<__half, LAYOUT_BRICK4>), g, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((trace_kernel<__half, LAYOUT_DENSE>), g, dim3(256), 0, s, a);
     } else {
-        if (layout == LAYOUT_BRICK4) hipLaunchKernelGGL((trace_kernel<float, LAYOUT_BRICK4, false>), g, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((trace_kernel<float, LAYOUT_DENSE, false>), g, dim3(256), 0, s, a);
+        if (layout == LAYOUT_BRICK4) hipLaunchKernelGGL((trace_kernel<float, LAYOUT_BRICK4>), g, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((trace_kernel<float, LAYOUT_DENSE>), g, dim3(256), 0, s, a);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_trace_write(const TraceArgs& a, int dtype, int layout, hipStream_t s)
+hipError_t launch_trace_expand(const TraceArgs& a, uint64_t records, hipStream_t s)
 {
-    dim3 g((a.p.numPaths + 255) / 256);
-    if (dtype == CR_DTYPE_F16) {
-        if (layout == LAYOUT_BRICK4) hipLaunchKernelGGL((trace_kernel<__half, LAYOUT_BRICK4, true>), g, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((trace_kernel<__half, LAYOUT_DENSE, true>), g, dim3(256), 0, s, a);
-    } else {
-        if (layout == LAYOUT_BRICK4) hipLaunchKernelGGL((trace_kernel<float, LAYOUT_BRICK4, true>), g, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((trace_kernel<float, LAYOUT_DENSE, true>), g, dim3(256), 0, s, a);
-    }
+    if (records == 0) return hipSuccess;
+    hipLaunchKernelGGL(expand_kernel, dim3((unsigned)((records + 3) / 4)), dim3(256), 0, s, a, records);
     return hipGetLastError();
 }
 

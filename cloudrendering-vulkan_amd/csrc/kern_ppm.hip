@@ -2,10 +2,10 @@
 // (shaders/PPM_PT.comp) and the ray-marched radiance estimate
 // (shaders/PPM_PE.comp) for gfx950.
 //
-// Tracing: one lane per photon path, run twice over the same RNG stream -- a
-// counting launch, then, after a scan gives every path its slots, a writing
-// launch -- so the deposits come out in emission order (path id, then
-// collision) instead of the reference's atomic arrival order
+// Tracing: one row of 16 lanes per photon path (row_walk.h).  The paths leave
+// their deposits as records; a scan of the paths' counts gives every path its
+// slots and a second kernel places the deposits there, in emission order (path
+// id, then collision) instead of the reference's atomic arrival order
 // (PPM_PT.comp:318).  A stable radix sort by cell then groups them, and a
 // cell keeps its first CR_PPM_PHOTONS_PER_CELL photons in that order: the map
 // is a pure function of the inputs, and the CPU oracle reproduces it.
@@ -16,6 +16,7 @@
 // edge, and the photons of the cells the query sphere overlaps.
 #include "cr_device.h"
 #include "cr_internal_ppm.h"
+#include "row_walk.h"
 
 using namespace crd;
 
@@ -60,15 +61,17 @@ __device__ __forceinline__ uint32_t cell_of(const cr_photon_map_properties& pm, 
     return (uint32_t)ix + ((uint32_t)iy + (uint32_t)iz * (uint32_t)pm.voxelCount[1]) * (uint32_t)pm.voxelCount[0];
 }
 
-// One photon path (PPM_PT.comp:452-488).  WRITE: deposits go to
-// photons/cells from slot `base`; otherwise only counted.
-template <typename T, int LAYOUT, bool WRITE>
+// One photon path per row of 16 lanes (PPM_PT.comp:452-488, row_walk.h).
+// Every deposit becomes a record in an arbitrary slot; counts[path] gets the
+// path's deposits.  12 800 paths on a 128^3 cloud: 2.26 ms when one lane walked
+// each path (200 waves), once to count and once more to write.
+template <typename T, int LAYOUT>
 __global__ void __launch_bounds__(256) ppm_trace_kernel(cr::PpmTraceArgs a)
 {
-    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t id = blockIdx.x * (256u / ROW) + threadIdx.x / ROW;
     if (id >= a.numPaths) return;
+    const RowLane R;
     uint32_t n = 0;
-    const uint32_t base = WRITE ? a.offsets[id] : 0u;
     const cr_cloud_properties& cp = a.cloud;
     if (cp.densityScaling > 0.0f) {
         const float* b0 = cp.bounds[0];
@@ -108,32 +111,22 @@ __global__ void __launch_bounds__(256) ppm_trace_kernel(cr::PpmTraceArgs a)
             if (!intersect_box(b0, b1, pos, dir, tmin, tmax)) break;
             const float dist = length(sub(pos, add(pos, mul(dir, tmax))));
             float t = 0.0f;
-            f3 cur = pos;
             bool hit = false;
-            for (uint32_t step = 0; step < TRACK_CEILING; step++) {
-                t = t + fdiv(-crd_logf(xs_float(rng)), sigmaBar);
-                if (!(t <= dist)) break;
-                cur = add(pos, mul(dir, t));
-                const float e = density<T, LAYOUT>(a.g, cp, cur);
-                if (xs_float(rng) < fdiv(e, cp.maxExtinction)) { hit = true; break; }
-            }
+            for (uint32_t round = 0; round < TRACK_CEILING / ROW; round++)
+                if (row_walk(R, sigmaBar, cp.maxExtinction, dist, t, rng, hit,
+                             [&](float d) { return density<T, LAYOUT>(a.g, cp, add(pos, mul(dir, d))); }))
+                    break;
             if (!hit) break;
-            pos = cur;
+            pos = add(pos, mul(dir, t));
             if (first) {
                 first = false;
             } else {
-                if (WRITE) {
-                    cr_photon ph;
-                    ph.position[0] = cur.x; ph.position[1] = cur.y; ph.position[2] = cur.z; ph.position[3] = 0.0f;
-                    ph.power[0] = col.x; ph.power[1] = col.y; ph.power[2] = col.z; ph.power[3] = col.w;
-                    ph.theta = crd_acosf(fminf(fmaxf(dir.z, -1.0f), 1.0f));
-                    const float phi = crd_atan2f(dir.y, dir.x);
-                    ph.phi = phi < 0.0f ? phi + TWO_PI : phi;
-                    ph._padding[0] = 0.0f;
-                    ph._padding[1] = 0.0f;
-                    a.photons[base + n] = ph;
-                    a.cells[base + n] = cell_of(a.pm, cur);
-                    a.order[base + n] = base + n;
+                const unsigned long long slot = row_slot(R, a.recordCount);
+                if (slot < a.recordCap && R.i == 0u) {
+                    float4* r = reinterpret_cast<float4*>(a.records + slot);
+                    r[0] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(id));
+                    r[1] = make_float4(dir.x, dir.y, dir.z, __uint_as_float(n));
+                    r[2] = make_float4(col.x, col.y, col.z, col.w);
                 }
                 n++;
             }
@@ -141,7 +134,29 @@ __global__ void __launch_bounds__(256) ppm_trace_kernel(cr::PpmTraceArgs a)
             dir = normalize(scatter(a.params, dir, rng));
         }
     }
-    if (!WRITE) a.counts[id] = n;
+    if (R.i == 0u) a.counts[id] = n;
+}
+
+// The deposits in emission order (path, then collision), their cells and slots.
+__global__ void __launch_bounds__(256) ppm_place_kernel(cr::PpmTraceArgs a, uint32_t nRecords)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= nRecords) return;
+    const float4* r = reinterpret_cast<const float4*>(a.records + i);
+    const float4 r0 = r[0], r1 = r[1], r2 = r[2];
+    const uint32_t at = a.offsets[__float_as_uint(r0.w)] + __float_as_uint(r1.w);
+    const f3 pos = mk(r0.x, r0.y, r0.z), dir = mk(r1.x, r1.y, r1.z);
+    cr_photon ph;
+    ph.position[0] = pos.x; ph.position[1] = pos.y; ph.position[2] = pos.z; ph.position[3] = 0.0f;
+    ph.power[0] = r2.x; ph.power[1] = r2.y; ph.power[2] = r2.z; ph.power[3] = r2.w;
+    ph.theta = crd_acosf(fminf(fmaxf(dir.z, -1.0f), 1.0f));
+    const float phi = crd_atan2f(dir.y, dir.x);
+    ph.phi = phi < 0.0f ? phi + TWO_PI : phi;
+    ph._padding[0] = 0.0f;
+    ph._padding[1] = 0.0f;
+    a.photons[at] = ph;
+    a.cells[at] = cell_of(a.pm, pos);
+    a.order[at] = at;
 }
 
 // Runs of the cell-sorted deposits: a run's first element records where it
@@ -334,12 +349,18 @@ namespace cr {
         }                                                                                                           \
     } while (0)
 
-hipError_t launch_ppm_trace(const PpmTraceArgs& a, bool write, int dtype, int layout, hipStream_t s)
+hipError_t launch_ppm_trace(const PpmTraceArgs& a, int dtype, int layout, hipStream_t s)
 {
     if (a.numPaths == 0) return hipSuccess;
-    const dim3 grid((a.numPaths + 255u) / 256u);
-    if (write) CR_PPM_DISPATCH(ppm_trace_kernel, grid, dim3(256), , true);
-    else CR_PPM_DISPATCH(ppm_trace_kernel, grid, dim3(256), , false);
+    const dim3 grid((a.numPaths + 256u / ROW - 1u) / (256u / ROW));
+    CR_PPM_DISPATCH(ppm_trace_kernel, grid, dim3(256), );
+    return hipGetLastError();
+}
+
+hipError_t launch_ppm_place(const PpmTraceArgs& a, uint32_t records, hipStream_t s)
+{
+    if (records == 0) return hipSuccess;
+    hipLaunchKernelGGL(ppm_place_kernel, dim3((records + 255u) / 256u), dim3(256), 0, s, a, records);
     return hipGetLastError();
 }
 
