@@ -14,15 +14,13 @@ struct PpmGrid {
     int32_t nx, ny, nz, nbx, nby;
 };
 
-// A deposit as its path left it.
+// A deposit as its path left it: position, power.x, direction, power.y,
+// power.z, power.w.
 struct PpmRecord {
-    float pos[3];
-    uint32_t path;
-    float dir[3];
-    uint32_t index;   // on its path
-    float power[4];
+    float v[12];
 };
-static_assert(sizeof(PpmRecord) == 48, "PpmRecord is three 16-B words");
+constexpr uint32_t PPM_FIRST = 8;    // record slots of every path
+constexpr uint32_t PPM_CHUNK = 16;   // record slots a path takes at a time after those
 
 struct PpmTraceArgs {
     PpmGrid g;
@@ -34,10 +32,12 @@ struct PpmTraceArgs {
     int32_t seed;
     float sunProbability;
     uint32_t maxCollisions;
+    uint32_t lanes;                   // trace: lanes of each wave that take a path
     uint32_t* counts;                 // trace: deposits per path
-    PpmRecord* records;
-    unsigned long long* recordCount;  // trace: records so far (may exceed recordCap; those past it are not stored)
-    uint64_t recordCap;
+    PpmRecord* records;               // PPM_FIRST per path, then the chunks
+    uint2* chunks;                    // (path, index of its first deposit) of each chunk
+    unsigned long long* chunkCount;   // trace: chunks taken (may exceed chunkCap; those past it are not stored)
+    uint64_t chunkCap;
     const uint32_t* offsets;          // place: first slot of each path
     cr_photon* photons;               // place: deposits in emission order
     uint32_t* cells;                  //   their cells
@@ -67,7 +67,7 @@ struct PpmEstimateArgs {
 };
 
 hipError_t launch_ppm_trace(const PpmTraceArgs& a, int dtype, int layout, hipStream_t s);
-hipError_t launch_ppm_place(const PpmTraceArgs& a, uint32_t records, hipStream_t s);
+hipError_t launch_ppm_place(const PpmTraceArgs& a, uint64_t chunks, hipStream_t s);
 hipError_t launch_ppm_runs(const uint32_t* keys, const uint32_t* vals, uint32_t n, uint32_t* start, uint32_t* arrivals,
                            const cr_photon* photons, cr_photon* sorted, float4* dirs, hipStream_t s);
 hipError_t launch_ppm_estimate(const PpmEstimateArgs& a, int dtype, int layout, hipStream_t s);

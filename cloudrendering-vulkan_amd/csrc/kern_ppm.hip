@@ -2,8 +2,7 @@
 // (shaders/PPM_PT.comp) and the ray-marched radiance estimate
 // (shaders/PPM_PE.comp) for gfx950.
 //
-// Tracing: one row of 16 lanes per photon path (row_walk.h).  The paths leave
-// their deposits as records; a scan of the paths' counts gives every path its
+// Tracing: one lane per photon path.  The paths leave their deposits as records; a scan of the paths' counts gives every path its
 // slots and a second kernel places the deposits there, in emission order (path
 // id, then collision) instead of the reference's atomic arrival order
 // (PPM_PT.comp:318).  A stable radix sort by cell then groups them, and a
@@ -16,7 +15,6 @@
 // edge, and the photons of the cells the query sphere overlaps.
 #include "cr_device.h"
 #include "cr_internal_ppm.h"
-#include "row_walk.h"
 
 using namespace crd;
 
@@ -61,16 +59,17 @@ __device__ __forceinline__ uint32_t cell_of(const cr_photon_map_properties& pm, 
     return (uint32_t)ix + ((uint32_t)iy + (uint32_t)iz * (uint32_t)pm.voxelCount[1]) * (uint32_t)pm.voxelCount[0];
 }
 
-// One photon path per row of 16 lanes (PPM_PT.comp:452-488, row_walk.h).
-// Every deposit becomes a record in an arbitrary slot; counts[path] gets the
-// path's deposits.  12 800 paths on a 128^3 cloud: 2.26 ms when one lane walked
-// each path (200 waves), once to count and once more to write.
+// One photon path per lane (PPM_PT.comp:452-488).  A path's first
+// PPM_FIRST deposits go to slots of its own, later ones to chunks taken from a
+// shared list (chunkCount); counts[path] gets the path's deposits.  A path is
+// one serial chain (a step, a collision, the next flight) and the lanes of a
+// wave wait for each other's walks, so few paths are spread over more waves,
+// a.lanes lanes of each in use.
 template <typename T, int LAYOUT>
-__global__ void __launch_bounds__(256) ppm_trace_kernel(cr::PpmTraceArgs a)
+__global__ void __launch_bounds__(64) ppm_trace_kernel(cr::PpmTraceArgs a)
 {
-    const uint32_t id = blockIdx.x * (256u / ROW) + threadIdx.x / ROW;
-    if (id >= a.numPaths) return;
-    const RowLane R;
+    const uint32_t id = blockIdx.x * a.lanes + threadIdx.x;
+    if (threadIdx.x >= a.lanes || id >= a.numPaths) return;
     uint32_t n = 0;
     const cr_cloud_properties& cp = a.cloud;
     if (cp.densityScaling > 0.0f) {
@@ -105,28 +104,42 @@ __global__ void __launch_bounds__(256) ppm_trace_kernel(cr::PpmTraceArgs a)
         }
         const float sigmaBar = fdiv(cp.maxExtinction * cp.densityScaling, cp.baseScaling);
         bool first = true;
+        uint64_t slot = (uint64_t)id * cr::PPM_FIRST;  // of the deposits being written
+        unsigned long long chunk = 0;
         for (uint32_t c = 0; c < a.maxCollisions; c++) {
             // interactWithMedium — PPM_PT.comp:398-446
             float tmin = 0.0f, tmax = 0.0f;
             if (!intersect_box(b0, b1, pos, dir, tmin, tmax)) break;
             const float dist = length(sub(pos, add(pos, mul(dir, tmax))));
             float t = 0.0f;
+            f3 cur = pos;
             bool hit = false;
-            for (uint32_t round = 0; round < TRACK_CEILING / ROW; round++)
-                if (row_walk(R, sigmaBar, cp.maxExtinction, dist, t, rng, hit,
-                             [&](float d) { return density<T, LAYOUT>(a.g, cp, add(pos, mul(dir, d))); }))
-                    break;
+            for (uint32_t step = 0; step < TRACK_CEILING; step++) {
+                t = t + fdiv(-crd_logf(xs_float(rng)), sigmaBar);
+                if (!(t <= dist)) break;
+                cur = add(pos, mul(dir, t));
+                const float e = density<T, LAYOUT>(a.g, cp, cur);
+                if (xs_float(rng) < fdiv(e, cp.maxExtinction)) { hit = true; break; }
+            }
             if (!hit) break;
-            pos = add(pos, mul(dir, t));
+            pos = cur;
             if (first) {
                 first = false;
             } else {
-                const unsigned long long slot = row_slot(R, a.recordCount);
-                if (slot < a.recordCap && R.i == 0u) {
-                    float4* r = reinterpret_cast<float4*>(a.records + slot);
-                    r[0] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(id));
-                    r[1] = make_float4(dir.x, dir.y, dir.z, __uint_as_float(n));
-                    r[2] = make_float4(col.x, col.y, col.z, col.w);
+                uint32_t k = n;
+                if (n >= cr::PPM_FIRST) {
+                    k = (n - cr::PPM_FIRST) % cr::PPM_CHUNK;
+                    if (k == 0u) {
+                        chunk = atomicAdd(a.chunkCount, 1ull);
+                        if (chunk < a.chunkCap) a.chunks[chunk] = make_uint2(id, n);
+                        slot = (uint64_t)a.numPaths * cr::PPM_FIRST + chunk * cr::PPM_CHUNK;
+                    }
+                }
+                if (n < cr::PPM_FIRST || chunk < a.chunkCap) {
+                    float4* r = reinterpret_cast<float4*>(a.records + slot + k);
+                    r[0] = make_float4(pos.x, pos.y, pos.z, col.x);
+                    r[1] = make_float4(dir.x, dir.y, dir.z, col.y);
+                    r[2] = make_float4(col.z, col.w, 0.0f, 0.0f);
                 }
                 n++;
             }
@@ -134,21 +147,32 @@ __global__ void __launch_bounds__(256) ppm_trace_kernel(cr::PpmTraceArgs a)
             dir = normalize(scatter(a.params, dir, rng));
         }
     }
-    if (R.i == 0u) a.counts[id] = n;
+    a.counts[id] = n;
 }
 
 // The deposits in emission order (path, then collision), their cells and slots.
-__global__ void __launch_bounds__(256) ppm_place_kernel(cr::PpmTraceArgs a, uint32_t nRecords)
+__global__ void __launch_bounds__(256) ppm_place_kernel(cr::PpmTraceArgs a, uint64_t nSlots)
 {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= nRecords) return;
+    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (i >= nSlots) return;
+    const uint64_t own = (uint64_t)a.numPaths * cr::PPM_FIRST;
+    uint32_t path, k;
+    if (i < own) {
+        path = (uint32_t)(i / cr::PPM_FIRST);
+        k = (uint32_t)(i % cr::PPM_FIRST);
+    } else {
+        const uint2 c = a.chunks[(i - own) / cr::PPM_CHUNK];
+        path = c.x;
+        k = c.y + (uint32_t)((i - own) % cr::PPM_CHUNK);
+    }
+    if (k >= a.counts[path]) return;
+    const uint32_t at = a.offsets[path] + k;
     const float4* r = reinterpret_cast<const float4*>(a.records + i);
     const float4 r0 = r[0], r1 = r[1], r2 = r[2];
-    const uint32_t at = a.offsets[__float_as_uint(r0.w)] + __float_as_uint(r1.w);
     const f3 pos = mk(r0.x, r0.y, r0.z), dir = mk(r1.x, r1.y, r1.z);
     cr_photon ph;
     ph.position[0] = pos.x; ph.position[1] = pos.y; ph.position[2] = pos.z; ph.position[3] = 0.0f;
-    ph.power[0] = r2.x; ph.power[1] = r2.y; ph.power[2] = r2.z; ph.power[3] = r2.w;
+    ph.power[0] = r0.w; ph.power[1] = r1.w; ph.power[2] = r2.x; ph.power[3] = r2.y;
     ph.theta = crd_acosf(fminf(fmaxf(dir.z, -1.0f), 1.0f));
     const float phi = crd_atan2f(dir.y, dir.x);
     ph.phi = phi < 0.0f ? phi + TWO_PI : phi;
@@ -352,15 +376,15 @@ namespace cr {
 hipError_t launch_ppm_trace(const PpmTraceArgs& a, int dtype, int layout, hipStream_t s)
 {
     if (a.numPaths == 0) return hipSuccess;
-    const dim3 grid((a.numPaths + 256u / ROW - 1u) / (256u / ROW));
-    CR_PPM_DISPATCH(ppm_trace_kernel, grid, dim3(256), );
+    const dim3 grid((a.numPaths + a.lanes - 1u) / a.lanes);
+    CR_PPM_DISPATCH(ppm_trace_kernel, grid, dim3(64), );
     return hipGetLastError();
 }
 
-hipError_t launch_ppm_place(const PpmTraceArgs& a, uint32_t records, hipStream_t s)
+hipError_t launch_ppm_place(const PpmTraceArgs& a, uint64_t chunks, hipStream_t s)
 {
-    if (records == 0) return hipSuccess;
-    hipLaunchKernelGGL(ppm_place_kernel, dim3((records + 255u) / 256u), dim3(256), 0, s, a, records);
+    const uint64_t slots = (uint64_t)a.numPaths * PPM_FIRST + chunks * PPM_CHUNK;
+    hipLaunchKernelGGL(ppm_place_kernel, dim3((unsigned)((slots + 255u) / 256u)), dim3(256), 0, s, a, slots);
     return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-// Delta-tracking walks by rows of 16 lanes, for the photon tracers.
+// Delta-tracking walks by rows of 16 lanes, for the photon-beam producer.
 //
 // A photon path is one chain of random numbers: where a walk ends decides from
 // which draw the next one goes on, so paths are serial and a trace of some
@@ -12,7 +12,10 @@
 // shift, all lookups go out at once, and the first lane whose step leaves the
 // segment or collides ends the walk; the steps past it are dropped and the
 // state is the one after the last draw the walk used.  Same draws, same sums
-// in the same order as one lane stepping alone.
+// in the same order as one lane stepping alone.  A path of the producer makes
+// 17 walks of some twenty steps per interaction; photon mapping's paths, whose
+// walks end after two or three steps in dense cloud, gain nothing from this
+// (12 800 paths 1.03 ms, one lane each 0.97; a million 50 ms against 4.9).
 #pragma once
 
 #include "cr_device.h"
