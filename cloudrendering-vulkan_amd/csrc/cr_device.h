@@ -360,6 +360,54 @@ __device__ __forceinline__ float trilinear(const GridView& g, f3 n)
     return c0 * oc + c1 * c;
 }
 
+// Division by a divisor the same for a whole launch, correctly rounded, without
+// the divide sequence: with y = 1/d correctly rounded, q0 = x y is within two
+// units of the quotient, one residual step q1 = q0 + (x - d q0) y makes it
+// faithful and the next one rounds it correctly (Markstein, IBM J. Res. Dev.
+// 34(1), 1990), while no intermediate value is subnormal or overflows.  A power
+// of two divides exactly by the multiplication alone.  Other divisors (0, tiny,
+// huge, NaN) take the IEEE division.  The numerators are finite coordinate
+// differences of at most a few divisors; one below 2^-100 may come out an ulp
+// off, a quotient far below what any use of it can tell from 0.
+enum : uint32_t { DIV_IEEE = 0, DIV_RESIDUAL = 1, DIV_POW2 = 2 };
+
+struct Divisors3 {
+    float d[3], y[3];
+    uint32_t how;
+};
+
+__host__ __device__ inline Divisors3 make_divisors(float dx, float dy, float dz)
+{
+    Divisors3 r = {{dx, dy, dz}, {1.0f / dx, 1.0f / dy, 1.0f / dz}, DIV_POW2};
+    for (int k = 0; k < 3; k++) {
+        const float a = r.d[k];
+        union { float f; uint32_t u; } b = {a};
+        if (!(a > 0x1p-60f && a < 0x1p60f)) r.how = DIV_IEEE;
+        else if ((b.u & 0x7fffffu) != 0u && r.how == DIV_POW2) r.how = DIV_RESIDUAL;
+    }
+    return r;
+}
+
+__device__ __forceinline__ float div_residual(float x, float d, float y)
+{
+    const float q0 = x * y;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-d, q0, x), y, q0);
+    return __builtin_fmaf(__builtin_fmaf(-d, q1, x), y, q1);
+}
+
+__device__ __forceinline__ f3 div3(const Divisors3& v, f3 x)
+{
+    if (v.how == DIV_POW2) return mk(x.x * v.y[0], x.y * v.y[1], x.z * v.y[2]);
+    if (v.how == DIV_RESIDUAL)
+        return mk(div_residual(x.x, v.d[0], v.y[0]), div_residual(x.y, v.d[1], v.y[1]), div_residual(x.z, v.d[2], v.y[2]));
+    return mk(fdiv(x.x, v.d[0]), fdiv(x.y, v.d[1]), fdiv(x.z, v.d[2]));
+}
+
+// Two consecutive values, read with one load (4-byte aligned).
+struct __attribute__((packed, aligned(4))) Pair {
+    float x, y;
+};
+
 // sampleCloud's normalisation — PathTracer.comp:115-119.
 __device__ __forceinline__ f3 cloud_norm(const cr_cloud_properties& cp, f3 p)
 {

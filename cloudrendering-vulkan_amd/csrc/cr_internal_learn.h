@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/cr/abi.h"
+#include "cr_device.h"
 
 namespace cr {
 
@@ -18,6 +19,7 @@ struct FeatureArgs {
     const float* mips[LEARN_LEVELS];
     int32_t dims[LEARN_LEVELS][3];
     cr_cloud_properties cloud;
+    crd::Divisors3 extent;  // of the box
     float light[3];         // propagation direction of sunlight
     float h0;               // world size of a level-0 voxel
     uint16_t* X;            // [n][224] bf16

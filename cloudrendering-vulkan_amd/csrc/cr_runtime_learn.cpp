@@ -132,6 +132,8 @@ cr_status learn_features_device(cr_context* ctx, const float* points, uint64_t n
         a.dims[k][0] = L->dims[k][0]; a.dims[k][1] = L->dims[k][1]; a.dims[k][2] = L->dims[k][2];
     }
     a.cloud = ctx->cloud;
+    a.extent = crd::make_divisors(ctx->cloud.bounds[1][0] - ctx->cloud.bounds[0][0], ctx->cloud.bounds[1][1] - ctx->cloud.bounds[0][1],
+                                  ctx->cloud.bounds[1][2] - ctx->cloud.bounds[0][2]);
     a.light[0] = ctx->svp.lightDirection[0];
     a.light[1] = ctx->svp.lightDirection[1];
     a.light[2] = ctx->svp.lightDirection[2];

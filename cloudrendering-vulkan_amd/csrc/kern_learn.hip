@@ -15,13 +15,6 @@ using namespace crd;
 
 namespace {
 
-__device__ __forceinline__ uint16_t f2bf(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    u = u + 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-
 // Level k+1 = mean of the existing voxels of each 2x2x2 block of level k.
 __global__ void __launch_bounds__(256) mip_kernel(const float* src, int32_t sx, int32_t sy, int32_t sz, float* dst,
                                                   int32_t dx, int32_t dy, int32_t dz)
@@ -40,19 +33,67 @@ __global__ void __launch_bounds__(256) mip_kernel(const float* src, int32_t sx, 
     dst[(size_t)x + (size_t)dx * ((size_t)y + (size_t)dy * z)] = fdiv(acc, cnt);
 }
 
-// The coarsest mip levels, as many as fit in this many floats (32 KB), are
+// The coarsest mip levels, as many as fit in this many floats (18.4 KB), are
 // copied into LDS by each workgroup: for a 128^3 grid, levels 3-7 (16^3 down
-// to 1^3, 18.3 KB), whose taps are 135 of a record's 216.
-constexpr uint32_t FEATURE_LDS_FLOATS = 8192;
+// to 1^3), whose taps are 135 of a record's 216.
+constexpr uint32_t FEATURE_LDS_FLOATS = 4736;
 
 __device__ __forceinline__ uint32_t mip_floats(const cr::FeatureArgs& a, int k)
 {
     return (uint32_t)a.dims[k][0] * (uint32_t)a.dims[k][1] * (uint32_t)a.dims[k][2];
 }
 
+struct Level {
+    const float* data;
+    int32_t nx, ny, nz;
+};
+
+// The trilinear lookup (cr_device.h) at normalised coordinates in [0, 1] of a
+// mip level in memory, or its copy m in LDS.  The two texels of an x pair are
+// neighbours and come with one load; at the first and last half texel, where
+// both are the edge texel, the pair next to it is loaded and the edge chosen
+// from it.
+__device__ __forceinline__ float tap(const Level& L, bool lds, const float* m, f3 n)
+{
+    const float ux = n.x * (float)L.nx - 0.5f, uy = n.y * (float)L.ny - 0.5f, uz = n.z * (float)L.nz - 0.5f;
+    const float fx = floorf(ux), fy = floorf(uy), fz = floorf(uz);
+    const float a = ux - fx, b = uy - fy, c = uz - fz;
+    const int32_t ix = (int32_t)fx, iy = (int32_t)fy, iz = (int32_t)fz;
+    const uint32_t sy = (uint32_t)L.nx, sz = (uint32_t)L.nx * (uint32_t)L.ny;
+    const uint32_t y0 = (uint32_t)clampi(iy, 0, L.ny - 1) * sy, y1 = (uint32_t)clampi(iy + 1, 0, L.ny - 1) * sy;
+    const uint32_t z0 = (uint32_t)clampi(iz, 0, L.nz - 1) * sz, z1 = (uint32_t)clampi(iz + 1, 0, L.nz - 1) * sz;
+    const int32_t x0 = max(min(ix, L.nx - 2), 0);
+    const uint32_t i00 = (uint32_t)x0 + (y0 + z0), i10 = (uint32_t)x0 + (y1 + z0);
+    const uint32_t i01 = (uint32_t)x0 + (y0 + z1), i11 = (uint32_t)x0 + (y1 + z1);
+    float v00, v00b, v10, v10b, v01, v01b, v11, v11b;
+    if (lds) {
+        // one texel past the level's last is still inside the LDS array
+        v00 = m[i00]; v00b = m[i00 + 1]; v10 = m[i10]; v10b = m[i10 + 1];
+        v01 = m[i01]; v01b = m[i01 + 1]; v11 = m[i11]; v11b = m[i11 + 1];
+    } else if (L.nx >= 2) {
+        const Pair p00 = *reinterpret_cast<const Pair*>(L.data + i00), p10 = *reinterpret_cast<const Pair*>(L.data + i10);
+        const Pair p01 = *reinterpret_cast<const Pair*>(L.data + i01), p11 = *reinterpret_cast<const Pair*>(L.data + i11);
+        v00 = p00.x; v00b = p00.y; v10 = p10.x; v10b = p10.y;
+        v01 = p01.x; v01b = p01.y; v11 = p11.x; v11b = p11.y;
+    } else {
+        v00 = v00b = L.data[i00]; v10 = v10b = L.data[i10];
+        v01 = v01b = L.data[i01]; v11 = v11b = L.data[i11];
+    }
+    if (ix < 0 || L.nx == 1) {  // both the first texel
+        v00b = v00; v10b = v10; v01b = v01; v11b = v11;
+    } else if (ix > L.nx - 2) {  // both the last one
+        v00 = v00b; v10 = v10b; v01 = v01b; v11 = v11b;
+    }
+    const float oa = 1.0f - a, ob = 1.0f - b, oc = 1.0f - c;
+    const float c00 = v00 * oa + v00b * a, c10 = v10 * oa + v10b * a;
+    const float c01 = v01 * oa + v01b * a, c11 = v11 * oa + v11b * a;
+    const float c0 = c00 * ob + c10 * b, c1 = c01 * ob + c11 * b;
+    return c0 * oc + c1 * c;
+}
+
 __global__ void __launch_bounds__(256) features_kernel(cr::FeatureArgs a)
 {
-    __shared__ float mipLds[FEATURE_LDS_FLOATS];
+    __shared__ float mipLds[FEATURE_LDS_FLOATS + 1];
     // The grid is sized for every record; the count of collisions among them
     // is known only on the device.  A workgroup wholly past it leaves before
     // staging (the test is the same for all its threads, so no thread is left
@@ -98,46 +139,31 @@ __global__ void __launch_bounds__(256) features_kernel(cr::FeatureArgs a)
 #pragma unroll 1
     for (int grp = 0; grp < 4; grp++) {
         uint32_t packed[28];
-        int idx = 0;
+        float last = 0.0f;
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
             const int k = 2 * grp + kk;
-            GridView g;
-            g.nx = a.dims[k][0]; g.ny = a.dims[k][1]; g.nz = a.dims[k][2];
-            g.nbx = 0; g.nby = 0;
-            // the 27 taps of level k; a staged level's copy reads LDS directly
-            auto taps = [&](const GridView& gv) {
+            const Level L = {a.mips[k], a.dims[k][0], a.dims[k][1], a.dims[k][2]};
+            const bool lds = k >= staged;
+            const float* const m = mipLds + (lds ? ldsOff : 0u);
 #pragma unroll
-                for (int l = -1; l <= 1; l++)
-#pragma unroll
-                    for (int j = -1; j <= 1; j++)
-#pragma unroll
-                        for (int ii = -1; ii <= 1; ii++) {
-                            const float fi = (float)ii * h, fj = (float)j * h, fl = (float)l * h;
-                            const f3 p = mk(x.x + ((fi * ex.x + fj * ey.x) + fl * ez.x),
-                                            x.y + ((fi * ex.y + fj * ey.y) + fl * ez.y),
-                                            x.z + ((fi * ex.z + fj * ey.z) + fl * ez.z));
-                            float d = 0.0f;
-                            if (in_box(b0, b1, p)) d = trilinear<float, LAYOUT_DENSE>(gv, cloud_norm(a.cloud, p));
-                            const uint16_t v = f2bf((d * sscale) * h);
-                            if (idx & 1) packed[idx >> 1] |= (uint32_t)v << 16;
-                            else packed[idx >> 1] = v;
-                            idx++;
-                        }
-            };
-            if (k >= staged) {
-                g.data = mipLds + ldsOff;
-                ldsOff += mip_floats(a, k);
-                taps(g);
-            } else {
-                g.data = a.mips[k];
-                taps(g);
+            for (int t = 0; t < 27; t++) {
+                const float fi = (float)(t % 3 - 1) * h, fj = (float)(t / 3 % 3 - 1) * h, fl = (float)(t / 9 - 1) * h;
+                const f3 p = mk(x.x + ((fi * ex.x + fj * ey.x) + fl * ez.x), x.y + ((fi * ex.y + fj * ey.y) + fl * ez.y),
+                                x.z + ((fi * ex.z + fj * ey.z) + fl * ez.z));
+                float d = 0.0f;
+                if (in_box(b0, b1, p)) d = tap(L, lds, m, div3(a.extent, sub(p, ld3(b0))));
+                const float v = (d * sscale) * h;
+                const int idx = 27 * kk + t;
+                if (idx & 1) packed[idx >> 1] = bf16x2_rne(last, v);
+                last = v;
             }
+            if (lds) ldsOff += mip_floats(a, k);
             h = h * 2.0f;
         }
         if (grp == 3) {
             const float c = dot(w, ez);
-            packed[27] = (uint32_t)f2bf(c) | ((uint32_t)f2bf(c * c) << 16);
+            packed[27] = bf16x2_rne(c, c * c);
         }
         uint32_t* o = out + 27 * grp;
 #pragma unroll
