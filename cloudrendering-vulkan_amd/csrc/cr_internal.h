@@ -51,7 +51,8 @@ struct PTArgs {
     uint32_t padded;        // 32 * (W/32 + 1), the reference's id stride
     uint32_t tilesX;
     uint32_t totalIdx;      // tiles * 64
-    uint32_t* queue;        // pixel work counter (zeroed before launch)
+    uint32_t* queue;        // PT_QUEUE_WORDS work counters, one per part of the items (zeroed before launch)
+    uint32_t logParts;      // the items are cut into 1 << logParts parts (0 or 3)
     unsigned long long* counters; // paths, vertices, lookups, svLookups, brickVisits
     uint32_t tileLog2W;     // a wave's claims walk tiles of (1 << tileLog2W) x (64 >> tileLog2W) pixels
     uint32_t base;          // batched launch: first work index of this job
@@ -68,9 +69,10 @@ struct PTArgs {
     uint32_t chunk, chunks;
     float4* samples;
     uint32_t blendBase;     // batched launch: first workgroup of this job in the blend kernel
-    // scheduling (render pass): claim order of the tiles, and per-tile work of this launch
-    const uint32_t* tileOrder;  // tile for each queue slot, or null (raster order)
-    uint32_t* tileCost;         // lookups + brick visits per tile, accumulated, or null
+    // scheduling (render pass): the tiles to claim, in order
+    const uint32_t* tileOrder;  // listed tiles, part after part, or null (all in raster order)
+    const uint32_t* partStart;  // 9 words: where the parts start in the list, and its length; or null.  The
+                                //   pixels that miss the box are rendered when the list is made
 };
 
 // One persistent launch over several jobs: the job table (PTArgs per job,
@@ -81,6 +83,7 @@ struct BatchArgs {
     uint32_t nJobs;
     uint32_t total;         // sum of the jobs' totalIdx
     uint32_t* queue;
+    uint32_t logParts;
     unsigned long long* counters;
 };
 
@@ -88,6 +91,7 @@ struct BatchArgs {
 // at most PT_FEW_FRAMES frames use the instantiation with gated pixel claims
 // (kern_pt_few.hip), which is faster when an item carries little work.
 constexpr uint32_t PT_FEW_FRAMES = 16;
+constexpr uint32_t PT_QUEUE_WORDS = 8;
 // Work items of a chunked pass: at least this many per resident lane while
 // there are samples to make them of, each of at most PT_FEW_FRAMES samples.
 // Frames per work item of a chunked pass: at least PT_ITEMS_PER_LANE items per
@@ -106,20 +110,20 @@ inline uint32_t pt_chunk(uint64_t pixels, uint32_t samples, uint64_t lanes, uint
     const uint64_t c = pixels * samples / (PT_ITEMS_PER_LANE * lanes);
     return (uint32_t)(c < 1 ? 1 : (c > most ? most : c));
 }
-// Renders of several frames are chunked, except brick-DDA renders of images
-// with this many pixels or more per resident lane: their lanes have pixels
-// enough to balance, and the claims and stored samples cost more than they
-// bring (ms unchunked / chunked, 64 spp: 1 GiB grid at 256^2 45 / 5.8, 800x600
-// 44 / 24, 720p 54 / 43, 1080p with 256 bounces 334 / 360 at 256 spp; 128^3
-// grid at 1280x960 29 / 24.5, 1080p 83 / 77 at 64 spp and 302 / 300 at 256).
-// Global-majorant renders gain at every size (1080p 113 / 72, 4K 438 / 294).
-constexpr uint64_t PT_SPLIT_PIXELS_DDA = 6;
 // Samples stored by one chunked launch at most (4 GiB); more go in several
 // launches, each of which ends on its longest paths (16-job batch: 88.6 ms
 // with 1 GiB).
 constexpr uint64_t PT_SAMPLE_BUDGET = 1ull << 28;
 hipError_t launch_pt(const PTArgs& a, int dtype, int layout, int grid_blocks, hipStream_t s);
 int pt_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee, uint32_t chunk);
+// The tile list of a render (lists: pt_list_words(a) words; the list ends where
+// the nine part starts begin, at pt_list_starts(a)).  The image is cut into
+// squares of 8x8 tiles, dealt to the eight XCDs in turn; tiles without a pixel
+// that hits the box are left out, and all frames of every pixel that misses it
+// are rendered here.
+uint64_t pt_list_words(const PTArgs& a);
+uint64_t pt_list_starts(const PTArgs& a);
+hipError_t launch_pt_list(const PTArgs& a, uint32_t* lists, hipStream_t s);
 // The second half of a chunked launch: blend the stored samples into the
 // image(s), or sum the stored continuations (total: samples per record).
 hipError_t launch_pt_blend(const PTArgs& a, hipStream_t s);
@@ -131,12 +135,6 @@ int pt_few_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee)
 hipError_t launch_pt_batch(const BatchArgs& b, int dtype, int layout, uint32_t tracking, uint32_t nee, int grid_blocks,
                            int block_threads, hipStream_t s);
 int pt_batch_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee, int block_threads, uint32_t n_jobs);
-// Tile claim order for the next render: tiles by decreasing cost (a stable
-// radix sort of ~cost; ties keep raster order).  keys/vals/tmp: n words each,
-// counts: the radix sort's histograms (pt_order_counts(n) bytes).
-uint32_t pt_order_counts(uint32_t n);
-hipError_t launch_tile_order(const uint32_t* cost, uint32_t n, uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp,
-                             uint32_t* vals_tmp, uint32_t* counts, hipStream_t s);
 // kern_pt_learn.hip
 hipError_t launch_pt_record(const PTArgs& a, int dtype, int layout, int blocks, hipStream_t s);
 hipError_t launch_pt_continue(const PTArgs& a, int dtype, int layout, int blocks, hipStream_t s);

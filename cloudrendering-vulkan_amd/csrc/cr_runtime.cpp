@@ -140,7 +140,7 @@ cr_status cr_destroy(cr_context* ctx)
     hipSetDevice(ctx->device);
     if (ctx->stream) hipStreamSynchronize(ctx->stream);
     void* bufs[] = {ctx->grid.data, ctx->grid.majorants, ctx->grid.skip, ctx->sv, ctx->image, ctx->dFrames, ctx->dQueue,
-                    ctx->tileCost, ctx->tileSort, ctx->ptSamples,
+                    ctx->tileList, ctx->ptSamples,
                     ctx->dCounters, ctx->dScalar};
     for (void* b : bufs)
         if (b) hipFree(b);
@@ -713,7 +713,7 @@ void fill_job_args(PTArgs& a, const DeviceGrid& g, const float* sv, const uint32
 }
 
 // Work items of `chunk` frames instead of whole pixels, as long as their
-// number fits the queue's 32-bit counter (which idle lanes overrun a little).
+// number fits the queue's 32-bit counters (which idle lanes overrun a little).
 void set_chunk(PTArgs& a, uint32_t chunk)
 {
     const uint32_t chunks = (a.nFrames + chunk - 1u) / chunk;
@@ -769,43 +769,28 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
     fill_pt_args(ctx, a, n_frames);
     const DeviceGrid& g = ctx->grid;
     // Work items of a few frames each, the samples stored and blended by a
-    // second kernel: whole pixels of a small image would leave lanes without
-    // work, and the last ones alone with a long pixel.
+    // second kernel: whole pixels would leave lanes without work in a small
+    // image, and the last ones alone with a long pixel in any.  (Without room
+    // for the samples the lanes render whole pixels.)
     const uint64_t px = (uint64_t)ctx->W * (uint64_t)ctx->H;
     const uint64_t lanes = (uint64_t)ctx->numCUs * 256u *
                            (uint64_t)pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, 1);
     uint32_t group = n_frames;  // frames per launch
-    if (n_frames > 1 && (ctx->ext.trackingMode != CR_TRACK_BRICK_DDA || px < PT_SPLIT_PIXELS_DDA * lanes)) {
+    if (n_frames > 1) {
         group = (uint32_t)std::min<uint64_t>(n_frames, std::max<uint64_t>(1, PT_SAMPLE_BUDGET / px));
         if (sample_buffer(&ctx->ptSamples, &ctx->ptSamplesCap, px * group)) a.samples = ctx->ptSamples;
         else group = n_frames;
     }
-    CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
-    // Otherwise claim tiles in decreasing order of the previous render's
-    // per-tile work (same image shape), so the persistent grid drains on cheap
-    // tiles.  Only the schedule changes; every pixel's arithmetic is the same.
-    const uint32_t nTiles = a.totalIdx / 64u;
-    if (!a.samples) {
-        if (ctx->tileN != nTiles || ctx->tileLog2W != a.tileLog2W || !ctx->tileCost) {
-            if (ctx->tileCost) hipFree(ctx->tileCost);
-            ctx->tileCost = nullptr;
-            ctx->tileCostValid = false;
-            CR_HIP(ctx, hipMalloc((void**)&ctx->tileCost, (size_t)nTiles * 4), "hipMalloc tile costs");
-            ctx->tileN = nTiles;
-            ctx->tileLog2W = a.tileLog2W;
-        }
-        if (ctx->tileCostValid) {
-            st = ensure_buffer(ctx, (void**)&ctx->tileSort, &ctx->tileSortCap,
-                               (size_t)nTiles * 16 + pt_order_counts(nTiles), "tile order");
-            if (st != CR_OK) return st;
-            uint32_t* k = ctx->tileSort;
-            CR_HIP(ctx, launch_tile_order(ctx->tileCost, nTiles, k, k + nTiles, k + 2 * (size_t)nTiles,
-                                          k + 3 * (size_t)nTiles, k + 4 * (size_t)nTiles, ctx->stream), "tile order");
-            a.tileOrder = k + nTiles;
-        }
-        CR_HIP(ctx, zero_async(ctx->tileCost, (size_t)nTiles * 4, ctx->stream), "zero tile costs");
-        a.tileCost = ctx->tileCost;
-        ctx->tileCostValid = true;
+    CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
+    if (n_frames > 1) {
+        // the tiles to claim, by XCD (a single frame takes all tiles in raster
+        // order: the lists cost it more than they bring)
+        st = ensure_buffer(ctx, (void**)&ctx->tileList, &ctx->tileListCap, (size_t)pt_list_words(a) * 4, "tile list");
+        if (st != CR_OK) return st;
+        CR_HIP(ctx, launch_pt_list(a, ctx->tileList, ctx->stream), "tile list kernels");
+        a.tileOrder = ctx->tileList + pt_list_starts(a) - a.totalIdx / 64u;
+        a.partStart = ctx->tileList + pt_list_starts(a);
+        a.logParts = 3;
     }
     if (ctx->ptEventsUsed >= 1024) {
         st = fold_pt_events(ctx);
@@ -829,7 +814,7 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
         const uint32_t needed = (b.totalIdx + 255u) / 256u;
         if ((uint32_t)blocks > needed) blocks = (int)needed;
         if (ctx->ptBlocksOverride > 0) blocks = ctx->ptBlocksOverride;
-        if (f0) CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
+        if (f0) CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
         CR_HIP(ctx, launch_pt(b, g.dtype, g.layout, blocks, ctx->stream), "path tracer kernel");
         if (b.samples) CR_HIP(ctx, launch_pt_blend(b, ctx->stream), "blend kernel");
     }

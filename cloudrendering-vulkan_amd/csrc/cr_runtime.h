@@ -75,12 +75,8 @@ struct cr_context {
     double ptTotalMs = 0.0;
     uint64_t ptLaunches = 0;
     int ptBlocksOverride = 0;
-    // cost-ordered tile scheduling: per-tile work of the last render, and the sort buffers
-    uint32_t* tileCost = nullptr;
-    uint32_t* tileSort = nullptr;   // keys, vals, keys_tmp, vals_tmp (nTiles each) + histograms
-    size_t tileSortCap = 0;
-    uint32_t tileN = 0, tileLog2W = 0;
-    bool tileCostValid = false;
+    uint32_t* tileList = nullptr;   // tile schedule of the last render
+    size_t tileListCap = 0;
     // samples of a chunked render or continuation pass (at most PT_SAMPLE_BUDGET)
     float4* ptSamples = nullptr;
     size_t ptSamplesCap = 0;

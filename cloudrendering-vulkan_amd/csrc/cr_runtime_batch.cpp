@@ -224,8 +224,9 @@ hipError_t enqueue_groups(cr_context* ctx, const Batch* b, const std::vector<Gro
         a.nJobs = g.n;
         a.total = g.total;
         a.queue = queue;
+        a.logParts = 3;
         a.counters = counters;
-        e = zero_async(queue, 4, ctx->stream);
+        e = zero_async(queue, PT_QUEUE_WORDS * 4, ctx->stream);
         if (e == hipSuccess)
             e = launch_pt_batch(a, b->dtype, b->layout, b->tracking, b->nee, launch_blocks(ctx, b, t, g), (int)t.blockThreads,
                                 ctx->stream);

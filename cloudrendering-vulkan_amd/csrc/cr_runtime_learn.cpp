@@ -217,7 +217,7 @@ cr_status record_pass(cr_context* ctx, Learn* L, const cr_push_constants* frames
     set_chunk(a, pt_chunk((uint64_t)ctx->W * (uint64_t)ctx->H, n_frames, (uint64_t)pass_blocks(ctx, 0, ~0u) * 256u, PT_CHUNK_RECORD));
     a.records = L->records;
     a.counters = ctx->dCounters + 8;
-    CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
+    CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
     CR_HIP(ctx, launch_pt_record(a, ctx->grid.dtype, ctx->grid.layout, pass_blocks(ctx, 0, a.totalIdx), ctx->stream),
            "record pass");
     *n_out = n;
@@ -250,7 +250,7 @@ cr_status continue_pass(cr_context* ctx, const float* pts, uint32_t m, uint32_t 
         a.spp = std::min(group, spp - s0);
         a.chunk = a.samples ? 1u : a.spp;
         a.totalIdx = m * ((a.spp + a.chunk - 1u) / a.chunk);
-        CR_HIP(ctx, zero_async(ctx->dQueue, 4, ctx->stream), "zero queue");
+        CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
         CR_HIP(ctx, launch_pt_continue(a, ctx->grid.dtype, ctx->grid.layout, pass_blocks(ctx, 1, a.totalIdx), ctx->stream),
                "continuation pass");
         if (a.samples) CR_HIP(ctx, launch_pt_sum(a, spp, ctx->stream), "continuation sums");

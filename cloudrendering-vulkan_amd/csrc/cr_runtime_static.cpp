@@ -1,19 +1,17 @@
 // Allocation-free path-tracer entry point (cr_pt_render_static).
 //
 // cr_pt_render keeps its scratch in context buffers that it grows on demand:
-// the work-queue counter, the statistics counters, the per-frame
-// (seed, frameCount) table and the per-tile cost and claim-order buffers.
-// This variant keeps the first three in one fixed device array per GPU,
-// resolved once per device when a context is created, and renders into an
-// image the caller owns; tiles are claimed in raster order, which changes the
-// schedule only (every pixel's arithmetic is cr_pt_render's).  It calls no
-// hipMalloc, hipFree or allocating library routine.
+// the work-queue counter, the per-frame (seed, frameCount) table, the tile
+// list and the samples.  This variant keeps the first two in one fixed device
+// array per GPU, resolved once per device when a context is created, and renders
+// whole pixels into an image the caller owns; tiles are claimed in raster order,
+// which changes the schedule only (every pixel's arithmetic is cr_pt_render's).
+// It calls no hipMalloc, hipFree or allocating library routine.
 //
 // The array is shared by every context on a GPU and keeps the last call's
-// contents: the queue and counters are cleared by a fill kernel at the start
-// of each call, the frame table is overwritten.  Calls that overlap on one
-// GPU (two host threads, or two contexts whose streams run concurrently)
-// race on it.
+// contents: the queue is cleared by a fill kernel at the start of each call, the
+// frame table is overwritten.  Calls that overlap on one GPU (two host threads,
+// or two contexts whose streams run concurrently) race on it.
 #include <mutex>
 
 #include "cr_runtime.h"
@@ -104,8 +102,6 @@ cr_status cr_pt_render_static(cr_context* ctx, const cr_push_constants* frames, 
                   dFrames, n_frames, accum, ctx->W, ctx->H, ctx->ptTileLog2W);
     a.queue = (uint32_t*)(base + QUEUE_OFF);
     a.counters = (unsigned long long*)(base + COUNTERS_OFF);
-    a.tileOrder = nullptr;
-    a.tileCost = nullptr;
     const DeviceGrid& g = ctx->grid;
     int blocks = ctx->numCUs * pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, n_frames);
     const uint32_t needed = (a.totalIdx + 255u) / 256u;

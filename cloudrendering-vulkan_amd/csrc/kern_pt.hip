@@ -1,42 +1,115 @@
 // Launches of the path tracer: the single-job render and the batched render.
 #include "pt_kernel.h"
 
-#include "cr_internal_ppb.h"
-
 namespace {
 
-__global__ void __launch_bounds__(256) order_keys_kernel(const uint32_t* cost, uint32_t n, uint32_t* keys, uint32_t* vals)
+// PathTracer.comp:420-424
+__device__ __forceinline__ void blend_sample(float4& acc, float4 L, uint32_t fc)
 {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    keys[i] = ~cost[i];
-    vals[i] = i;
+    const float n = (float)fc, d = (float)(fc + 1u);
+    acc.x = fdiv(L.x + acc.x * n, d);
+    acc.y = fdiv(L.y + acc.y * n, d);
+    acc.z = fdiv(L.z + acc.z * n, d);
+    acc.w = fdiv(L.w + acc.w * n, d);
 }
 
-// The running mean of nf stored samples of pixel p, in frame order
-// (PathTracer.comp:420-424), blended into the image.
-__device__ __forceinline__ void blend_pixel(const float4* samples, const int32_t* frames, uint32_t nf, float4* image,
-                                            uint32_t pixels, uint32_t p)
+// The running mean of the stored samples of pixel p, in frame order, blended
+// into the image.
+__device__ __forceinline__ void blend_pixel(const cr::PTArgs& a, uint32_t pixels, uint32_t p)
 {
-    float4 acc = image[p];
+    float4 acc = a.image[p];
 #pragma unroll 4
-    for (uint32_t f = 0; f < nf; f++) {
-        const float4 L = samples[(size_t)f * pixels + p];
-        const uint32_t fc = (uint32_t)frames[2 * f + 1];
-        const float n = (float)fc, d = (float)(fc + 1u);
-        acc.x = fdiv(L.x + acc.x * n, d);
-        acc.y = fdiv(L.y + acc.y * n, d);
-        acc.z = fdiv(L.z + acc.z * n, d);
-        acc.w = fdiv(L.w + acc.w * n, d);
-    }
-    image[p] = acc;
+    for (uint32_t f = 0; f < a.nFrames; f++)
+        blend_sample(acc, a.samples[(size_t)f * pixels + p], (uint32_t)a.frames[2 * f + 1]);
+    a.image[p] = acc;
 }
 
-__global__ void __launch_bounds__(256) blend_kernel(const float4* samples, const int32_t* frames, uint32_t nf, float4* image,
-                                                    uint32_t pixels)
+// One workgroup per square of 8x8 tiles.  A pixel that misses the box shows the
+// background in every frame and is finished here; masks[square] gets the tiles
+// with a pixel that hits it.
+__global__ void __launch_bounds__(256) squares_kernel(cr::PTArgs a, uint32_t sqX, unsigned long long* masks)
 {
-    const uint32_t p = blockIdx.x * 256 + threadIdx.x;
-    if (p < pixels) blend_pixel(samples, frames, nf, image, pixels, p);
+    __shared__ uint32_t sky;
+    __shared__ unsigned long long mask;
+    if (threadIdx.x == 0) { sky = 0u; mask = 0ull; }
+    __syncthreads();
+    const uint32_t lane = lane_id(), sq = blockIdx.x, tilesY = ((uint32_t)a.H + 7u) >> 3;
+    uint32_t skyPixels = 0;
+    for (uint32_t k = threadIdx.x >> 6; k < 64u; k += 4u) {
+        const uint32_t tx = (sq % sqX) * 8u + (k & 7u), ty = (sq / sqX) * 8u + (k >> 3);
+        if (tx >= a.tilesX || ty >= tilesY) continue;
+        const int32_t x = (int32_t)(tx * 8u + (lane & 7u)), y = (int32_t)(ty * 8u + (lane >> 3));
+        const bool inside = x < a.W && y < a.H;
+        f3 pos, dir;
+        const bool miss = inside && camera_entry(a, x, y, pos, dir);
+        const bool hit = __ballot(inside && !miss) != 0ull;
+        if (lane == 0 && hit) atomicOr(&mask, 1ull << k);
+        if (miss) {
+            skyPixels++;
+            const f4 bg = background(a.ext, dir);
+            const float4 L = make_float4(bg.x, bg.y, bg.z, bg.w);
+            float4* px = a.image + (size_t)y * a.W + x;
+            float4 acc = *px;
+            for (uint32_t f = 0; f < a.nFrames; f++) blend_sample(acc, L, (uint32_t)a.frames[2 * f + 1]);
+            *px = acc;
+        }
+    }
+    if (skyPixels) atomicAdd(&sky, skyPixels);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        masks[sq] = mask;
+        if (sky) {
+            const unsigned long long paths = (unsigned long long)sky * a.nFrames;
+            atomicAdd(a.counters + 0, paths);
+            atomicAdd(a.counters + 1, paths);
+        }
+    }
+}
+
+// The list from the squares' masks: square r goes to part r mod 8; one wave per
+// part, one lane per square.
+__global__ void __launch_bounds__(512) list_kernel(const unsigned long long* masks, uint32_t squares, uint32_t sqX,
+                                                   uint32_t tilesX, uint32_t* list, uint32_t* starts)
+{
+    __shared__ uint32_t total[8];
+    const uint32_t lane = lane_id(), part = threadIdx.x >> 6;
+    const uint32_t mine = squares > part ? (squares - part + 7u) / 8u : 0u;  // squares of this part
+    uint32_t n = 0;
+    for (uint32_t j = lane; j < mine; j += 64u) n += (uint32_t)__popcll(masks[part + 8u * j]);
+    for (int off = 32; off >= 1; off >>= 1) n += (uint32_t)__shfl_xor((int)n, off, 64);
+    if (lane == 0) total[part] = n;
+    __syncthreads();
+    uint32_t at = 0;
+    for (uint32_t k = 0; k < part; k++) at += total[k];
+    if (lane == 0) starts[part] = at;
+    if (threadIdx.x == 511u) starts[8] = at + total[7];
+    for (uint32_t j0 = 0; j0 < mine; j0 += 64u) {
+        const uint32_t j = j0 + lane, sq = j < mine ? part + 8u * j : 0u;
+        unsigned long long m = j < mine ? masks[sq] : 0ull;
+        const uint32_t c = (uint32_t)__popcll(m);
+        uint32_t incl = c;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)incl, off, 64);
+            if (lane >= (uint32_t)off) incl += o;
+        }
+        uint32_t w = at + incl - c;
+        while (m) {
+            const uint32_t k = (uint32_t)__ffsll((long long)m) - 1u;
+            m &= m - 1ull;
+            list[w++] = ((sq / sqX) * 8u + (k >> 3)) * tilesX + (sq % sqX) * 8u + (k & 7u);
+        }
+        at += (uint32_t)__shfl((int)incl, 63, 64);
+    }
+}
+
+__global__ void __launch_bounds__(256) blend_kernel(cr::PTArgs a)
+{
+    const uint32_t p = blockIdx.x * 256 + threadIdx.x, pixels = (uint32_t)a.W * (uint32_t)a.H;
+    if (p >= pixels) return;
+    f3 pos, dir;
+    if (camera_entry(a, (int32_t)(p % (uint32_t)a.W), (int32_t)(p / (uint32_t)a.W), pos, dir)) return;  // see squares_kernel
+    blend_pixel(a, pixels, p);
 }
 
 // The jobs of one batched launch; a job's workgroups start at its blendBase
@@ -52,7 +125,7 @@ __global__ void __launch_bounds__(256) blend_batch_kernel(cr::BatchArgs b)
     const cr::PTArgs& J = b.jobs[lo];
     const uint32_t pixels = (uint32_t)J.W * (uint32_t)J.H;
     const uint32_t p = (blockIdx.x - J.blendBase) * 256 + threadIdx.x;
-    if (p < pixels && J.samples) blend_pixel(J.samples, J.frames, J.nFrames, J.image, pixels, p);
+    if (p < pixels && J.samples) blend_pixel(J, pixels, p);
 }
 
 // out[r] = ((0 + sample 0) + sample 1) + ..., over `total` samples at the end;
@@ -85,11 +158,25 @@ __global__ void __launch_bounds__(64) sum_kernel(const float4* samples, const fl
 
 namespace cr {
 
+// Layout of `lists`: the squares' masks (2 words each), the list, the nine part starts.
+static uint64_t list_squares(const PTArgs& a) { return (uint64_t)((a.W + 63) / 64) * (uint64_t)((a.H + 63) / 64); }
+uint64_t pt_list_starts(const PTArgs& a) { return 2u * list_squares(a) + a.totalIdx / 64u; }
+uint64_t pt_list_words(const PTArgs& a) { return pt_list_starts(a) + 9u; }
+
+hipError_t launch_pt_list(const PTArgs& a, uint32_t* lists, hipStream_t s)
+{
+    const uint32_t n = (uint32_t)list_squares(a), sqX = (uint32_t)(a.W + 63) / 64u;
+    unsigned long long* masks = reinterpret_cast<unsigned long long*>(lists);
+    hipLaunchKernelGGL(squares_kernel, dim3(n), dim3(256), 0, s, a, sqX, masks);
+    hipLaunchKernelGGL(list_kernel, dim3(1), dim3(512), 0, s, masks, n, sqX, a.tilesX, lists + 2u * n,
+                       lists + pt_list_starts(a));
+    return hipGetLastError();
+}
+
 hipError_t launch_pt_blend(const PTArgs& a, hipStream_t s)
 {
     const uint32_t pixels = (uint32_t)a.W * (uint32_t)a.H;
-    hipLaunchKernelGGL(blend_kernel, dim3((pixels + 255) / 256), dim3(256), 0, s, a.samples, a.frames, a.nFrames, a.image,
-                       pixels);
+    hipLaunchKernelGGL(blend_kernel, dim3((pixels + 255) / 256), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -105,16 +192,6 @@ hipError_t launch_pt_sum(const PTArgs& a, uint32_t total, hipStream_t s)
     hipLaunchKernelGGL(sum_kernel, dim3((a.nPoints + 63) / 64), dim3(64), 0, s, a.samples, a.points, a.nPoints, a.spp,
                        a.sample0, total, a.out);
     return hipGetLastError();
-}
-
-uint32_t pt_order_counts(uint32_t n) { return sort_counts_words(n) * 4u; }
-
-hipError_t launch_tile_order(const uint32_t* cost, uint32_t n, uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp,
-                             uint32_t* vals_tmp, uint32_t* counts, hipStream_t s)
-{
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(order_keys_kernel, dim3((n + 255) / 256), dim3(256), 0, s, cost, n, keys, vals);
-    return launch_radix_sort(keys, vals, keys_tmp, vals_tmp, counts, n, s);
 }
 
 hipError_t launch_pt(const PTArgs& a, int dtype, int layout, int blocks, hipStream_t s)

@@ -6,20 +6,25 @@
 // image with the reference's running mean (:420-424).
 //
 // Shape of the computation on CDNA4:
-//  * Persistent grid: a few waves per SIMD loop until a global pixel queue is
+//  * Persistent grid: a few waves per SIMD loop until the pixel queues are
 //    drained.  Lanes claim pixels individually: the wave ballots its idle
 //    lanes, one lane advances the queue counter by the popcount, and each
 //    lane takes base + its rank among the idle lanes.  Claimed indices walk
-//    8x8 pixel tiles so neighbouring lanes trace neighbouring pixels.
+//    8x8 pixel tiles so neighbouring lanes trace neighbouring pixels, and in
+//    renders of several frames squares of 64x64 pixels go to the XCDs in turn,
+//    one queue each, so that rays through one region share an L2 (1080p at 64
+//    spp: 113 -> 66 ms with shadow-volume NEE, 83 -> 64 with brick tracking,
+//    chunks of frames included; a single frame is faster from one queue in
+//    raster order, 1.28 ms against 1.55 at 512x512).
 //  * Path regeneration: a lane renders the frames of its work item back to
 //    back (frame f uses initializeRandom(seed_f * id) exactly as the
-//    reference).  In a large render of many frames an item is a whole pixel,
-//    its running mean kept in registers: 32 B of image traffic per pixel per
-//    launch.  Otherwise it is a chunk of a few frames whose samples go to
+//    reference).  An item is a chunk of a few frames whose samples go to
 //    memory, and a blend kernel forms the mean in frame order (16 B written and
 //    read per sample, under 1% of the time of the paths): 256x256 pixels at 64
-//    spp on a 128^3 cloud went from 10.4 to 3.2 ms, as 65 536 lanes with 64
-//    frames each leave three quarters of the chip's wave slots empty.
+//    spp on a 128^3 cloud went from 10.4 to 2.7 ms, as 65 536 lanes with 64
+//    frames each leave three quarters of the chip's wave slots empty.  Single
+//    frames, and calls that may not allocate, have whole pixels as items and
+//    their running mean in registers.
 //  * Flattened state machine: every loop iteration performs at most one
 //    density lookup per lane (a delta-tracking step of the camera path, or a
 //    ratio-tracking step of a shadow ray); collisions, escapes, frame and
@@ -59,7 +64,6 @@ enum : uint32_t { MODE_PRIMARY = 0, MODE_SHADOW = 1 };
 
 struct Lane {
     uint32_t job;  // batched launch: index into the job table
-    uint32_t cost0;  // the lane's work counters when it took its pixel
     int32_t px, py;
     uint32_t id;
     uint32_t f;
@@ -414,6 +418,19 @@ __device__ __forceinline__ void finish_sample(const cr::PTArgs& a, Lane& L)
     }
 }
 
+// The camera ray of a pixel: its entry point into the box (or the camera
+// position when it misses the box) and direction; true when it misses.
+__device__ __forceinline__ bool camera_entry(const cr::PTArgs& a, int32_t x, int32_t y, f3& pos, f3& dir)
+{
+    f3 cp, cd;
+    camera_ray(a.cam, (float)(x - a.cam.halfWidth), (float)(y - a.cam.halfHeight), cp, cd);
+    float tmax = 0.0f, tmin = 0.0f;
+    const bool miss = !intersect_box(B0(a), B1(a), cp, cd, tmin, tmax) || tmax < 0.0f || a.cloud.densityScaling <= 0.0f;
+    pos = miss ? cp : add(cp, mul(cd, tmax < tmin ? tmax : tmin));
+    dir = cd;
+    return miss;
+}
+
 // The job table of a batched launch lives in dynamic LDS.
 template <bool BATCH> __device__ __forceinline__ cr::PTArgs* job_table();
 template <> __device__ __forceinline__ cr::PTArgs* job_table<false>() { return nullptr; }
@@ -421,6 +438,19 @@ template <> __device__ __forceinline__ cr::PTArgs* job_table<true>()
 {
     extern __shared__ uint64_t pt_job_lds[];
     return reinterpret_cast<cr::PTArgs*>(pt_job_lds);
+}
+
+// The kernel's first argument, read again from the argument segment (scalar
+// loads that hit the constant cache) instead of being kept in scalar registers
+// across the main loop: for the places that run rarely.  The argument block is
+// larger than the scalar register file, and every value the loop keeps spills
+// another one.
+__device__ __forceinline__ const cr::PTArgs& cold_args()
+{
+    typedef const __attribute__((address_space(4))) cr::PTArgs* ConstArgs;
+    ConstArgs p = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const cr::PTArgs*)p;
 }
 
 // Last job whose first work index is <= idx (jobs are stored by increasing base).
@@ -435,12 +465,41 @@ __device__ __forceinline__ uint32_t find_job(const cr::PTArgs* jobs, uint32_t n,
     return lo;
 }
 
+// Work items [at, end) of a part: as the tile list has them, or an equal share.
+template <bool BATCH, int KMODE>
+__device__ __forceinline__ void part_range(const cr::BatchArgs& b, uint32_t part, uint32_t logParts, uint32_t& at, uint32_t& end)
+{
+    if (!BATCH && renders(KMODE)) {
+        const cr::PTArgs& k = cold_args();
+        if (k.partStart) {
+            at = k.partStart[part] * 64u * k.chunks;
+            end = k.partStart[part + 1u] * 64u * k.chunks;
+            return;
+        }
+    }
+    const uint32_t total = BATCH ? b.total : cold_args().totalIdx, units = (total + 63u) >> 6;
+    at = ((units * part) >> logParts) << 6;
+    end = min(((units * (part + 1u)) >> logParts) << 6, total);
+}
+
+// Waves per SIMD the registers are to allow (1: no demand).  Renders of FP32
+// grids with brick tracking take 103 registers unasked and run as well with the
+// 96 that five waves leave each (1080p at 64 spp: 71.3 ms with four waves of
+// either code, 65.9 with five); FP16 grids and the global majorant lose more in
+// the tighter code than the fifth wave brings (1 GiB FP16 grid 326 ms against
+// 404, shadow-volume NEE at 256x256 3.09 against 3.59).
+template <typename T, int TRACK, bool BATCH, int KMODE>
+constexpr int min_waves()
+{
+    return sizeof(T) == 4 && TRACK == CR_TRACK_BRICK_DDA && !BATCH && renders(KMODE) ? 5 : 1;
+}
+
 // BATCH = false: one job, `a0`.  BATCH = true: the jobs of `b`, one shared
 // work queue over the concatenated pixel ranges; every lane follows its own
 // job's arguments (read from LDS), so lanes of one wave may render different
 // jobs.  Per pixel the arithmetic is the same in both forms.
 template <typename T, int LAYOUT, int TRACK, int NEE, bool BATCH, int KMODE>
-__global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
+__global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
 {
     cr::PTArgs* const jobs = job_table<BATCH>();
     if (BATCH) {
@@ -451,7 +510,6 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
         __syncthreads();
     }
     uint32_t* const queue = BATCH ? b.queue : a0.queue;
-    const uint32_t totalIdx = BATCH ? b.total : a0.totalIdx;
     Lane L;
     Counters c = {0, 0, 0, 0, 0};
     uint32_t state = ST_IDLE;
@@ -460,20 +518,39 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
     L.mode = MODE_PRIMARY;
     L.job = 0;
     uint32_t ev = EV_NONE;  // the lane's pending event, resolved in the tail
+    // The work items come in parts, one per XCD (workgroup b runs on XCD b mod 8)
+    // or one in all: the waves of an XCD work on the same regions of the image,
+    // whose rays share its L2, and go on to the next part when theirs is drained.
+    const uint32_t logParts = BATCH ? b.logParts : a0.logParts;
+    uint32_t part = blockIdx.x & ((1u << logParts) - 1u), partsLeft = 1u << logParts;
+    uint32_t partAt, partEnd;
+    part_range<BATCH, KMODE>(b, part, logParts, partAt, partEnd);
 
     for (;;) {
         // ---- claim pixels for idle lanes (wave-wide, one atomic per wave)
         const unsigned long long idle = __ballot(state == ST_IDLE);
         if (idle && (!gated_claims(KMODE, BATCH) ||
                      (uint32_t)__popcll(idle) >= min(CLAIM_MIN_LANES, (uint32_t)__popcll(__ballot(state != ST_DEAD))))) {
-            uint32_t base = 0;
-            const uint32_t leader = (uint32_t)__ffsll((long long)idle) - 1u;
-            if (lane == leader) base = atomicAdd(queue, (uint32_t)__popcll(idle));
-            base = __shfl(base, (int)leader, 64);
+            uint32_t at = 0, end = 0;  // this claim's first item, and the end of the part's
+            if (partsLeft != 0u) {
+                const uint32_t n = (uint32_t)__popcll(idle);
+                const uint32_t leader = (uint32_t)__ffsll((long long)idle) - 1u;
+                uint32_t base = 0;
+                if (lane == leader) base = atomicAdd(queue + part, n);
+                at = partAt + (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
+                end = partEnd;
+                if (at + n >= end) {
+                    part = (part + 1u) & ((1u << logParts) - 1u);
+                    part_range<BATCH, KMODE>(b, part, logParts, partAt, partEnd);
+                    partsLeft--;
+                }
+            } else if (state == ST_IDLE) {
+                state = ST_DEAD;
+            }
             if (state == ST_IDLE) {
-                const uint32_t idx = base + (uint32_t)__popcll(idle & lt_mask);
-                if (idx >= totalIdx) {
-                    state = ST_DEAD;
+                const uint32_t idx = at + (uint32_t)__popcll(idle & lt_mask);
+                if (idx >= end) {
+                    // this part is drained: the lane claims from the next one
                 } else if (KMODE == K_CONTINUE) {
                     // a chunk of one recorded collision's samples, which start in the event loop
                     const uint32_t ch = idx / a0.nPoints;
@@ -488,7 +565,7 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                     L.mode = 0xFFu;
                 } else {
                     const uint32_t j = BATCH ? find_job(jobs, b.nJobs, idx) : 0u;
-                    const cr::PTArgs& J = BATCH ? jobs[j] : a0;
+                    const cr::PTArgs& J = BATCH ? jobs[j] : cold_args();
                     const uint32_t local = BATCH ? idx - J.base : idx;
                     const uint32_t within = local & 63u;
                     uint32_t slot = local >> 6, ch = 0;
@@ -497,8 +574,7 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                         slot = unit / J.chunks;
                         ch = unit - slot * J.chunks;
                     }
-                    // tiles in the order of the previous launch's cost, dearest first, so the
-                    // queue ends on cheap tiles and the last lanes finish together
+                    // the tiles listed for this launch, or all in raster order
                     const uint32_t tile = J.tileOrder ? J.tileOrder[slot] : slot;
                     const uint32_t tl = J.tileLog2W, tw = 1u << tl;
                     const int32_t x = (int32_t)((tile % J.tilesX) * tw + (within & (tw - 1u)));
@@ -512,26 +588,20 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                             float4 v = J.image[(size_t)y * J.W + x];
                             L.acc.x = v.x; L.acc.y = v.y; L.acc.z = v.z; L.acc.w = v.w;
                         }
-                        if (!BATCH) {
-                            f3 cp, cd;
-                            camera_ray(J.cam, (float)(x - J.cam.halfWidth), (float)(y - J.cam.halfHeight), cp, cd);
-                            float tmax = 0.0f, tmin = 0.0f;
-                            L.camMiss = !intersect_box(B0(J), B1(J), cp, cd, tmin, tmax) || tmax < 0.0f ||
-                                        J.cloud.densityScaling <= 0.0f;
-                            L.camPos = L.camMiss ? cp : add(cp, mul(cd, tmax < tmin ? tmax : tmin));
-                            L.camDir = cd;
-                        }
+                        if (!BATCH) L.camMiss = camera_entry(J, x, y, L.camPos, L.camDir);
                         L.f = chunked(KMODE, BATCH) ? ch * J.chunk : 0u;
                         if (chunked(KMODE, BATCH)) L.fEnd = min(J.nFrames, L.f + J.chunk);
                         if (J.nFrames > 0u) {
                             L.seedNext = J.frames[2 * L.f];
                             L.countNext = J.frames[2 * L.f + 1];
                         }
-                        L.cost0 = c.lookups + c.brickVisits;
-                        state = ST_ACTIVE;
-                        ev = EV_NONE;
-                        // start frame 0: handled by the event loop below
-                        L.mode = 0xFFu;  // marker: needs a new sample
+                        // a listed tile's pixels that miss the box were rendered when it was listed
+                        if (!(renders(KMODE) && !BATCH && J.partStart && L.camMiss)) {
+                            state = ST_ACTIVE;
+                            ev = EV_NONE;
+                            // start the first frame: handled by the event loop below
+                            L.mode = 0xFFu;  // marker: needs a new sample
+                        }
                     }
                 }
             }
@@ -570,40 +640,36 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
             bool cam = false;  // batched: a camera ray, its box test after the shared reciprocal below
             if (needSample) {
                 needSample = false;
-                if (L.f >= (chunked(KMODE, BATCH) ? L.fEnd : a.nFrames)) {
-                    if (chunked(KMODE, BATCH) && KMODE != K_RECORD && a.samples) {
+                const cr::PTArgs& k = BATCH ? a : cold_args();
+                if (L.f >= (chunked(KMODE, BATCH) ? L.fEnd : k.nFrames)) {
+                    if (chunked(KMODE, BATCH) && KMODE != K_RECORD && k.samples) {
                         // the samples are stored; the blend (or sum) kernel takes them in order
                     } else if (renders(KMODE)) {
                         float4 o;
                         o.x = L.acc.x; o.y = L.acc.y; o.z = L.acc.z; o.w = L.acc.w;
-                        a.image[(size_t)L.py * a.W + L.px] = o;
-                        if (a.tileCost) {
-                            const uint32_t tl = a.tileLog2W;
-                            const uint32_t tile = ((uint32_t)L.py >> (6u - tl)) * a.tilesX + ((uint32_t)L.px >> tl);
-                            atomicAdd(a.tileCost + tile, (c.lookups + c.brickVisits) - L.cost0);
-                        }
+                        k.image[(size_t)L.py * k.W + L.px] = o;
                     } else if (KMODE == K_CONTINUE) {
-                        const float n = (float)a.spp;
-                        a.out[L.px] = make_float4(fdiv(L.acc.x, n), fdiv(L.acc.y, n), fdiv(L.acc.z, n), fdiv(L.acc.w, n));
+                        const float n = (float)k.spp;
+                        k.out[L.px] = make_float4(fdiv(L.acc.x, n), fdiv(L.acc.y, n), fdiv(L.acc.z, n), fdiv(L.acc.w, n));
                     }
                     state = ST_IDLE;
                     break;
                 }
                 if (KMODE == K_CONTINUE) {
                     // continuation L.f of recorded collision L.px
-                    const float4* r = reinterpret_cast<const float4*>(a.points + (size_t)L.px * 8u);
+                    const float4* r = reinterpret_cast<const float4*>(k.points + (size_t)L.px * 8u);
                     const float4 r0 = r[0], r1 = r[1];
                     if (!(r1.w > 0.5f)) {
                         // not a collision: the path escaped, nothing to continue
                         // (the sum kernel tests the flag itself)
-                        if (!a.samples) a.out[L.px] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                        if (!k.samples) k.out[L.px] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                         state = ST_IDLE;
                         break;
                     }
                     L.pos = mk(r0.x, r0.y, r0.z);
                     L.dir = mk(r0.w, r1.x, r1.y);
                     const uint32_t s0 = __float_as_uint(r1.z);
-                    const uint32_t si = a.sample0 + L.f;
+                    const uint32_t si = k.sample0 + L.f;
                     L.rng = si == 0 ? s0 : continuation_seed(s0, si);
                     L.res.x = 0.0f; L.res.y = 0.0f; L.res.z = 0.0f; L.res.w = 0.0f;
                     L.thr = 1.0f;
@@ -619,13 +685,13 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                 // frames, measures faster forming them per frame)
                 const int32_t seed = L.seedNext;
                 L.count = (uint32_t)L.countNext;
-                if (L.f + 1u < a.nFrames) {
-                    L.seedNext = a.frames[2 * (L.f + 1u)];
-                    L.countNext = a.frames[2 * (L.f + 1u) + 1];
+                if (L.f + 1u < k.nFrames) {
+                    L.seedNext = k.frames[2 * (L.f + 1u)];
+                    L.countNext = k.frames[2 * (L.f + 1u) + 1];
                 }
                 xs_init(L.rng, (uint32_t)seed * L.id);
                 if (BATCH) {
-                    camera_ray(a.cam, (float)(L.px - a.cam.halfWidth), (float)(L.py - a.cam.halfHeight), L.pos, L.dir);
+                    camera_ray(k.cam, (float)(L.px - k.cam.halfWidth), (float)(L.py - k.cam.halfHeight), L.pos, L.dir);
                 } else {
                     L.pos = L.camPos;
                     L.dir = L.camDir;
@@ -657,7 +723,7 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
             } else {  // EV_COLLIDE
                 if (KMODE == K_RECORD && L.bounces == 0) {
                     // first real collision: record it and end the frame here
-                    float4* r = reinterpret_cast<float4*>(record_of(a, L));
+                    float4* r = reinterpret_cast<float4*>(record_of(BATCH ? a : cold_args(), L));
                     r[0] = make_float4(L.pos.x, L.pos.y, L.pos.z, L.dir.x);
                     r[1] = make_float4(L.dir.y, L.dir.z, __uint_as_float(L.rng), 1.0f);
                     L.f++;
@@ -714,7 +780,7 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                 }
             }
             if (sky) {
-                const f4 bg = background(a.ext, L.dir);
+                const f4 bg = background((BATCH ? a : cold_args()).ext, L.dir);
                 if (missed) {
                     L.res = bg;
                 } else {
@@ -723,7 +789,7 @@ __global__ void __launch_bounds__(256) pt_kernel(cr::PTArgs a0, cr::BatchArgs b)
                 fin = true;
             }
             if (fin) {
-                finish_sample<KMODE, BATCH>(a, L);
+                finish_sample<KMODE, BATCH>(BATCH ? a : cold_args(), L);
                 L.f++;
                 ev = EV_NONE;
                 needSample = true;
