@@ -112,7 +112,7 @@ struct GatherArgs {
     float4* image;
     int32_t W, H;
     uint32_t padded;
-    unsigned long long* counters;    // rays, nodesVisited, beamsTested
+    unsigned long long* counters;    // COUNTER_SLOTS x (rays, nodesVisited, beamsTested)
     uint32_t* overflow;              // set when a traversal stack would overflow
 };
 hipError_t launch_gather(const GatherArgs& a, int dtype, int layout, hipStream_t s);

@@ -118,8 +118,8 @@ cr_status cr_create(int device, cr_context** out)
     cr_shadow_volume_default(&ctx->svp);
     cr_render_ext_default(&ctx->ext);
     cr_photon_map_default(&ctx->pm);
-    if (ensure_buffer(ctx, (void**)&ctx->dQueue, &ctx->queueCap, 64, "queue") != CR_OK ||
-        ensure_buffer(ctx, (void**)&ctx->dCounters, &ctx->countersCap, 16 * sizeof(unsigned long long), "counters") != CR_OK ||
+    if (ensure_buffer(ctx, (void**)&ctx->dQueue, &ctx->queueCap, PT_QUEUE_WORDS * 4, "queue") != CR_OK ||
+        ensure_buffer(ctx, (void**)&ctx->dCounters, &ctx->countersCap, COUNTER_WORDS * sizeof(unsigned long long), "counters") != CR_OK ||
         ensure_buffer(ctx, (void**)&ctx->dScalar, &ctx->scalarCap, 64, "scalar") != CR_OK) {
         cr_destroy(ctx);
         return CR_ERR_OUT_OF_MEMORY;
@@ -128,7 +128,7 @@ cr_status cr_create(int device, cr_context** out)
         cr_destroy(ctx);
         return CR_ERR_DEVICE;
     }
-    zero_async(ctx->dCounters, 16 * sizeof(unsigned long long), ctx->stream);
+    zero_async(ctx->dCounters, COUNTER_WORDS * sizeof(unsigned long long), ctx->stream);
     hipStreamSynchronize(ctx->stream);
     *out = ctx;
     return CR_OK;
@@ -740,6 +740,18 @@ bool sample_buffer(float4** p, size_t* cap, uint64_t count)
     return true;
 }
 
+cr_status read_counters(cr_context* ctx, const unsigned long long* slots, unsigned long long* out, uint32_t n)
+{
+    std::vector<unsigned long long> c(COUNTER_WORDS);
+    CR_HIP(ctx, hipMemcpyAsync(c.data(), slots, COUNTER_WORDS * sizeof(c[0]), hipMemcpyDeviceToHost, ctx->stream), "copy counters");
+    CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
+    for (uint32_t i = 0; i < n; i++) {
+        out[i] = 0;
+        for (uint32_t s = 0; s < COUNTER_SLOTS; s++) out[i] += c[s * COUNTER_STRIDE + i];
+    }
+    return CR_OK;
+}
+
 cr_status fill_pt_args(cr_context* ctx, PTArgs& a, uint32_t n_frames)
 {
     fill_job_args(a, ctx->grid, ctx->sv, ctx->svDimsBuilt, ctx->cam, ctx->cloud, ctx->params, ctx->svp, ctx->ext,
@@ -847,15 +859,15 @@ cr_status cr_pt_stats_get(cr_context* ctx, cr_pt_stats* out)
 {
     CR_CHECK_CTX(ctx);
     if (!out) return fail(ctx, CR_ERR_INVALID_ARGUMENT, "null output");
-    unsigned long long c[8];
-    CR_HIP(ctx, hipMemcpyAsync(c, ctx->dCounters, sizeof(c), hipMemcpyDeviceToHost, ctx->stream), "copy counters");
-    CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
+    unsigned long long c[5];
+    cr_status st = read_counters(ctx, ctx->dCounters, c, 5);
+    if (st != CR_OK) return st;
     out->paths = c[0];
     out->vertices = c[1];
     out->lookups = c[2];
     out->svLookups = c[3];
     out->brickVisits = c[4];
-    cr_status st = fold_pt_events(ctx);
+    st = fold_pt_events(ctx);
     if (st != CR_OK) return st;
     out->lastKernelMs = ctx->ptLastMs;
     out->totalKernelMs = ctx->ptTotalMs;
@@ -870,7 +882,7 @@ cr_status cr_pt_stats_reset(cr_context* ctx)
     if (st != CR_OK) return st;
     ctx->ptTotalMs = 0.0;
     ctx->ptLaunches = 0;
-    CR_HIP(ctx, zero_async(ctx->dCounters, 8 * sizeof(unsigned long long), ctx->stream), "zero counters");
+    CR_HIP(ctx, zero_async(ctx->dCounters, COUNTER_WORDS * sizeof(unsigned long long), ctx->stream), "zero counters");
     return CR_OK;
 }
 

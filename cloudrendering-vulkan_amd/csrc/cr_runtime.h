@@ -104,6 +104,8 @@ cr_status fail(cr_context* ctx, cr_status code, const std::string& msg);
 cr_status hip_fail(cr_context* ctx, hipError_t e, const char* what);
 cr_status ensure_buffer(cr_context* ctx, void** p, size_t* cap, size_t bytes, const char* what);
 hipError_t zero_async(void* p, size_t bytes, hipStream_t s);
+// The first n statistics counters, summed over their COUNTER_SLOTS copies (synchronises the stream).
+cr_status read_counters(cr_context* ctx, const unsigned long long* slots, unsigned long long* out, uint32_t n);
 cr_status upload_frames(cr_context* ctx, const cr_push_constants* frames, uint32_t n);
 int majorant_brick(const cr_render_ext& e);
 void fill_job_args(PTArgs& a, const DeviceGrid& g, const float* sv, const uint32_t svDims[3],

@@ -69,8 +69,8 @@ struct Batch {
     size_t tableCap = 0;
     PTArgs* dTuneTable = nullptr;   // autotuner trial table
     size_t tuneTableCap = 0;
-    uint32_t* dQueue = nullptr;     // [0] render queue, [16] trial queue
-    unsigned long long* dCounters = nullptr;   // [0..7] render, [8..15] trials
+    uint32_t* dQueue = nullptr;     // render queue, then trial queue
+    unsigned long long* dCounters = nullptr;   // renders; trials are not counted
     float* dScratch = nullptr;      // trial images
     size_t scratchCap = 0;
     float4* dSamples = nullptr;     // a launch group's samples
@@ -110,9 +110,9 @@ cr_status ensure_batch(cr_context* ctx)
     if (ctx->batch) return CR_OK;
     Batch* b = new Batch();
     cr_batch_tuning_default(&b->tuning);
-    hipError_t e = hipMalloc((void**)&b->dQueue, 32 * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void**)&b->dCounters, 16 * sizeof(unsigned long long));
-    if (e == hipSuccess) e = zero_async(b->dCounters, 16 * sizeof(unsigned long long), ctx->stream);
+    hipError_t e = hipMalloc((void**)&b->dQueue, 2 * PT_QUEUE_WORDS * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMalloc((void**)&b->dCounters, COUNTER_WORDS * sizeof(unsigned long long));
+    if (e == hipSuccess) e = zero_async(b->dCounters, COUNTER_WORDS * sizeof(unsigned long long), ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     ctx->batch = b;
     if (e != hipSuccess) {
@@ -277,7 +277,7 @@ cr_status trial(cr_context* ctx, Batch* b, const std::vector<uint32_t>& which, c
     float best = 1e30f;
     for (int r = 0; r <= reps && e == hipSuccess; r++) {
         e = hipEventRecord(e0, ctx->stream);
-        if (e == hipSuccess) e = enqueue_groups(ctx, b, groups, b->dTuneTable, t, b->dQueue + 16, b->dCounters + 8);
+        if (e == hipSuccess) e = enqueue_groups(ctx, b, groups, b->dTuneTable, t, b->dQueue + PT_QUEUE_WORDS, nullptr);
         if (e == hipSuccess) e = hipEventRecord(e1, ctx->stream);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
         float ms = 0.0f;
@@ -574,15 +574,15 @@ cr_status cr_batch_stats_get(cr_context* ctx, cr_pt_stats* out)
     memset(out, 0, sizeof(*out));
     Batch* b = ctx->batch;
     if (!b) return CR_OK;
-    unsigned long long c[8];
-    CR_HIP(ctx, hipMemcpyAsync(c, b->dCounters, sizeof(c), hipMemcpyDeviceToHost, ctx->stream), "copy counters");
-    CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
+    unsigned long long c[5];
+    cr_status st = read_counters(ctx, b->dCounters, c, 5);
+    if (st != CR_OK) return st;
     out->paths = c[0];
     out->vertices = c[1];
     out->lookups = c[2];
     out->svLookups = c[3];
     out->brickVisits = c[4];
-    cr_status st = fold_events(ctx, b);
+    st = fold_events(ctx, b);
     if (st != CR_OK) return st;
     out->lastKernelMs = b->lastMs;
     out->totalKernelMs = b->totalMs;
@@ -597,7 +597,7 @@ cr_status cr_batch_stats_reset(cr_context* ctx)
     if (!b) return CR_OK;
     cr_status st = fold_events(ctx, b);
     if (st != CR_OK) return st;
-    CR_HIP(ctx, zero_async(b->dCounters, 8 * sizeof(unsigned long long), ctx->stream), "zero counters");
+    CR_HIP(ctx, zero_async(b->dCounters, COUNTER_WORDS * sizeof(unsigned long long), ctx->stream), "zero counters");
     CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
     b->totalMs = 0.0;
     b->lastMs = 0.0f;

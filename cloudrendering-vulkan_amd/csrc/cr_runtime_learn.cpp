@@ -216,7 +216,7 @@ cr_status record_pass(cr_context* ctx, Learn* L, const cr_push_constants* frames
     CR_TRY(fill_pt_args(ctx, a, n_frames));
     set_chunk(a, pt_chunk((uint64_t)ctx->W * (uint64_t)ctx->H, n_frames, (uint64_t)pass_blocks(ctx, 0, ~0u) * 256u, PT_CHUNK_RECORD));
     a.records = L->records;
-    a.counters = ctx->dCounters + 8;
+    a.counters = nullptr;
     CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
     CR_HIP(ctx, launch_pt_record(a, ctx->grid.dtype, ctx->grid.layout, pass_blocks(ctx, 0, a.totalIdx), ctx->stream),
            "record pass");
@@ -238,7 +238,7 @@ cr_status continue_pass(cr_context* ctx, const float* pts, uint32_t m, uint32_t 
     a.points = pts;
     a.out = reinterpret_cast<float4*>(out);
     a.nPoints = m;
-    a.counters = ctx->dCounters + 8;
+    a.counters = nullptr;
     uint32_t group = spp;
     if (spp > 1) {
         group = (uint32_t)std::min<uint64_t>(spp, std::max<uint64_t>(1, PT_SAMPLE_BUDGET / m));

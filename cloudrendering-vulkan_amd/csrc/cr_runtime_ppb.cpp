@@ -74,11 +74,11 @@ static cr_status ppb_get(cr_context* ctx, Ppb** out)
         Ppb* p = new Ppb();
         for (hipEvent_t& e : p->ev) hipEventCreate(&e);
         ctx->ppb = p;
-        cr_status st = ensure_buffer(ctx, (void**)&p->gcounters, &p->gcountersCap, 8 * sizeof(unsigned long long), "gather counters");
+        cr_status st = ensure_buffer(ctx, (void**)&p->gcounters, &p->gcountersCap, COUNTER_WORDS * sizeof(unsigned long long), "gather counters");
         if (st != CR_OK) return st;
         st = ensure_buffer(ctx, (void**)&p->overflow, &p->overflowCap, 64, "overflow flag");
         if (st != CR_OK) return st;
-        zero_async(p->gcounters, 8 * sizeof(unsigned long long), ctx->stream);
+        zero_async(p->gcounters, COUNTER_WORDS * sizeof(unsigned long long), ctx->stream);
         zero_async(p->overflow, 4, ctx->stream);
     }
     *out = ctx->ppb;
@@ -450,8 +450,7 @@ cr_status cr_gather_stats_get(cr_context* ctx, cr_gather_stats* out)
     Ppb* p;
     CR_TRY(ppb_get(ctx, &p));
     unsigned long long c[3];
-    CR_HIP(ctx, hipMemcpyAsync(c, p->gcounters, sizeof(c), hipMemcpyDeviceToHost, ctx->stream), "copy counters");
-    CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
+    CR_TRY(read_counters(ctx, p->gcounters, c, 3));
     out->rays = c[0];
     out->nodesVisited = c[1];
     out->beamsTested = c[2];

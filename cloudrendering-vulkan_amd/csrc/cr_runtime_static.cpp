@@ -25,10 +25,8 @@ using namespace cr;
 
 namespace {
 
-// Layout: [0, 64) work-queue counter, [64, 192) 16 statistics counters,
-// [256, 256 + 8 CR_PT_STATIC_MAX_FRAMES) the (seed, frameCount) pairs.
+// Layout: [0, 64) work-queue counter, [256, 256 + 8 CR_PT_STATIC_MAX_FRAMES) the (seed, frameCount) pairs.
 constexpr size_t QUEUE_OFF = 0;
-constexpr size_t COUNTERS_OFF = 64;
 constexpr size_t FRAMES_OFF = 256;
 static_assert(FRAMES_OFF + 8ull * CR_PT_STATIC_MAX_FRAMES == CR_PT_STATIC_SCRATCH_BYTES, "scratch layout");
 
@@ -95,13 +93,13 @@ cr_status cr_pt_render_static(cr_context* ctx, const cr_push_constants* frames, 
     // stream order: the copy waits for any earlier kernel that still reads the table
     CR_HIP(ctx, hipMemcpyAsync(dFrames, fr, (size_t)n_frames * 8, hipMemcpyHostToDevice, ctx->stream), "copy frames");
     CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync frames");
-    CR_HIP(ctx, zero_async(base + QUEUE_OFF, FRAMES_OFF - QUEUE_OFF, ctx->stream), "clear queue and counters");
+    CR_HIP(ctx, zero_async(base + QUEUE_OFF, 64, ctx->stream), "clear queue");
 
     PTArgs a;
     fill_job_args(a, ctx->grid, ctx->sv, ctx->svDimsBuilt, ctx->cam, ctx->cloud, ctx->params, ctx->svp, ctx->ext,
                   dFrames, n_frames, accum, ctx->W, ctx->H, ctx->ptTileLog2W);
     a.queue = (uint32_t*)(base + QUEUE_OFF);
-    a.counters = (unsigned long long*)(base + COUNTERS_OFF);
+    a.counters = nullptr;
     const DeviceGrid& g = ctx->grid;
     int blocks = ctx->numCUs * pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, n_frames);
     const uint32_t needed = (a.totalIdx + 255u) / 256u;

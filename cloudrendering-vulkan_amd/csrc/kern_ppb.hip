@@ -19,6 +19,7 @@
 // written; boxes are tested with half their size (the reference passes the
 // full size to intersectBox, PPB_PE.comp:424-431).
 #include "cr_device.h"
+#include "cr_internal.h"
 #include "cr_internal_ppb.h"
 #include "row_walk.h"
 
@@ -499,9 +500,11 @@ __global__ void __launch_bounds__(GATHER_THREADS, 4) gather_kernel(cr::GatherArg
     }
     const unsigned long long s0 = wave_sum_u64(rays), s1 = wave_sum_u64(visited), s2 = wave_sum_u64(tested);
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(a.counters + 0, s0);
-        atomicAdd(a.counters + 1, s1);
-        atomicAdd(a.counters + 2, s2);
+        unsigned long long* const cnt =
+            a.counters + ((blockIdx.x + blockIdx.y * gridDim.x) % cr::COUNTER_SLOTS) * cr::COUNTER_STRIDE;
+        atomicAdd(cnt + 0, s0);
+        atomicAdd(cnt + 1, s1);
+        atomicAdd(cnt + 2, s2);
     }
 }
 

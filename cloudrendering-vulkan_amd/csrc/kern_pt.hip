@@ -60,8 +60,9 @@ __global__ void __launch_bounds__(256) squares_kernel(cr::PTArgs a, uint32_t sqX
         masks[sq] = mask;
         if (sky) {
             const unsigned long long paths = (unsigned long long)sky * a.nFrames;
-            atomicAdd(a.counters + 0, paths);
-            atomicAdd(a.counters + 1, paths);
+            unsigned long long* const cnt = a.counters + (sq % cr::COUNTER_SLOTS) * cr::COUNTER_STRIDE;
+            atomicAdd(cnt + 0, paths);
+            atomicAdd(cnt + 1, paths);
         }
     }
 }

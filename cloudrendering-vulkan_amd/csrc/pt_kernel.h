@@ -482,6 +482,12 @@ __device__ __forceinline__ void part_range(const cr::BatchArgs& b, uint32_t part
     end = min(((units * (part + 1u)) >> logParts) << 6, total);
 }
 
+// Items of a part that its waves (four per workgroup) start with.
+__device__ __forceinline__ uint32_t part_first(uint32_t part, uint32_t logParts)
+{
+    return ((gridDim.x - part + (1u << logParts) - 1u) >> logParts) << 8;
+}
+
 // Waves per SIMD the registers are to allow (1: no demand).  Renders of FP32
 // grids with brick tracking take 103 registers unasked and run as well with the
 // 96 that five waves leave each (1080p at 64 spp: 71.3 ms with four waves of
@@ -525,6 +531,13 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
     uint32_t part = blockIdx.x & ((1u << logParts) - 1u), partsLeft = 1u << logParts;
     uint32_t partAt, partEnd;
     part_range<BATCH, KMODE>(b, part, logParts, partAt, partEnd);
+    // In renders each wave's first 64 items are set by its number in the part and
+    // the queue deals out those after them: the waves of a launch need not wait
+    // for each other's atomics (512x512 at 1 spp 1.00 -> 0.93 ms).
+    constexpr bool FIRST_SET = renders(KMODE) && !BATCH;
+    const uint32_t first = partAt + (((blockIdx.x >> logParts) * 4u + (threadIdx.x >> 6)) << 6);
+    bool started = !FIRST_SET;
+    if (FIRST_SET) partAt += part_first(part, logParts);
 
     for (;;) {
         // ---- claim pixels for idle lanes (wave-wide, one atomic per wave)
@@ -536,14 +549,20 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
                 const uint32_t n = (uint32_t)__popcll(idle);
                 const uint32_t leader = (uint32_t)__ffsll((long long)idle) - 1u;
                 uint32_t base = 0;
-                if (lane == leader) base = atomicAdd(queue + part, n);
-                at = partAt + (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
+                if (started) {
+                    if (lane == leader) base = atomicAdd(queue + part * cr::PT_QUEUE_STRIDE, n);
+                    at = partAt + (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
+                } else {
+                    at = first;
+                }
                 end = partEnd;
-                if (at + n >= end) {
+                if (started && at + n >= end) {
                     part = (part + 1u) & ((1u << logParts) - 1u);
                     part_range<BATCH, KMODE>(b, part, logParts, partAt, partEnd);
+                    if (FIRST_SET) partAt += part_first(part, logParts);
                     partsLeft--;
                 }
+                started = true;
             } else if (state == ST_IDLE) {
                 state = ST_DEAD;
             }
@@ -800,11 +819,13 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
         }
     }
 
-    // ---- counters: one atomic per wave (all lanes have reconverged here)
+    // ---- counters: one atomic each per wave (all lanes have reconverged here)
+    unsigned long long* cnt = BATCH ? b.counters : a0.counters;
+    if (!cnt) return;
+    cnt += (blockIdx.x % cr::COUNTER_SLOTS) * cr::COUNTER_STRIDE;
     unsigned long long s0 = wave_sum_u64(c.paths), s1 = wave_sum_u64(c.vertices), s2 = wave_sum_u64(c.lookups);
     unsigned long long s3 = wave_sum_u64(c.svLookups), s4 = wave_sum_u64(c.brickVisits);
     if (lane == 0) {
-        unsigned long long* const cnt = BATCH ? b.counters : a0.counters;
         atomicAdd(cnt + 0, s0);
         atomicAdd(cnt + 1, s1);
         atomicAdd(cnt + 2, s2);
