@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/cr/abi.h"
+#include "cr_device.h"
 
 namespace cr {
 
@@ -39,9 +40,12 @@ struct PTArgs {
     cr_camera_properties cam;
     cr_cloud_properties cloud;
     cr_parameters params;
-    cr_shadow_volume_properties svp;
+    float lightDirection[3];
     cr_render_ext ext;
-    float sigmaBar;
+    crd::BoxMap box;
+    crd::SvMap svMap;
+    crd::Divisor sigmaDiv;  // (maxExtinction * densityScaling) / baseScaling
+    crd::Divisor extDiv;    // maxExtinction
     // frames
     const int32_t* frames;  // pairs (seed, frameCount)
     uint32_t nFrames;
@@ -151,6 +155,8 @@ struct SVArgs {
     const void* grid;
     int32_t nx, ny, nz, nbx, nby;
     cr_cloud_properties cloud;
+    crd::BoxMap box;
+    crd::Divisor scaleDiv;  // baseScaling
     cr_shadow_volume_properties svp;
     float* out;
     int32_t dx, dy, dz;

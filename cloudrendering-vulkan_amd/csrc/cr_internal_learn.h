@@ -36,6 +36,7 @@ struct FirstNee {
     const float* sv;
     int32_t svx, svy, svz;
     cr_shadow_volume_properties svp;
+    crd::SvMap svMap;
     cr_parameters params;
     float intensity;
     float albedo;

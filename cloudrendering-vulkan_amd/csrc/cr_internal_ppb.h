@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/cr/abi.h"
+#include "cr_device.h"
 
 namespace cr {
 
@@ -70,6 +71,8 @@ struct TraceArgs {
     const void* grid;
     int32_t nx, ny, nz, nbx, nby;
     cr_cloud_properties cloud;
+    crd::BoxMap box;
+    crd::Divisor sigmaDiv, extDiv;  // majorant in world units, maxExtinction
     cr_parameters params;
     cr_beam_trace_params p;
     uint32_t firstPath, nPaths;  // trace: the launch's paths; expand: paths that have offsets

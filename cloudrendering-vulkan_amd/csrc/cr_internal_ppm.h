@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/cr/abi.h"
+#include "cr_device.h"
 
 namespace cr {
 
@@ -25,6 +26,8 @@ constexpr uint32_t PPM_CHUNK = 16;   // record slots a path takes at a time afte
 struct PpmTraceArgs {
     PpmGrid g;
     cr_cloud_properties cloud;
+    crd::BoxMap box;
+    crd::Divisor sigmaDiv, extDiv;  // majorant in world units, maxExtinction
     cr_parameters params;
     cr_photon_map_properties pm;
     cr_render_ext ext;          // the sky the sky photons carry
@@ -50,6 +53,9 @@ struct PpmEstimateArgs {
     int32_t svx, svy, svz;
     cr_camera_properties cam;
     cr_cloud_properties cloud;
+    crd::BoxMap box;
+    crd::SvMap svMap;
+    crd::Divisor scaleDiv, cellDiv;  // baseScaling, the photon grid's voxelSize
     cr_parameters params;
     cr_shadow_volume_properties svp;
     cr_photon_map_properties pm;

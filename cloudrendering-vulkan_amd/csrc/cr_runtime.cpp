@@ -603,6 +603,8 @@ cr_status cr_sv_build(cr_context* ctx)
     const DeviceGrid& g = ctx->grid;
     a.grid = g.data; a.nx = g.nx; a.ny = g.ny; a.nz = g.nz; a.nbx = g.nbx; a.nby = g.nby;
     a.cloud = ctx->cloud;
+    a.box = crd::make_box_map(ctx->cloud);
+    a.scaleDiv = crd::make_divisor(ctx->cloud.baseScaling);
     a.svp = ctx->svp;
     a.out = ctx->sv;
     a.dx = (int32_t)d[0]; a.dy = (int32_t)d[1]; a.dz = (int32_t)d[2];
@@ -694,9 +696,12 @@ void fill_job_args(PTArgs& a, const DeviceGrid& g, const float* sv, const uint32
     a.cam = cam;
     a.cloud = cloud;
     a.params = params;
-    a.svp = svp;
+    for (int k = 0; k < 3; k++) a.lightDirection[k] = svp.lightDirection[k];
     a.ext = ext;
-    a.sigmaBar = (cloud.maxExtinction * cloud.densityScaling) / cloud.baseScaling;
+    a.box = crd::make_box_map(cloud);
+    a.svMap = crd::make_sv_map(svp);
+    a.sigmaDiv = crd::make_divisor((cloud.maxExtinction * cloud.densityScaling) / cloud.baseScaling);
+    a.extDiv = crd::make_divisor(cloud.maxExtinction);
     a.frames = frames;
     a.nFrames = n_frames;
     a.image = (float4*)image;

@@ -61,6 +61,7 @@ FirstNee first_nee_of(const cr_context* ctx)
     e.svy = (int32_t)ctx->svDimsBuilt[1];
     e.svz = (int32_t)ctx->svDimsBuilt[2];
     e.svp = ctx->svp;
+    e.svMap = crd::make_sv_map(ctx->svp);
     e.params = ctx->params;
     e.intensity = ctx->params.lightIntensity;
     e.albedo = ctx->ext.albedo;

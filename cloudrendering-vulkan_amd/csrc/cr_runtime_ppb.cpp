@@ -186,6 +186,9 @@ cr_status cr_ppb_trace_beams(cr_context* ctx, const cr_beam_trace_params* prm, u
     memset(&a, 0, sizeof(a));
     a.grid = g.data; a.nx = g.nx; a.ny = g.ny; a.nz = g.nz; a.nbx = g.nbx; a.nby = g.nby;
     a.cloud = ctx->cloud;
+    a.box = crd::make_box_map(ctx->cloud);
+    a.sigmaDiv = crd::make_divisor((ctx->cloud.maxExtinction * ctx->cloud.densityScaling) / ctx->cloud.baseScaling);
+    a.extDiv = crd::make_divisor(ctx->cloud.maxExtinction);
     a.params = ctx->params;
     a.p = *prm;
     // Paths are traced in order, in launches, until they fill max_beams: the

@@ -181,6 +181,9 @@ cr_status cr_ppm_trace(cr_context* ctx, int32_t seed, const cr_ppm_params* prm, 
     memset(&a, 0, sizeof(a));
     a.g = grid_args(ctx);
     a.cloud = ctx->cloud;
+    a.box = crd::make_box_map(ctx->cloud);
+    a.sigmaDiv = crd::make_divisor((ctx->cloud.maxExtinction * ctx->cloud.densityScaling) / ctx->cloud.baseScaling);
+    a.extDiv = crd::make_divisor(ctx->cloud.maxExtinction);
     a.params = ctx->params;
     a.pm = ctx->pm;
     a.ext = ctx->ext;
@@ -295,6 +298,10 @@ cr_status cr_ppm_estimate(cr_context* ctx, const cr_push_constants* frames, uint
     a.svx = (int32_t)ctx->svDimsBuilt[0]; a.svy = (int32_t)ctx->svDimsBuilt[1]; a.svz = (int32_t)ctx->svDimsBuilt[2];
     a.cam = ctx->cam;
     a.cloud = ctx->cloud;
+    a.box = crd::make_box_map(ctx->cloud);
+    a.svMap = crd::make_sv_map(ctx->svp);
+    a.scaleDiv = crd::make_divisor(ctx->cloud.baseScaling);
+    a.cellDiv = crd::make_divisor(ctx->pm.voxelSize);
     a.params = ctx->params;
     a.svp = ctx->svp;
     a.pm = ctx->pm;

@@ -186,7 +186,7 @@ __device__ __forceinline__ float first_nee(const cr::FirstNee& e, f3 pos, f3 dir
     const float w = 1.0f * e.albedo;
     GridView g;
     g.data = e.sv; g.nx = e.svx; g.ny = e.svy; g.nz = e.svz; g.nbx = 0; g.nby = 0;
-    const float Tv = trilinear<float, LAYOUT_DENSE>(g, sv_norm(e.svp, pos));
+    const float Tv = trilinear<float, LAYOUT_DENSE>(g, sv_norm(e.svMap, pos));
     return (((1.0f * e.intensity) * pdf) * Tv) * w;
 }
 

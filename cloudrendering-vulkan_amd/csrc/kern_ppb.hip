@@ -32,13 +32,13 @@ constexpr uint32_t NONE = 0xFFFFFFFFu;
 // unit box with majorant 64 takes ~64 steps); it only bounds the loop.
 constexpr uint32_t TRACK_CEILING = 1u << 16;
 
-template <typename T, int LAYOUT>
+template <typename T, int LAYOUT, class Map>
 __device__ __forceinline__ float cloud_at(const void* grid, int32_t nx, int32_t ny, int32_t nz, int32_t nbx, int32_t nby,
-                                          const cr_cloud_properties& cp, f3 p)
+                                          const Map& map, f3 p)
 {
     GridView g;
     g.data = grid; g.nx = nx; g.ny = ny; g.nz = nz; g.nbx = nbx; g.nby = nby;
-    return trilinear<T, LAYOUT>(g, cloud_norm(cp, p));
+    return trilinear<T, LAYOUT>(g, cloud_norm(map, p));
 }
 
 // scatterRay of PPB_PT.comp:268-304 (with the final normalize).
@@ -126,7 +126,6 @@ __global__ void __launch_bounds__(256) trace_kernel(cr::TraceArgs a)
         }
         f3 dir = L;
         const float r = a.p.radius;
-        const float sigmaBar = fdiv(cp.maxExtinction * cp.densityScaling, cp.baseScaling);
         const float absorption = 1.0f - a.p.albedo;
         bool alive = a.p.maxInteractions > 0u;
         float len = 0.0f, tr = 0.0f, t = 0.0f;
@@ -138,8 +137,8 @@ __global__ void __launch_bounds__(256) trace_kernel(cr::TraceArgs a)
         }
         while (alive) {
             bool hit = false;
-            bool end = row_walk(R, sigmaBar, cp.maxExtinction, len, t, rng, hit, [&](float d) {
-                return cloud_at<T, LAYOUT>(a.grid, a.nx, a.ny, a.nz, a.nbx, a.nby, cp, add(pos, mul(dir, d)));
+            bool end = row_walk(R, a.sigmaDiv, a.extDiv, len, t, rng, hit, [&](float d) {
+                return cloud_at<T, LAYOUT>(a.grid, a.nx, a.ny, a.nz, a.nbx, a.nby, a.box, add(pos, mul(dir, d)));
             });
             if (++rounds == TRACK_CEILING / ROW) end = true;
             if (!end) continue;

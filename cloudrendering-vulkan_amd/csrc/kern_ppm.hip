@@ -27,11 +27,11 @@ constexpr uint32_t TRACK_CEILING = 1u << 16;   // delta-tracking steps of one fl
 constexpr uint32_t MARCH_CEILING = 1u << 16;   // estimate steps per pixel, sky-ray steps per estimate step
 
 template <typename T, int LAYOUT>
-__device__ __forceinline__ float density(const cr::PpmGrid& g, const cr_cloud_properties& cp, f3 p)
+__device__ __forceinline__ float density(const cr::PpmGrid& g, const BoxMap& box, f3 p)
 {
     GridView v;
     v.data = g.grid; v.nx = g.nx; v.ny = g.ny; v.nz = g.nz; v.nbx = g.nbx; v.nby = g.nby;
-    return trilinear<T, LAYOUT>(v, cloud_norm(cp, p));
+    return trilinear<T, LAYOUT, true>(v, cloud_norm(box, p));
 }
 
 // Entry point on the faces a ray of direction d enters the box through,
@@ -102,7 +102,6 @@ __global__ void __launch_bounds__(64) ppm_trace_kernel(cr::PpmTraceArgs a)
             col.z = fdiv(fdiv(bg.z, k) * 0.5f, q) * 0.5f;
             col.w = fdiv(fdiv(bg.w, k) * 0.5f, q) * 0.5f;
         }
-        const float sigmaBar = fdiv(cp.maxExtinction * cp.densityScaling, cp.baseScaling);
         bool first = true;
         uint64_t slot = (uint64_t)id * cr::PPM_FIRST;  // of the deposits being written
         unsigned long long chunk = 0;
@@ -115,11 +114,11 @@ __global__ void __launch_bounds__(64) ppm_trace_kernel(cr::PpmTraceArgs a)
             f3 cur = pos;
             bool hit = false;
             for (uint32_t step = 0; step < TRACK_CEILING; step++) {
-                t = t + fdiv(-crd_logf(xs_float(rng)), sigmaBar);
+                t = t + div1(a.sigmaDiv, -crd_logf(xs_float(rng)));
                 if (!(t <= dist)) break;
                 cur = add(pos, mul(dir, t));
-                const float e = density<T, LAYOUT>(a.g, cp, cur);
-                if (xs_float(rng) < fdiv(e, cp.maxExtinction)) { hit = true; break; }
+                const float e = density<T, LAYOUT>(a.g, a.box, cur);
+                if (xs_float(rng) < div1(a.extDiv, e)) { hit = true; break; }
             }
             if (!hit) break;
             pos = cur;
@@ -219,12 +218,12 @@ __device__ __forceinline__ f4 photon_query(const cr::PpmEstimateArgs& a, f3 p, f
     if (scatter == 0.0f) return acc;
     const cr_photon_map_properties& pm = a.pm;
     const f3 g = sub(p, ld3(pm.bounds[0]));
-    const int32_t x0 = max((int32_t)fdiv(g.x - r, pm.voxelSize), 0);
-    const int32_t x1 = min((int32_t)fdiv(g.x + r, pm.voxelSize), pm.voxelCount[0] - 1);
-    const int32_t y0 = max((int32_t)fdiv(g.y - r, pm.voxelSize), 0);
-    const int32_t y1 = min((int32_t)fdiv(g.y + r, pm.voxelSize), pm.voxelCount[1] - 1);
-    const int32_t z0 = max((int32_t)fdiv(g.z - r, pm.voxelSize), 0);
-    const int32_t z1 = min((int32_t)fdiv(g.z + r, pm.voxelSize), pm.voxelCount[2] - 1);
+    const int32_t x0 = max((int32_t)div1(a.cellDiv, g.x - r), 0);
+    const int32_t x1 = min((int32_t)div1(a.cellDiv, g.x + r), pm.voxelCount[0] - 1);
+    const int32_t y0 = max((int32_t)div1(a.cellDiv, g.y - r), 0);
+    const int32_t y1 = min((int32_t)div1(a.cellDiv, g.y + r), pm.voxelCount[1] - 1);
+    const int32_t z0 = max((int32_t)div1(a.cellDiv, g.z - r), 0);
+    const int32_t z1 = min((int32_t)div1(a.cellDiv, g.z + r), pm.voxelCount[2] - 1);
     const float r2 = r * r;
     for (int32_t z = z0; z <= z1; z++)
         for (int32_t y = y0; y <= y1; y++)
@@ -285,10 +284,10 @@ __device__ __forceinline__ f4 estimate(const cr::PpmEstimateArgs& a, int32_t x, 
     for (uint32_t k = 0; k < MARCH_CEILING && cur < maxDist; k++) {
         pos = sub(pos, mul(dir, step));
         cur = cur + step;
-        const float ext = fdiv(density<T, LAYOUT>(a.g, cp, pos) * cp.densityScaling, cp.baseScaling);
+        const float ext = div1(a.scaleDiv, density<T, LAYOUT>(a.g, a.box, pos) * cp.densityScaling);
         const float sc = albedo * ext;
         // direct sunlight through the shadow volume
-        const float tsun = trilinear<float, LAYOUT_DENSE>(sv, sv_norm(a.svp, pos));
+        const float tsun = trilinear<float, LAYOUT_DENSE, true>(sv, sv_norm(a.svMap, pos));
         const float dl = ((1.0f * a.params.lightIntensity) * pdf) * tsun;
         f4 direct = {dl, dl, dl, dl};
         // one sky direction, its transmittance by a Riemann sum to the cloud's edge
@@ -306,8 +305,8 @@ __device__ __forceinline__ f4 estimate(const cr::PpmEstimateArgs& a, int32_t x, 
         for (uint32_t j = 0; j < MARCH_CEILING && in_box(cp.bounds[0], cp.bounds[1], q); j += 2) {
             const f3 q1 = add(q, dq);
             const f3 q2 = add(q1, dq);
-            const float v1 = density<T, LAYOUT>(a.g, cp, q1);
-            const float v2 = density<T, LAYOUT>(a.g, cp, q2);
+            const float v1 = density<T, LAYOUT>(a.g, a.box, q1);
+            const float v2 = density<T, LAYOUT>(a.g, a.box, q2);
             accD = accD + v1;
             accL = accL + a.ambientStep;
             samples++;

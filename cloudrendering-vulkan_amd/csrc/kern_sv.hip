@@ -37,8 +37,7 @@ __global__ void __launch_bounds__(256) sv_kernel(cr::SVArgs a)
         p.y = P.bounds[0][1] + ((fx * P.right[1] + fy * P.up[1]) + fz * P.lightDirection[1]) * P.voxelSize;
         p.z = P.bounds[0][2] + ((fx * P.right[2] + fy * P.up[2]) + fz * P.lightDirection[2]) * P.voxelSize;
         if (in_box(a.cloud.bounds[0], a.cloud.bounds[1], p)) {
-            acc = acc + fdiv(trilinear<T, LAYOUT>(g, cloud_norm(a.cloud, p)) * a.cloud.densityScaling,
-                             a.cloud.baseScaling);
+            acc = acc + div1(a.scaleDiv, trilinear<T, LAYOUT, true>(g, cloud_norm(a.box, p)) * a.cloud.densityScaling);
         }
         accDist = accDist + hz;
         out[(size_t)z * plane] = crd_expf(fdiv((-accDist) * acc, (float)((uint32_t)z + 1u)));

@@ -101,19 +101,19 @@ struct Counters {
 __device__ __forceinline__ const float* B0(const cr::PTArgs& a) { return a.cloud.bounds[0]; }
 __device__ __forceinline__ const float* B1(const cr::PTArgs& a) { return a.cloud.bounds[1]; }
 
-template <typename T, int LAYOUT>
+template <typename T, int LAYOUT, bool PAIRS>
 __device__ __forceinline__ float sample_cloud(const cr::PTArgs& a, f3 p)
 {
     GridView g;
     g.data = a.grid; g.nx = a.nx; g.ny = a.ny; g.nz = a.nz; g.nbx = a.nbx; g.nby = a.nby;
-    return trilinear<T, LAYOUT>(g, cloud_norm(a.cloud, p));
+    return trilinear<T, LAYOUT, PAIRS>(g, cloud_norm(a.box, p));
 }
 
 __device__ __forceinline__ float sample_sv(const cr::PTArgs& a, f3 p)
 {
     GridView g;
     g.data = a.sv; g.nx = a.svx; g.ny = a.svy; g.nz = a.svz; g.nbx = 0; g.nby = 0;
-    return trilinear<float, LAYOUT_DENSE>(g, sv_norm(a.svp, p));
+    return trilinear<float, LAYOUT_DENSE, true>(g, sv_norm(a.svMap, p));
 }
 
 // Per lane and axis, for the lane's current segment (written once per segment
@@ -280,7 +280,7 @@ __device__ __forceinline__ uint32_t track_step(const cr::PTArgs& a, Lane& L, f3 
         // the division is made once here, not at each unrolled visit
         L.t = L.t + fdiv(L.tau, sbHit);
         f3 cur = add(L.pos, mul(dir, L.t));
-        float e = sample_cloud<T, LAYOUT>(a, cur);
+        float e = sample_cloud<T, LAYOUT, TRACK != CR_TRACK_BRICK_DDA>(a, cur);
         c.lookups++;
         // shadow and primary lanes of a wave share the division and the next
         // free-flight draw (one copy of each instead of one per branch)
@@ -300,12 +300,12 @@ __device__ __forceinline__ uint32_t track_step(const cr::PTArgs& a, Lane& L, f3 
         return ev;
     }
     float zeta = xs_float(L.rng);
-    L.t = L.t + fdiv(-crd_log_normal(zeta), a.sigmaBar);
+    L.t = L.t + div1(a.sigmaDiv, -crd_log_normal(zeta));
     if (!(L.t < L.dist)) return EV_EXIT;
     f3 cur = add(L.pos, mul(dir, L.t));
-    float e = sample_cloud<T, LAYOUT>(a, cur);
+    float e = sample_cloud<T, LAYOUT, TRACK != CR_TRACK_BRICK_DDA>(a, cur);
     c.lookups++;
-    const float q = fdiv(e, a.cloud.maxExtinction);
+    const float q = div1(a.extDiv, e);
     if (shadow) {
         L.T = L.T * (1.0f - q);
         if (L.T == 0.0f) return EV_EXIT;
@@ -629,7 +629,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
         if (state != ST_ACTIVE) continue;
 
         const cr::PTArgs& a = BATCH ? jobs[L.job] : a0;
-        const f3 ldir = ld3(a.svp.lightDirection);
+        const f3 ldir = ld3(a.lightDirection);
         const f3 sdir = neg(ldir);
         const float I = a.params.lightIntensity;
         const float albedo = a.ext.albedo;

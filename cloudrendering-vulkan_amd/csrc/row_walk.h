@@ -78,14 +78,14 @@ __device__ __forceinline__ unsigned long long row_slot(const RowLane& R, unsigne
 // segment) and rng the state after its last draw; otherwise t and rng are
 // those after 16 steps.  `density`: the cloud's density at a distance.
 template <class Density>
-__device__ __forceinline__ bool row_walk(const RowLane& R, float sigmaBar, float maxExtinction, float len, float& t,
+__device__ __forceinline__ bool row_walk(const RowLane& R, const Divisor& sigmaBar, const Divisor& maxExtinction, float len, float& t,
                                          uint32_t& rng, bool& hit, Density density)
 {
     uint32_t s = R.ahead(rng);
     const float zeta = xs_float(s);
     const uint32_t afterFlight = s;
     const float xi = xs_float(s);
-    const float d = fdiv(-crd_logf(zeta), sigmaBar);
+    const float d = div1(sigmaBar, -crd_logf(zeta));
     // t + d of the row's first lane, then lane by lane (row_shr:1)
     float at = t;
 #pragma unroll
@@ -93,7 +93,7 @@ __device__ __forceinline__ bool row_walk(const RowLane& R, float sigmaBar, float
         at = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(t), __float_as_int(at), 0x111, 0xf, 0xf, false)) + d;
     const bool left = !(at <= len);
     bool stop = left;
-    if (!left) stop = xi < fdiv(density(at), maxExtinction);
+    if (!left) stop = xi < div1(maxExtinction, density(at));
     const uint32_t row = (threadIdx.x & 63u) & ~(uint32_t)(ROW - 1);
     const uint32_t ends = (uint32_t)(__ballot(stop) >> row) & 0xffffu;
     const int last = ends ? (int)__ffs((int)ends) - 1 : ROW - 1;
