@@ -395,10 +395,11 @@ __device__ __forceinline__ float trilinear(const GridView& g, f3 n)
 
 // Division by a divisor the same for a whole launch, correctly rounded, without
 // the divide sequence (path tracer at 256x256 and 64 spp 2.69 -> 2.53 ms, 1080p
-// with bricks 63.6 -> 62.3, 1 GiB grid 321 -> 319): with y = 1/d correctly rounded, q0 = x y is within two
-// units of the quotient, one residual step q1 = q0 + (x - d q0) y makes it
-// faithful and the next one rounds it correctly (Markstein, IBM J. Res. Dev.
-// 34(1), 1990), while no intermediate value is subnormal or overflows.  A power
+// with bricks 63.6 -> 62.3, 1 GiB grid 321 -> 319): with y = 1/d correctly
+// rounded, q0 = x y is within two units of the quotient, one residual step
+// q1 = q0 + (x - d q0) y makes it faithful and the next one rounds it correctly
+// (Markstein, IBM J. Res. Dev. 34(1), 1990), while no intermediate value is
+// subnormal or overflows.  A power
 // of two divides exactly by the multiplication alone.  Other divisors (0, tiny,
 // huge, NaN) take the IEEE division.  The numerators are finite coordinate
 // differences of at most a few divisors; one below 2^-100 may come out an ulp

@@ -2,12 +2,13 @@
 // (shaders/PPM_PT.comp) and the ray-marched radiance estimate
 // (shaders/PPM_PE.comp) for gfx950.
 //
-// Tracing: one lane per photon path.  The paths leave their deposits as records; a scan of the paths' counts gives every path its
-// slots and a second kernel places the deposits there, in emission order (path
-// id, then collision) instead of the reference's atomic arrival order
-// (PPM_PT.comp:318).  A stable radix sort by cell then groups them, and a
-// cell keeps its first CR_PPM_PHOTONS_PER_CELL photons in that order: the map
-// is a pure function of the inputs, and the CPU oracle reproduces it.
+// Tracing: one lane per photon path.  The paths leave their deposits as records;
+// a scan of the paths' counts gives every path its slots and a second kernel
+// places the deposits there, in emission order (path id, then collision) instead
+// of the reference's atomic arrival order (PPM_PT.comp:318).  A stable radix sort
+// by cell then groups them, and a cell keeps its first CR_PPM_PHOTONS_PER_CELL
+// photons in that order: the map is a pure function of the inputs, and the CPU
+// oracle reproduces it.
 //
 // Estimate: one lane per pixel in 8x8-pixel workgroups, marching from the
 // far side of the cloud toward the camera (PPM_PE.comp:443-545).  Per step:
@@ -256,6 +257,18 @@ __device__ __forceinline__ f4 photon_query(const cr::PpmEstimateArgs& a, f3 p, f
     return acc;
 }
 
+// The kernel's arguments, read again from the argument segment: what a step
+// needs outside the sky ray's loop does not fit the scalar registers beside what
+// the loop holds (92 of them were spilled; 144 vector registers became 118, four
+// waves per SIMD instead of three).
+__device__ __forceinline__ const cr::PpmEstimateArgs& cold_args()
+{
+    typedef const __attribute__((address_space(4))) cr::PpmEstimateArgs* ConstArgs;
+    ConstArgs p = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const cr::PpmEstimateArgs*)p;
+}
+
 // PPM_PE.comp main (:443-545) for one pixel and one frame.
 template <typename T, int LAYOUT>
 __device__ __forceinline__ f4 estimate(const cr::PpmEstimateArgs& a, int32_t x, int32_t y, int32_t seed, float radius)
@@ -278,43 +291,36 @@ __device__ __forceinline__ f4 estimate(const cr::PpmEstimateArgs& a, int32_t x, 
     const float dsbs = fdiv(cp.densityScaling, cp.baseScaling);
     // the direct light's phase term: the same for every step of the ray
     const float pdf = phase_pdf(a.params, neg(dir), L);
-    GridView sv;
-    sv.data = a.sv; sv.nx = a.svx; sv.ny = a.svy; sv.nz = a.svz; sv.nbx = 0; sv.nby = 0;
     float cur = 0.0f;
     for (uint32_t k = 0; k < MARCH_CEILING && cur < maxDist; k++) {
+        const cr::PpmEstimateArgs& e = cold_args();
         pos = sub(pos, mul(dir, step));
         cur = cur + step;
-        const float ext = div1(a.scaleDiv, density<T, LAYOUT>(a.g, a.box, pos) * cp.densityScaling);
+        const float ext = div1(e.scaleDiv, density<T, LAYOUT>(a.g, a.box, pos) * e.cloud.densityScaling);
         const float sc = albedo * ext;
         // direct sunlight through the shadow volume
-        const float tsun = trilinear<float, LAYOUT_DENSE, true>(sv, sv_norm(a.svMap, pos));
-        const float dl = ((1.0f * a.params.lightIntensity) * pdf) * tsun;
+        GridView sv;
+        sv.data = e.sv; sv.nx = e.svx; sv.ny = e.svy; sv.nz = e.svz; sv.nbx = 0; sv.nby = 0;
+        const float tsun = trilinear<float, LAYOUT_DENSE, true>(sv, sv_norm(e.svMap, pos));
+        const float dl = ((1.0f * e.params.lightIntensity) * pdf) * tsun;
         f4 direct = {dl, dl, dl, dl};
         // one sky direction, its transmittance by a Riemann sum to the cloud's edge
-        const f3 ad = scatter(a.params, dir, rng);
+        const f3 ad = scatter(e.params, dir, rng);
         f3 q = pos;
         float accD = 0.0f, accL = 0.0f;
         uint32_t samples = 0;
-        f4 amb = background(a.ext, ad);
-        // Two samples per iteration, their lookups issued together: the second
-        // is taken only if the point before it is still inside the box, as
-        // the one-sample loop would (a sample outside the box reads clamped
-        // texels, so the speculative lookup stays in bounds).  Same points,
-        // same sums in the same order.
+        f4 amb = background(e.ext, ad);
         const f3 dq = mul(ad, a.ambientStep);
-        for (uint32_t j = 0; j < MARCH_CEILING && in_box(cp.bounds[0], cp.bounds[1], q); j += 2) {
-            const f3 q1 = add(q, dq);
-            const f3 q2 = add(q1, dq);
-            const float v1 = density<T, LAYOUT>(a.g, a.box, q1);
-            const float v2 = density<T, LAYOUT>(a.g, a.box, q2);
-            accD = accD + v1;
+        // One sample per iteration: lookups are bound by the cache lines they
+        // touch, and a second one taken on trust touches them for nothing at the
+        // end of a ray (whole frame at 1080p 15.2 ms; by twos 16.9, by fours 21.6;
+        // letting lanes go on to their next step alone, as their rays end, 18.9
+        // and more, as the rest of a step is dearer than the wait).
+        for (uint32_t j = 0; j < MARCH_CEILING && in_box(cp.bounds[0], cp.bounds[1], q); j++) {
+            q = add(q, dq);
+            accD = accD + density<T, LAYOUT>(a.g, a.box, q);
             accL = accL + a.ambientStep;
             samples++;
-            if (!(j + 1 < MARCH_CEILING && in_box(cp.bounds[0], cp.bounds[1], q1))) break;
-            accD = accD + v2;
-            accL = accL + a.ambientStep;
-            samples++;
-            q = q2;
         }
         accD = accD * dsbs;
         const float ta = crd_expf(fdiv(-accL * accD, (float)samples));
@@ -324,7 +330,7 @@ __device__ __forceinline__ f4 estimate(const cr::PpmEstimateArgs& a, int32_t x, 
             direct.z = direct.z + amb.z; direct.w = direct.w + amb.w;
         }
         // photons
-        const f4 ind0 = photon_query(a, pos, neg(dir), sc, radius);
+        const f4 ind0 = photon_query(cold_args(), pos, neg(dir), sc, radius);
         const f4 ind = {albedo * ind0.x, albedo * ind0.y, albedo * ind0.z, albedo * ind0.w};
         const float att = crd_expf(-step * ext);
         res.x = res.x * att + (sc * (direct.x + ind.x)) * step;
