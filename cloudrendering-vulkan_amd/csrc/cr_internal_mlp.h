@@ -20,9 +20,9 @@ inline uint64_t mlp_padded_rows(uint64_t B) { return (B + MLP_TILE - 1) / MLP_TI
 inline unsigned mlp_tiles(uint64_t B) { return (unsigned)((B + MLP_TILE - 1) / MLP_TILE); }
 
 // The training kernel keeps, for the weight-gradient GEMM, every layer's input
-// and every layer's output gradient feature-major ([feature][Bp] bf16, Bp the
-// padded row count): X^T (224 rows), H1..H4^T (128 each), dZ0..dZ3^T (128
-// each), dZ4^T (16).  Offsets in elements, in units of Bp.
+// and every layer's output gradient, per 32-row tile and feature-major in it
+// ([tile][feature][32] bf16): X^T (224 features), H1..H4^T (128 each),
+// dZ0..dZ3^T (128 each), dZ4^T (16).  Offsets in features.
 constexpr uint32_t MLP_TR_IN[MLP_LAYERS] = {0, 224, 352, 480, 608};
 constexpr uint32_t MLP_TR_DZ[MLP_LAYERS] = {736, 864, 992, 1120, 1248};
 constexpr uint32_t MLP_TR_ROWS = 1264;
@@ -49,13 +49,12 @@ struct MlpArgs {
     uint64_t dsN;
     uint32_t seed, step;
     int64_t B;
-    uint64_t Bp;             // padded row count (a multiple of 32)
     const uint32_t* Bdev;    // inference only: when set, the row count is *Bdev (<= B, B sizes the launch)
     uint16_t* WT[MLP_LAYERS];  // bf16 [N][K]
     uint16_t* W[MLP_LAYERS];   // bf16 [K][N]
     const float* bias[MLP_LAYERS];
     float* Y;                // inference: [B][4] fp32 outputs (log(1 + radiance), 3 used)
-    uint16_t* tr;            // training: feature-major inputs and output gradients (MLP_TR_ROWS x Bp)
+    uint16_t* tr;            // training: inputs and output gradients, [tile][MLP_TR_ROWS][32]
     float* loss;             // training: per-tile loss shares, added in order by the host
     float* grad;             // flat fp32 gradients (same layout as the parameters), written by the Adam kernel
     float* slot;             // [slots][total] gradient sums of the weight-gradient GEMM

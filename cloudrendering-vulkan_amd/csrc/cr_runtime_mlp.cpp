@@ -153,7 +153,6 @@ MlpArgs args_of(Mlp* m, const uint16_t* X, uint64_t B)
     memset(&a, 0, sizeof(a));
     a.X = X;
     a.B = (int64_t)B;
-    a.Bp = mlp_padded_rows(B);
     for (int l = 0; l < MLP_LAYERS; l++) {
         a.WT[l] = m->WT[l];
         a.W[l] = m->W[l];

@@ -14,14 +14,22 @@
 //    the activations in LDS (each of the four waves owns 32 output columns of
 //    every hidden layer), forms the loss share and dY, and runs the backward
 //    chain dA = dZ W^T, dZ_prev = dA * (H > 0).  It writes every layer's input
-//    and every layer's output gradient feature-major ([feature][row], bf16)
-//    for the weight-gradient GEMM, and no activations are re-read.
+//    and every layer's output gradient by tile and feature ([tile][feature][32
+//    rows], bf16) for the weight-gradient GEMM, whose loads are then 1 KB in one
+//    piece (whole columns of the batch, 16 KB apart, shared few memory channels:
+//    14.3 -> 11.8 us), and no activations are re-read.  One workgroup per CU and
+//    nine barriers: bound by latency.  Weights are fetched two layers ahead,
+//    biases and targets at the start (21.3 -> 18.8 us; with the weights fetched
+//    where they are used 21.9).  Measured and slower: eight waves of 16 columns,
+//    a loop over the equal layers, all loads at the start and all stores at the end.
 //  * mlp_wgrad_kernel: dW_l = H_l^T dZ_l and db_l = 1^T dZ_l as MFMA GEMMs
 //    reducing over the batch (32 x 32 output tiles; the batch split into a few
 //    contiguous ranges, one gradient slot each; the four waves of a
-//    workgroup add their partial tiles in wave order).
-//  * mlp_adam_kernel adds the slots in slot order, so a step is
-//    bit-reproducible, then Adam and the bf16 weight copies.
+//    workgroup add their partial tiles in wave order).  A slot's tiles follow
+//    each other 8 or 16 blocks apart, so with 8 or 16 slots an XCD reads an
+//    eighth of the copies, which its L2 holds (11.8 -> 8.8 us).
+//  * mlp_adam_kernel adds the slots in slot order (fetched together: 5.3 -> 4.5
+//    us), so a step is bit-reproducible, then Adam and the bf16 weight copies.
 // Inference (mlp_infer_kernel): persistent, one workgroup per CU holding the
 // whole network in LDS (159,744 B of bf16 weights + biases); each wave takes
 // 64 rows at a time and keeps their activations in registers between layers:
@@ -97,14 +105,37 @@ struct TrainLds {
     uint16_t dz[2][32 * HS];   // output gradients, ping-pong between backward layers
     uint64_t src[32];          // the tile's source rows
     float lossPart[2];
+    float target[96];
 };
+
+// A wave's share of one layer's weights, in registers: the B operands of output
+// columns [32 w, 32 w + 32) over a reduction of length K (rows of `w` have K
+// entries; K = 16 is the last layer's, zero-padded to one step).  A workgroup has
+// one wave per SIMD and every layer ends in a barrier, so weights fetched when
+// they are used cost each layer a trip to L2; they are fetched two layers ahead.
+template <int K>
+struct LayerW {
+    v8bf b[(K + 31) / 32][2];
+};
+template <int K>
+__device__ __forceinline__ LayerW<K> load_layer(const uint16_t* w)
+{
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, m = l & 15, g = l >> 4;
+    LayerW<K> r;
+#pragma unroll
+    for (int q = 0; q < (K + 31) / 32; q++)
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++)
+            r.b[q][ct] = (K == 16 && g >= 2) ? zero8() : ld16(w + (size_t)(wave * 32 + ct * 16 + m) * K + 32 * q + 8 * g);
+    return r;
+}
 
 // One hidden layer forward for the tile: wave w computes output columns
 // [32 w, 32 w + 32) of all 32 rows, H_out = max(H_in WT^T + b, 0), into LDS and
-// feature-major into `trOut` (the weight-gradient GEMM's copy).
+// into `trOut` (the weight-gradient GEMM's copy).
 template <int K, int IS>
-__device__ __forceinline__ void fwd_layer(const uint16_t* in, const uint16_t* WT, const float* bias, uint16_t* out,
-                                          uint16_t* trOut, uint64_t Bp, int64_t row0)
+__device__ __forceinline__ void fwd_layer(const uint16_t* in, const LayerW<K>& WT, const float (&bias)[2], uint16_t* out,
+                                          uint16_t* trOut)
 {
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, m = l & 15, g = l >> 4;
     const int n0 = wave * 32;
@@ -115,8 +146,7 @@ __device__ __forceinline__ void fwd_layer(const uint16_t* in, const uint16_t* WT
         for (int ct = 0; ct < 2; ct++) acc[rt][ct] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int q = 0; q < K / 32; q++) {
-        const v8bf b0 = ld16(WT + (size_t)(n0 + m) * K + 32 * q + 8 * g);
-        const v8bf b1 = ld16(WT + (size_t)(n0 + 16 + m) * K + 32 * q + 8 * g);
+        const v8bf b0 = WT.b[q][0], b1 = WT.b[q][1];
         const v8bf a0 = ld16(in + m * IS + 32 * q + 8 * g);
         const v8bf a1 = ld16(in + (16 + m) * IS + 32 * q + 8 * g);
         acc[0][0] = mfma(a0, b0, acc[0][0]);
@@ -127,7 +157,7 @@ __device__ __forceinline__ void fwd_layer(const uint16_t* in, const uint16_t* WT
 #pragma unroll
     for (int ct = 0; ct < 2; ct++) {
         const int n = n0 + ct * 16 + m;
-        const float bn = bias[n];
+        const float bn = bias[ct];
 #pragma unroll
         for (int rt = 0; rt < 2; rt++) {
             const v4f z = acc[rt][ct];
@@ -137,7 +167,7 @@ __device__ __forceinline__ void fwd_layer(const uint16_t* in, const uint16_t* WT
             o[HS] = (uint16_t)(h.x >> 16);
             o[2 * HS] = (uint16_t)h.y;
             o[3 * HS] = (uint16_t)(h.y >> 16);
-            *reinterpret_cast<uint2*>(trOut + (size_t)n * Bp + row0 + rt * 16 + 4 * g) = h;
+            *reinterpret_cast<uint2*>(trOut + n * 32 + rt * 16 + 4 * g) = h;
         }
     }
 }
@@ -147,8 +177,8 @@ __device__ __forceinline__ void fwd_layer(const uint16_t* in, const uint16_t* WT
 // input's gradient dZ_prev = dA * (H > 0).  Wave w owns input columns
 // [32 w, 32 w + 32).
 template <int N>
-__device__ __forceinline__ void bwd_layer(const uint16_t* dzIn, const uint16_t* W, const uint16_t* h, uint16_t* dzOut,
-                                          uint16_t* trOut, uint64_t Bp, int64_t row0)
+__device__ __forceinline__ void bwd_layer(const uint16_t* dzIn, const LayerW<N>& W, const uint16_t* h, uint16_t* dzOut,
+                                          uint16_t* trOut)
 {
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, m = l & 15, g = l >> 4;
     const int c0 = wave * 32;
@@ -159,10 +189,7 @@ __device__ __forceinline__ void bwd_layer(const uint16_t* dzIn, const uint16_t* 
         for (int ct = 0; ct < 2; ct++) acc[rt][ct] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int q = 0; q < (N + 31) / 32; q++) {
-        v8bf b[2];
-#pragma unroll
-        for (int ct = 0; ct < 2; ct++)
-            b[ct] = (N == 16 && g >= 2) ? zero8() : ld16(W + (size_t)(c0 + ct * 16 + m) * N + 32 * q + 8 * g);
+        const v8bf* b = W.b[q];
         const v8bf a0 = ld16(dzIn + m * HS + 32 * q + 8 * g);
         const v8bf a1 = ld16(dzIn + (16 + m) * HS + 32 * q + 8 * g);
         acc[0][0] = mfma(a0, b[0], acc[0][0]);
@@ -189,7 +216,7 @@ __device__ __forceinline__ void bwd_layer(const uint16_t* dzIn, const uint16_t* 
                 o[2 * HS] = (uint16_t)d.y;
                 o[3 * HS] = (uint16_t)(d.y >> 16);
             }
-            *reinterpret_cast<uint2*>(trOut + (size_t)c * Bp + row0 + rt * 16 + 4 * g) = d;
+            *reinterpret_cast<uint2*>(trOut + c * 32 + rt * 16 + 4 * g) = d;
         }
     }
 }
@@ -203,12 +230,21 @@ __global__ void __launch_bounds__(256) mlp_train_kernel(cr::MlpArgs a)
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, m = l & 15, g = l >> 4;
     const int64_t row0 = (int64_t)blockIdx.x * 32;
     const int64_t B = a.B;
-    const uint64_t Bp = a.Bp;
-    uint16_t* tr = a.tr;
+    uint16_t* const tr = a.tr + (size_t)blockIdx.x * cr::MLP_TR_ROWS * 32;
     if (tid < 32)
         S.src[tid] = a.dsX ? cr::mlp_draw(a.seed, a.step, (uint32_t)(row0 + tid), a.dsN) : (uint64_t)(row0 + tid);
     __syncthreads();
     const uint16_t* Xs = a.dsX ? a.dsX : a.X;
+    const LayerW<224> w0 = load_layer<224>(a.WT[0]);
+    const LayerW<128> w1 = load_layer<128>(a.WT[1]);
+    float bias[4][2];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) bias[k][ct] = a.bias[k][wave * 32 + ct * 16 + m];
+    const float bias4 = a.bias[4][m];
+    float tgt = 0.0f;
+    if (tid < 96 && row0 + tid / 3 < B) tgt = a.dsX ? a.dsT[S.src[tid / 3] * 3 + tid % 3] : a.T[row0 * 3 + tid];
     for (int idx = tid; idx < 32 * 28; idx += 256) {
         const int r = idx / 28, c = idx % 28;
         uint4 v = make_uint4(0u, 0u, 0u, 0u);
@@ -216,31 +252,40 @@ __global__ void __launch_bounds__(256) mlp_train_kernel(cr::MlpArgs a)
         *reinterpret_cast<uint4*>(S.x + r * XS + c * 8) = v;
     }
     __syncthreads();
+    if (tid < 96) S.target[tid] = log1pf(fmaxf(tgt, 0.0f));
     // X^T: (feature, 8 rows) per item
     for (int idx = tid; idx < 224 * 4; idx += 256) {
         const int k = idx >> 2, r8 = (idx & 3) * 8;
         uint16_t h[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) h[j] = S.x[(r8 + j) * XS + k];
-        *reinterpret_cast<uint4*>(tr + (size_t)(cr::MLP_TR_IN[0] + k) * Bp + row0 + r8) =
+        *reinterpret_cast<uint4*>(tr + (cr::MLP_TR_IN[0] + k) * 32 + r8) =
             make_uint4(pk(h[0], h[1]), pk(h[2], h[3]), pk(h[4], h[5]), pk(h[6], h[7]));
     }
-    fwd_layer<224, XS>(S.x, a.WT[0], a.bias[0], S.h[0], tr + (size_t)cr::MLP_TR_IN[1] * Bp, Bp, row0);
+    const LayerW<128> w2 = load_layer<128>(a.WT[2]);
+    fwd_layer<224, XS>(S.x, w0, bias[0], S.h[0], tr + cr::MLP_TR_IN[1] * 32);
     __syncthreads();
-    fwd_layer<128, HS>(S.h[0], a.WT[1], a.bias[1], S.h[1], tr + (size_t)cr::MLP_TR_IN[2] * Bp, Bp, row0);
+    const LayerW<128> w3 = load_layer<128>(a.WT[3]);
+    fwd_layer<128, HS>(S.h[0], w1, bias[1], S.h[1], tr + cr::MLP_TR_IN[2] * 32);
     __syncthreads();
-    fwd_layer<128, HS>(S.h[1], a.WT[2], a.bias[2], S.h[2], tr + (size_t)cr::MLP_TR_IN[3] * Bp, Bp, row0);
+    v8bf w4[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) w4[q] = ld16(a.WT[4] + m * 128 + 32 * q + 8 * g);
+    const LayerW<16> v4 = load_layer<16>(a.W[4]);
+    fwd_layer<128, HS>(S.h[1], w2, bias[2], S.h[2], tr + cr::MLP_TR_IN[3] * 32);
     __syncthreads();
-    fwd_layer<128, HS>(S.h[2], a.WT[3], a.bias[3], S.h[3], tr + (size_t)cr::MLP_TR_IN[4] * Bp, Bp, row0);
+    const LayerW<128> v3 = load_layer<128>(a.W[3]);
+    fwd_layer<128, HS>(S.h[2], w3, bias[3], S.h[3], tr + cr::MLP_TR_IN[4] * 32);
     __syncthreads();
+    const LayerW<128> v2 = load_layer<128>(a.W[2]);
     // output layer, loss and dY: waves 0 and 1, one 16-row tile each
     if (wave < 2) {
         const int rt = wave;
         v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int q = 0; q < 4; q++)
-            acc = mfma(ld16(S.h[3] + (rt * 16 + m) * HS + 32 * q + 8 * g), ld16(a.WT[4] + m * 128 + 32 * q + 8 * g), acc);
-        const float bn = a.bias[4][m];
+            acc = mfma(ld16(S.h[3] + (rt * 16 + m) * HS + 32 * q + 8 * g), w4[q], acc);
+        const float bn = bias4;
         const float scale = 2.0f / ((float)B * 3.0f);
         float lsum = 0.0f;
         float dy[4];
@@ -250,8 +295,7 @@ __global__ void __launch_bounds__(256) mlp_train_kernel(cr::MlpArgs a)
             const int64_t row = row0 + r;
             dy[j] = 0.0f;
             if (m < 3 && row < B) {
-                const float t = a.dsX ? a.dsT[S.src[r] * 3 + m] : a.T[row * 3 + m];
-                const float diff = (acc[j] + bn) - log1pf(fmaxf(t, 0.0f));
+                const float diff = (acc[j] + bn) - S.target[r * 3 + m];
                 dy[j] = scale * diff;
                 lsum += diff * diff;
             }
@@ -264,19 +308,20 @@ __global__ void __launch_bounds__(256) mlp_train_kernel(cr::MlpArgs a)
             S.dz[0][r * HS + m] = dh[j];
             S.dz[0][r * HS + 16 + m] = 0;  // the padded half of the 32-wide reduction step
         }
-        *reinterpret_cast<uint2*>(tr + (size_t)(cr::MLP_TR_DZ[4] + m) * Bp + row0 + rt * 16 + 4 * g) = d;
+        *reinterpret_cast<uint2*>(tr + (cr::MLP_TR_DZ[4] + m) * 32 + rt * 16 + 4 * g) = d;
         for (int off = 32; off >= 1; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
         if (l == 0) S.lossPart[wave] = lsum;
     }
     __syncthreads();
     if (tid == 0) a.loss[blockIdx.x] = (S.lossPart[0] + S.lossPart[1]) / ((float)B * 3.0f);
-    bwd_layer<16>(S.dz[0], a.W[4], S.h[3], S.dz[1], tr + (size_t)cr::MLP_TR_DZ[3] * Bp, Bp, row0);
+    const LayerW<128> v1 = load_layer<128>(a.W[1]);
+    bwd_layer<16>(S.dz[0], v4, S.h[3], S.dz[1], tr + cr::MLP_TR_DZ[3] * 32);
     __syncthreads();
-    bwd_layer<128>(S.dz[1], a.W[3], S.h[2], S.dz[0], tr + (size_t)cr::MLP_TR_DZ[2] * Bp, Bp, row0);
+    bwd_layer<128>(S.dz[1], v3, S.h[2], S.dz[0], tr + cr::MLP_TR_DZ[2] * 32);
     __syncthreads();
-    bwd_layer<128>(S.dz[0], a.W[2], S.h[1], S.dz[1], tr + (size_t)cr::MLP_TR_DZ[1] * Bp, Bp, row0);
+    bwd_layer<128>(S.dz[0], v2, S.h[1], S.dz[1], tr + cr::MLP_TR_DZ[1] * 32);
     __syncthreads();
-    bwd_layer<128>(S.dz[1], a.W[1], S.h[0], nullptr, tr + (size_t)cr::MLP_TR_DZ[0] * Bp, Bp, row0);
+    bwd_layer<128>(S.dz[1], v1, S.h[0], nullptr, tr + cr::MLP_TR_DZ[0] * 32);
 }
 
 // One output tile of dW_l = H_l^T dZ_l (32 input features x NT * 16 outputs)
@@ -287,10 +332,10 @@ __device__ __forceinline__ void wgrad_tile(const cr::MlpArgs& a, int layer, int 
     __shared__ float red[3][2][2][4][64];
     __shared__ float redb[3][2][64];
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, m = l & 15, g = l >> 4;
-    const uint64_t Bp = a.Bp;
-    const uint16_t* A = a.tr + (size_t)(cr::MLP_TR_IN[layer] + kt * 32) * Bp;
-    const uint16_t* D = a.tr + (size_t)(cr::MLP_TR_DZ[layer] + nt * 32) * Bp;
-    const uint64_t C = Bp / 32;
+    const uint16_t* A = a.tr + (cr::MLP_TR_IN[layer] + kt * 32 + m) * 32 + 8 * g;
+    const uint16_t* D = a.tr + (cr::MLP_TR_DZ[layer] + nt * 32 + m) * 32 + 8 * g;
+    constexpr uint64_t CHUNK = cr::MLP_TR_ROWS * 32;
+    const uint64_t C = ((uint64_t)a.B + 31) / 32;
     const uint64_t c0 = s * C / a.slots, c1 = (s + 1) * C / a.slots;
     const v8bf ones = as_bf(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
     v4f acc[2][2], accb[2];
@@ -301,15 +346,16 @@ __device__ __forceinline__ void wgrad_tile(const cr::MlpArgs& a, int layer, int 
         for (int mt = 0; mt < 2; mt++) acc[mt][ct] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
     for (uint64_t c = c0 + wave; c < c1; c += 4) {
-        const uint64_t b0 = c * 32 + 8 * g;
-        const v8bf a0 = ld16(A + (size_t)m * Bp + b0);
-        const v8bf a1 = ld16(A + (size_t)(16 + m) * Bp + b0);
+        const uint64_t at = c * CHUNK;
+        const v8bf a0 = ld16(A + at), a1 = ld16(A + at + 16 * 32);
+        v8bf b[NT];
+#pragma unroll
+        for (int ct = 0; ct < NT; ct++) b[ct] = ld16(D + at + ct * 16 * 32);
 #pragma unroll
         for (int ct = 0; ct < NT; ct++) {
-            const v8bf bb = ld16(D + (size_t)(ct * 16 + m) * Bp + b0);
-            acc[0][ct] = mfma(a0, bb, acc[0][ct]);
-            acc[1][ct] = mfma(a1, bb, acc[1][ct]);
-            if (kt == 0) accb[ct] = mfma(ones, bb, accb[ct]);
+            acc[0][ct] = mfma(a0, b[ct], acc[0][ct]);
+            acc[1][ct] = mfma(a1, b[ct], acc[1][ct]);
+            if (kt == 0) accb[ct] = mfma(ones, b[ct], accb[ct]);
         }
     }
     // add the waves' tiles in wave order
@@ -344,10 +390,10 @@ __device__ __forceinline__ void wgrad_tile(const cr::MlpArgs& a, int layer, int 
     }
 }
 
-// Grid: MLP_GRAD_TILES x slots workgroups; tile t of slot s is block s * tiles + t.
+// Grid: MLP_GRAD_TILES x slots workgroups; tile t of slot s is block t * slots + s.
 __global__ void __launch_bounds__(256) mlp_wgrad_kernel(cr::MlpArgs a)
 {
-    const uint32_t t = blockIdx.x % cr::MLP_GRAD_TILES, s = blockIdx.x / cr::MLP_GRAD_TILES;
+    const uint32_t s = blockIdx.x % a.slots, t = blockIdx.x / a.slots;
     if (t < 28) {
         wgrad_tile<2>(a, 0, (int)(t / 4), (int)(t % 4), s);
     } else if (t < 76) {
@@ -367,13 +413,15 @@ __global__ void __launch_bounds__(256) mlp_adam_kernel(cr::MlpArgs a, cr::AdamAr
     if (i >= o.n) return;
     float g = 0.0f;
     const float* part = a.slot + i;
+    const float m0 = o.m[i], v0 = o.v[i], p0 = o.params[i];
+#pragma unroll 8
     for (uint32_t s = 0; s < a.slots; s++) g += part[(size_t)s * a.total];
     a.grad[i] = g;
-    const float m = o.beta1 * o.m[i] + (1.0f - o.beta1) * g;
-    const float v = o.beta2 * o.v[i] + (1.0f - o.beta2) * g * g;
+    const float m = o.beta1 * m0 + (1.0f - o.beta1) * g;
+    const float v = o.beta2 * v0 + (1.0f - o.beta2) * g * g;
     o.m[i] = m;
     o.v[i] = v;
-    const float p = o.params[i] - o.lr * fdiv(fdiv(m, o.c1), fsqrt(fdiv(v, o.c2)) + o.eps);
+    const float p = p0 - o.lr * fdiv(fdiv(m, o.c1), fsqrt(fdiv(v, o.c2)) + o.eps);
     o.params[i] = p;
     // moving average of the parameters, bias-corrected for inference
     float eh = 0.0f;
