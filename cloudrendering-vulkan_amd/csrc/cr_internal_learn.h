@@ -59,7 +59,7 @@ hipError_t launch_features(const FeatureArgs& a, hipStream_t s);
 hipError_t launch_compose(const ComposeArgs& a, hipStream_t s);
 hipError_t launch_count(const float* rec, uint64_t n, uint32_t* counts, hipStream_t s);
 hipError_t launch_compact(const float* rec, uint64_t n, const uint32_t* offsets, float* pts, uint32_t* slot, hipStream_t s);
-hipError_t launch_scan_counts(uint32_t* counts, uint32_t nb, uint32_t* total, hipStream_t s);
+hipError_t launch_compact_any(const float* rec, uint64_t n, uint32_t* total, float* pts, uint32_t* slot, hipStream_t s);
 hipError_t launch_select(const float* src, uint32_t stride, uint32_t count, float* dst, hipStream_t s);
 // Append rows k * stride of X / T4 (and of the records pts) to the data set;
 // the targets leave out nee's term of each record.

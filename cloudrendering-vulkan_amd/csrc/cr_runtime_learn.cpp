@@ -285,19 +285,16 @@ cr_status compact(cr_context* ctx, Learn* L, uint64_t n, uint32_t* m_out)
     return CR_OK;
 }
 
-// The same compaction with the scan on the device: no host round trip; the
-// count stays in L->mdev and L->points / L->slot are sized for all n records.
+// The same in one pass and in any order: no host round trip; the count stays in
+// L->mdev and L->points / L->slot are sized for all n records.
 cr_status compact_device(cr_context* ctx, Learn* L, uint64_t n)
 {
-    const uint64_t nb = (n + 255) / 256;
-    if (nb > 0xFFFFFFFFull) return fail(ctx, CR_ERR_CAPACITY, "too many records in one pass");
-    CR_TRY(ensure_buffer(ctx, (void**)&L->counts, &L->countsCap, nb * 4, "counts"));
+    if ((n + 255) / 256 > 0xFFFFFFFFull) return fail(ctx, CR_ERR_CAPACITY, "too many records in one pass");
     CR_TRY(ensure_buffer(ctx, (void**)&L->slot, &L->slotCap, n * 4, "slots"));
     CR_TRY(ensure_buffer(ctx, (void**)&L->mdev, &L->mdevCap, 4, "collision count"));
     CR_TRY(ensure_buffer(ctx, (void**)&L->points, &L->pointsCap, n * 32, "points"));
-    CR_HIP(ctx, launch_count(L->records, n, L->counts, ctx->stream), "count collisions");
-    CR_HIP(ctx, launch_scan_counts(L->counts, (uint32_t)nb, L->mdev, ctx->stream), "scan counts");
-    CR_HIP(ctx, launch_compact(L->records, n, L->counts, L->points, L->slot, ctx->stream), "compact collisions");
+    CR_HIP(ctx, zero_async(L->mdev, 4, ctx->stream), "zero count");
+    CR_HIP(ctx, launch_compact_any(L->records, n, L->mdev, L->points, L->slot, ctx->stream), "compact collisions");
     return CR_OK;
 }
 

@@ -269,31 +269,64 @@ __global__ void __launch_bounds__(256) compact_kernel(const float* rec, uint64_t
     dst[1] = src[1];
 }
 
-// Exclusive scan of nb block counts in place, in one workgroup of 1024
-// threads (each scans a contiguous run); *total = the sum.
-__global__ void __launch_bounds__(1024) scan_counts_kernel(uint32_t* counts, uint32_t nb, uint32_t* total)
+// The compaction of a learned render, whose rows may come in any order (the
+// network treats each by itself): one pass, each workgroup taking the slots of
+// its 4096 records from *total (zeroed before) with one atomic.  Bound by memory:
+// the records are read once and the collided ones written (1080p at 32 spp, 66 M
+// records: 513 us; counts, a scan of them and a second pass took 1360).
+__global__ void __launch_bounds__(1024) compact_any_kernel(const float* rec, uint64_t n, uint32_t* total, float* pts,
+                                                           uint32_t* slot)
 {
-    __shared__ uint32_t part[1024];
-    const uint32_t t = threadIdx.x;
-    const uint32_t per = (nb + 1023u) / 1024u;
-    const uint32_t b0 = min(nb, t * per), b1 = min(nb, b0 + per);
-    uint32_t s = 0;
-    for (uint32_t i = b0; i < b1; i++) s += counts[i];
-    part[t] = s;
+    constexpr int R = 4;
+    __shared__ uint32_t count[16 * R];
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint64_t i0 = (uint64_t)blockIdx.x * (1024 * R) + threadIdx.x;
+    float4 v[R][2];
+    unsigned long long bal[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint64_t i = i0 + 1024u * r;
+        const float4* src = reinterpret_cast<const float4*>(rec) + 2 * i;
+        v[r][0] = v[r][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (i < n) {
+            v[r][0] = src[0];
+            v[r][1] = src[1];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        bal[r] = __ballot(v[r][1].w > 0.5f);
+        if (lane == 0) count[16 * r + w] = (uint32_t)__popcll(bal[r]);
+    }
     __syncthreads();
-    for (uint32_t off = 1; off < 1024u; off <<= 1) {
-        const uint32_t v = t >= off ? part[t - off] : 0u;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
+    if (threadIdx.x < 64u) {
+        const uint32_t c = count[lane];
+        uint32_t incl = c;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)incl, off, 64);
+            if (lane >= (uint32_t)off) incl += o;
+        }
+        uint32_t base = 0;
+        if (lane == 63u) base = atomicAdd(total, incl);
+        base = (uint32_t)__shfl((int)base, 63, 64);
+        count[lane] = base + incl - c;
     }
-    uint32_t run = part[t] - s;  // exclusive prefix of this thread's run
-    for (uint32_t i = b0; i < b1; i++) {
-        const uint32_t c = counts[i];
-        counts[i] = run;
-        run += c;
+    __syncthreads();
+    const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint64_t i = i0 + 1024u * r;
+        if (i >= n) continue;
+        uint32_t s = 0xFFFFFFFFu;
+        if (bal[r] >> lane & 1ull) {
+            s = count[16 * r + w] + (uint32_t)__popcll(bal[r] & lt);
+            float4* dst = reinterpret_cast<float4*>(pts) + 2 * (size_t)s;
+            dst[0] = v[r][0];
+            dst[1] = v[r][1];
+        }
+        slot[i] = s;
     }
-    if (t == 1023u) *total = part[1023];
 }
 
 // Rows k*stride (k < count) of 8-float records copied to dst[k].
@@ -348,9 +381,10 @@ hipError_t launch_compact(const float* rec, uint64_t n, const uint32_t* offsets,
     return hipGetLastError();
 }
 
-hipError_t launch_scan_counts(uint32_t* counts, uint32_t nb, uint32_t* total, hipStream_t s)
+hipError_t launch_compact_any(const float* rec, uint64_t n, uint32_t* total, float* pts, uint32_t* slot, hipStream_t s)
 {
-    hipLaunchKernelGGL(scan_counts_kernel, dim3(1), dim3(1024), 0, s, counts, nb, total);
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(compact_any_kernel, dim3((unsigned)((n + 4095) / 4096)), dim3(1024), 0, s, rec, n, total, pts, slot);
     return hipGetLastError();
 }
 
