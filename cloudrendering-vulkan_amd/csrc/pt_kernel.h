@@ -101,12 +101,13 @@ struct Counters {
 __device__ __forceinline__ const float* B0(const cr::PTArgs& a) { return a.cloud.bounds[0]; }
 __device__ __forceinline__ const float* B1(const cr::PTArgs& a) { return a.cloud.bounds[1]; }
 
-template <typename T, int LAYOUT, bool PAIRS>
+template <typename T, int LAYOUT, bool PAIRS, bool WHOLE>
 __device__ __forceinline__ float sample_cloud(const cr::PTArgs& a, f3 p)
 {
     GridView g;
     g.data = a.grid; g.nx = a.nx; g.ny = a.ny; g.nz = a.nz; g.nbx = a.nbx; g.nby = a.nby;
-    return trilinear<T, LAYOUT, PAIRS>(g, cloud_norm(a.box, p));
+    if (WHOLE) return trilinear<T, LAYOUT>(g, cloud_norm(a.cloud, p));
+    return trilinear<T, LAYOUT, PAIRS && sizeof(T) == 4>(g, cloud_norm(a.box, p));
 }
 
 __device__ __forceinline__ float sample_sv(const cr::PTArgs& a, f3 p)
@@ -222,7 +223,10 @@ enum : uint32_t { EV_NONE = 0, EV_COLLIDE = 1, EV_EXIT = 2 };
 
 // One tracking step: at most one density lookup.  Primary mode: delta
 // tracking (PathTracer.comp:335-355); shadow mode: ratio tracking.
-template <typename T, int LAYOUT, int TRACK>
+// WHOLE: passes of whole pixels of many frames are bound by the latency of one
+// path's chain, where the divide sequence and eight loads end sooner than uniform
+// branches and selects (68x68 pixels at 53 spp 14.6 ms, 16.1 with the others).
+template <typename T, int LAYOUT, int TRACK, bool WHOLE>
 __device__ __forceinline__ uint32_t track_step(const cr::PTArgs& a, Lane& L, f3 sdir, Counters& c)
 {
     const bool shadow = L.mode == MODE_SHADOW;
@@ -280,7 +284,7 @@ __device__ __forceinline__ uint32_t track_step(const cr::PTArgs& a, Lane& L, f3 
         // the division is made once here, not at each unrolled visit
         L.t = L.t + fdiv(L.tau, sbHit);
         f3 cur = add(L.pos, mul(dir, L.t));
-        float e = sample_cloud<T, LAYOUT, TRACK != CR_TRACK_BRICK_DDA>(a, cur);
+        float e = sample_cloud<T, LAYOUT, TRACK != CR_TRACK_BRICK_DDA, WHOLE>(a, cur);
         c.lookups++;
         // shadow and primary lanes of a wave share the division and the next
         // free-flight draw (one copy of each instead of one per branch)
@@ -300,12 +304,12 @@ __device__ __forceinline__ uint32_t track_step(const cr::PTArgs& a, Lane& L, f3 
         return ev;
     }
     float zeta = xs_float(L.rng);
-    L.t = L.t + div1(a.sigmaDiv, -crd_log_normal(zeta));
+    L.t = L.t + (WHOLE ? fdiv(-crd_log_normal(zeta), a.sigmaDiv.d) : div1(a.sigmaDiv, -crd_log_normal(zeta)));
     if (!(L.t < L.dist)) return EV_EXIT;
     f3 cur = add(L.pos, mul(dir, L.t));
-    float e = sample_cloud<T, LAYOUT, TRACK != CR_TRACK_BRICK_DDA>(a, cur);
+    float e = sample_cloud<T, LAYOUT, TRACK != CR_TRACK_BRICK_DDA, WHOLE>(a, cur);
     c.lookups++;
-    const float q = div1(a.extDiv, e);
+    const float q = WHOLE ? fdiv(e, a.cloud.maxExtinction) : div1(a.extDiv, e);
     if (shadow) {
         L.T = L.T * (1.0f - q);
         if (L.T == 0.0f) return EV_EXIT;
@@ -453,6 +457,13 @@ __device__ __forceinline__ const cr::PTArgs& cold_args()
     return *(const cr::PTArgs*)p;
 }
 
+// The same where a pass rereads rarely used arguments; whole-pixel passes keep them.
+template <int KMODE>
+__device__ __forceinline__ const cr::PTArgs& rare_args(const cr::PTArgs& a0)
+{
+    return KMODE == 0 ? a0 : cold_args();
+}
+
 // Last job whose first work index is <= idx (jobs are stored by increasing base).
 __device__ __forceinline__ uint32_t find_job(const cr::PTArgs* jobs, uint32_t n, uint32_t idx)
 {
@@ -497,7 +508,7 @@ __device__ __forceinline__ uint32_t part_first(uint32_t part, uint32_t logParts)
 template <typename T, int TRACK, bool BATCH, int KMODE>
 constexpr int min_waves()
 {
-    return sizeof(T) == 4 && TRACK == CR_TRACK_BRICK_DDA && !BATCH && renders(KMODE) ? 5 : 1;
+    return sizeof(T) == 4 && TRACK == CR_TRACK_BRICK_DDA && !BATCH && KMODE == K_RENDER_FEW ? 5 : 1;
 }
 
 // BATCH = false: one job, `a0`.  BATCH = true: the jobs of `b`, one shared
@@ -584,7 +595,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
                     L.mode = 0xFFu;
                 } else {
                     const uint32_t j = BATCH ? find_job(jobs, b.nJobs, idx) : 0u;
-                    const cr::PTArgs& J = BATCH ? jobs[j] : cold_args();
+                    const cr::PTArgs& J = BATCH ? jobs[j] : rare_args<KMODE>(a0);
                     const uint32_t local = BATCH ? idx - J.base : idx;
                     const uint32_t within = local & 63u;
                     uint32_t slot = local >> 6, ch = 0;
@@ -635,7 +646,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
         const float albedo = a.ext.albedo;
         const uint32_t cap = a.ext.bounceCap;
 
-        if (ev == EV_NONE && L.mode != 0xFFu) ev = track_step<T, LAYOUT, TRACK>(a, L, sdir, c);
+        if (ev == EV_NONE && L.mode != 0xFFu) ev = track_step<T, LAYOUT, TRACK, KMODE == K_RENDER && !BATCH>(a, L, sdir, c);
 
         // ---- divergent tail: events that need no lookup are resolved here,
         // possibly several in a row (e.g. a camera ray that misses the box).
@@ -659,7 +670,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
             bool cam = false;  // batched: a camera ray, its box test after the shared reciprocal below
             if (needSample) {
                 needSample = false;
-                const cr::PTArgs& k = BATCH ? a : cold_args();
+                const cr::PTArgs& k = BATCH ? a : rare_args<KMODE>(a0);
                 if (L.f >= (chunked(KMODE, BATCH) ? L.fEnd : k.nFrames)) {
                     if (chunked(KMODE, BATCH) && KMODE != K_RECORD && k.samples) {
                         // the samples are stored; the blend (or sum) kernel takes them in order
@@ -742,7 +753,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
             } else {  // EV_COLLIDE
                 if (KMODE == K_RECORD && L.bounces == 0) {
                     // first real collision: record it and end the frame here
-                    float4* r = reinterpret_cast<float4*>(record_of(BATCH ? a : cold_args(), L));
+                    float4* r = reinterpret_cast<float4*>(record_of(BATCH ? a : rare_args<KMODE>(a0), L));
                     r[0] = make_float4(L.pos.x, L.pos.y, L.pos.z, L.dir.x);
                     r[1] = make_float4(L.dir.y, L.dir.z, __uint_as_float(L.rng), 1.0f);
                     L.f++;
@@ -799,7 +810,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
                 }
             }
             if (sky) {
-                const f4 bg = background((BATCH ? a : cold_args()).ext, L.dir);
+                const f4 bg = background((BATCH ? a : rare_args<KMODE>(a0)).ext, L.dir);
                 if (missed) {
                     L.res = bg;
                 } else {
@@ -808,7 +819,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
                 fin = true;
             }
             if (fin) {
-                finish_sample<KMODE, BATCH>(BATCH ? a : cold_args(), L);
+                finish_sample<KMODE, BATCH>(BATCH ? a : rare_args<KMODE>(a0), L);
                 L.f++;
                 ev = EV_NONE;
                 needSample = true;
