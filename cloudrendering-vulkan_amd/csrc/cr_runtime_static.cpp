@@ -2,16 +2,16 @@
 //
 // cr_pt_render keeps its scratch in context buffers that it grows on demand:
 // the work-queue counter, the per-frame (seed, frameCount) table, the tile
-// list and the samples.  This variant keeps the first two in one fixed device
-// array per GPU, resolved once per device when a context is created, and renders
-// whole pixels into an image the caller owns; tiles are claimed in raster order,
-// which changes the schedule only (every pixel's arithmetic is cr_pt_render's).
-// It calls no hipMalloc, hipFree or allocating library routine.
+// list and the samples.  This variant keeps the frame table in one fixed device
+// array per GPU, resolved once per device when a context is created, uses the
+// work-queue counter the context was created with, and renders whole pixels into
+// an image the caller owns; tiles are claimed in raster order, which changes the
+// schedule only (every pixel's arithmetic is cr_pt_render's).  It calls no
+// hipMalloc, hipFree or allocating library routine.
 //
 // The array is shared by every context on a GPU and keeps the last call's
-// contents: the queue is cleared by a fill kernel at the start of each call, the
-// frame table is overwritten.  Calls that overlap on one GPU (two host threads,
-// or two contexts whose streams run concurrently) race on it.
+// contents.  Calls of several threads or contexts take turns: each call's stream
+// waits for the event the call before recorded.
 #include <mutex>
 
 #include "cr_runtime.h"
@@ -25,8 +25,7 @@ using namespace cr;
 
 namespace {
 
-// Layout: [0, 64) work-queue counter, [256, 256 + 8 CR_PT_STATIC_MAX_FRAMES) the (seed, frameCount) pairs.
-constexpr size_t QUEUE_OFF = 0;
+// Layout: [256, 256 + 8 CR_PT_STATIC_MAX_FRAMES) the (seed, frameCount) pairs.
 constexpr size_t FRAMES_OFF = 256;
 static_assert(FRAMES_OFF + 8ull * CR_PT_STATIC_MAX_FRAMES == CR_PT_STATIC_SCRATCH_BYTES, "scratch layout");
 
@@ -35,6 +34,8 @@ static __device__ __align__(256) unsigned char scratch[CR_PT_STATIC_SCRATCH_BYTE
 constexpr int MAX_DEVICES = 64;
 std::mutex g_mutex;
 unsigned char* g_scratch[MAX_DEVICES] = {};   // this GPU's copy of `scratch`, by device ordinal
+hipEvent_t g_done[MAX_DEVICES] = {};          // recorded after the last call on it
+std::mutex g_turn[MAX_DEVICES];               // held while a call is enqueued
 
 unsigned char* scratch_of(int device)
 {
@@ -58,6 +59,8 @@ cr_status static_scratch_init(cr_context* ctx)
     void* p = nullptr;
     hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
     if (e != hipSuccess) return hip_fail(ctx, e, "hipGetSymbolAddress(scratch)");
+    e = hipEventCreateWithFlags(&g_done[ctx->device], hipEventDisableTiming);
+    if (e != hipSuccess) return hip_fail(ctx, e, "hipEventCreate(static render)");
     g_scratch[ctx->device] = (unsigned char*)p;
     return CR_OK;
 }
@@ -90,21 +93,24 @@ cr_status cr_pt_render_static(cr_context* ctx, const cr_push_constants* frames, 
         fr[2 * i + 1] = (int32_t)frames[i].frameCount;
     }
     int32_t* dFrames = (int32_t*)(base + FRAMES_OFF);
-    // stream order: the copy waits for any earlier kernel that still reads the table
+    std::lock_guard<std::mutex> turn(g_turn[ctx->device]);
+    // the copy waits for any earlier kernel that still reads the table
+    CR_HIP(ctx, hipStreamWaitEvent(ctx->stream, g_done[ctx->device], 0), "wait for the static scratch");
     CR_HIP(ctx, hipMemcpyAsync(dFrames, fr, (size_t)n_frames * 8, hipMemcpyHostToDevice, ctx->stream), "copy frames");
     CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync frames");
-    CR_HIP(ctx, zero_async(base + QUEUE_OFF, 64, ctx->stream), "clear queue");
+    CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "clear queue");
 
     PTArgs a;
     fill_job_args(a, ctx->grid, ctx->sv, ctx->svDimsBuilt, ctx->cam, ctx->cloud, ctx->params, ctx->svp, ctx->ext,
                   dFrames, n_frames, accum, ctx->W, ctx->H, ctx->ptTileLog2W);
-    a.queue = (uint32_t*)(base + QUEUE_OFF);
+    a.queue = ctx->dQueue;
     a.counters = nullptr;
     const DeviceGrid& g = ctx->grid;
     int blocks = ctx->numCUs * pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, n_frames);
     const uint32_t needed = (a.totalIdx + 255u) / 256u;
     if ((uint32_t)blocks > needed) blocks = (int)needed;
     CR_HIP(ctx, launch_pt(a, g.dtype, g.layout, blocks, ctx->stream), "path tracer kernel");
+    CR_HIP(ctx, hipEventRecord(g_done[ctx->device], ctx->stream), "static render event");
     return CR_OK;
 }
 
