@@ -41,3 +41,14 @@ def test_lookups_bitexact(ctx, cfg, S, O, dims, scale, half):
         # (it shows where a ray crosses more than 88 mean free paths).
         img = ctx.download_image(h, w).reshape(-1, 4)[1:]
         assert_bitexact(img, ref.reshape(-1, 4)[1:], f"image, light {light}")
+
+
+# 320 x 511 columns are summed in two passes, 320 x 512 in one; 17 texels: one
+# more than the second pass fetches together
+@pytest.mark.parametrize("dims", [(2, 2, 2), (65, 5, 17), (320, 511, 3), (320, 512, 3), (9, 7, 33)])
+def test_shadow_volume_passes(ctx, cfg, S, O, dims):
+    sc = cfg.c1(width=4, height=4, size=24, sv_axis=33)
+    sc.ext = cfg.render_ext(albedo=0.9, bounce_cap=16, sky=cfg.SKY, sv_dims=dims)
+    cloud, svp = sc.setup(ctx)
+    s, _, sv = oracle_scene_from_ctx(O, ctx, sc.cam, sc.params, svp, sc.ext)
+    assert_bitexact(sv, O.sv_build(s), f"shadow volume of {dims}")
