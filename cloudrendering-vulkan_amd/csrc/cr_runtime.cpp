@@ -120,13 +120,11 @@ cr_status cr_create(int device, cr_context** out)
     cr_photon_map_default(&ctx->pm);
     if (ensure_buffer(ctx, (void**)&ctx->dQueue, &ctx->queueCap, PT_QUEUE_WORDS * 4, "queue") != CR_OK ||
         ensure_buffer(ctx, (void**)&ctx->dCounters, &ctx->countersCap, COUNTER_WORDS * sizeof(unsigned long long), "counters") != CR_OK ||
+        ensure_buffer(ctx, (void**)&ctx->staticFrames, &ctx->staticFramesCap, CR_PT_STATIC_SCRATCH_BYTES, "static frames") !=
+            CR_OK ||
         ensure_buffer(ctx, (void**)&ctx->dScalar, &ctx->scalarCap, 64, "scalar") != CR_OK) {
         cr_destroy(ctx);
         return CR_ERR_OUT_OF_MEMORY;
-    }
-    if (static_scratch_init(ctx) != CR_OK) {
-        cr_destroy(ctx);
-        return CR_ERR_DEVICE;
     }
     zero_async(ctx->dCounters, COUNTER_WORDS * sizeof(unsigned long long), ctx->stream);
     hipStreamSynchronize(ctx->stream);
@@ -141,7 +139,7 @@ cr_status cr_destroy(cr_context* ctx)
     if (ctx->stream) hipStreamSynchronize(ctx->stream);
     void* bufs[] = {ctx->grid.data, ctx->grid.majorants, ctx->grid.skip, ctx->sv, ctx->image, ctx->dFrames, ctx->dQueue,
                     ctx->tileList, ctx->ptSamples,
-                    ctx->dCounters, ctx->dScalar};
+                    ctx->dCounters, ctx->staticFrames, ctx->dScalar};
     for (void* b : bufs)
         if (b) hipFree(b);
     ppb_free(ctx);

@@ -211,13 +211,11 @@ CR_API cr_status cr_pt_upload(cr_context* ctx, const float* rgba);
  * loops, harnesses that forbid hipMalloc): cr_pt_render's frames rendered
  * into a caller-owned device image `accum` (W x H RGBA32F of the current
  * camera, read and written as the running mean) with no allocation.  The
- * per-frame seed table is one fixed CR_PT_STATIC_SCRATCH_BYTES array per GPU,
- * resolved at cr_create, the work-queue counter the context's; at most
- * CR_PT_STATIC_MAX_FRAMES frames per call (CR_ERR_CAPACITY beyond).  Whole
- * pixels are claimed in raster order; every pixel equals cr_pt_render's bit for
- * bit.  cr_pt_stats does not see these launches.  The array is shared by every
- * context on a GPU: calls of several contexts or threads take turns, each
- * waiting for the render before it.  Blocks until the
+ * per-frame seed table (CR_PT_STATIC_SCRATCH_BYTES) and the work-queue counters
+ * are made with the context at cr_create; at most CR_PT_STATIC_MAX_FRAMES frames
+ * per call (CR_ERR_CAPACITY beyond).  Whole pixels are claimed in raster order;
+ * every pixel equals cr_pt_render's bit for bit.  cr_pt_stats does not see these
+ * launches.  Contexts share nothing, so their calls may overlap.  Blocks until the
  * frame table is copied, then returns with the render queued on the
  * context's stream (cr_synchronize waits for it). */
 #define CR_PT_STATIC_MAX_FRAMES 4096u
