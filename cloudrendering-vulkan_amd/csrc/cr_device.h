@@ -85,8 +85,10 @@ __device__ __forceinline__ f3 ld3(const float* p) { return mk(p[0], p[1], p[2]);
 __device__ __forceinline__ float fdiv(float a, float b) { return __fdiv_rn(a, b); }
 
 // log x for a normal, finite x > 0 (scaled by 2^e0 before the call): the
-// core of crd_logf without its special cases.  xs_float's values, in
-// [2^-32, 1], are such x, so the free-flight draws call this directly.
+// core of crd_logf without its special cases.  xs_float's values are such x, in
+// [2^-32, 1], unless the generator's state is 0 (then they are all 0); the path
+// tracer's free-flight draws call this directly and take that state by itself
+// where a segment begins.
 __device__ __forceinline__ float crd_log_normal(float x, int32_t e0 = 0)
 {
     int32_t e = e0;

@@ -211,10 +211,16 @@ __device__ __forceinline__ bool begin_segment(const cr::PTArgs& a, Lane& L, f3 d
     if (!intersect_box_inv(B0(a), B1(a), L.pos, invd, tmin, tmax)) return false;
     f3 exitp = add(L.pos, mul(dir, tmax));
     L.dist = length(sub(L.pos, exitp));
-    L.t = 0.0f;
+    // The state 0 draws nothing but 0, whose flights -log 0 are infinite: such a
+    // path leaves every segment.  No other state ever becomes 0, so this is the
+    // one place that has to look (one select per segment).
     if (TRACK == CR_TRACK_BRICK_DDA) {
+        L.t = 0.0f;
         dda_init(a, L.pos, dir, invd, L);
-        L.tau = -crd_log_normal(xs_float(L.rng));
+        const float tau = -crd_log_normal(xs_float(L.rng));
+        L.tau = L.rng != 0u ? tau : __builtin_inff();
+    } else {
+        L.t = L.rng != 0u ? 0.0f : __builtin_inff();
     }
     return true;
 }
