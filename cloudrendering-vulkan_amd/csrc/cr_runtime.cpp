@@ -796,16 +796,9 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
         if (sample_buffer(&ctx->ptSamples, &ctx->ptSamplesCap, px * group)) a.samples = ctx->ptSamples;
         else group = n_frames;
     }
-    CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
     if (n_frames > 1) {
-        // the tiles to claim, by XCD (a single frame takes all tiles in raster
-        // order: the lists cost it more than they bring)
         st = ensure_buffer(ctx, (void**)&ctx->tileList, &ctx->tileListCap, (size_t)pt_list_words(a) * 4, "tile list");
         if (st != CR_OK) return st;
-        CR_HIP(ctx, launch_pt_list(a, ctx->tileList, ctx->stream), "tile list kernels");
-        a.tileOrder = ctx->tileList + pt_list_starts(a) - a.totalIdx / 64u;
-        a.partStart = ctx->tileList + pt_list_starts(a);
-        a.logParts = 3;
     }
     if (ctx->ptEventsUsed >= 1024) {
         st = fold_pt_events(ctx);
@@ -818,7 +811,17 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
         ctx->ptEvents.push_back(ev);
     }
     const auto& ev = ctx->ptEvents[ctx->ptEventsUsed];
+    // the measured time starts before the listing, which renders the sky's pixels
     CR_HIP(ctx, hipEventRecord(ev.first, ctx->stream), "event");
+    CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
+    if (n_frames > 1) {
+        // the tiles to claim, by XCD (a single frame takes all tiles in raster
+        // order: the lists cost it more than they bring)
+        CR_HIP(ctx, launch_pt_list(a, ctx->tileList, ctx->stream), "tile list kernels");
+        a.tileOrder = ctx->tileList + pt_list_starts(a) - a.totalIdx / 64u;
+        a.partStart = ctx->tileList + pt_list_starts(a);
+        a.logParts = 3;
+    }
     for (uint32_t f0 = 0; f0 < n_frames; f0 += group) {
         PTArgs b = a;
         b.nFrames = std::min(group, n_frames - f0);
