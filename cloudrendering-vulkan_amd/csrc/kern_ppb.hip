@@ -186,11 +186,8 @@ __global__ void __launch_bounds__(256) trace_kernel(cr::TraceArgs a)
 
 // One wave per record: its beam data and its segments, in the slots its path
 // and its place on the path give it.
-__global__ void __launch_bounds__(256) expand_kernel(cr::TraceArgs a, uint64_t nRecords)
+__device__ __forceinline__ void expand_record(const cr::TraceArgs& a, uint64_t ri, uint32_t lane)
 {
-    const uint64_t ri = (uint64_t)blockIdx.x * 4 + threadIdx.x / 64;
-    const uint32_t lane = threadIdx.x & 63u;
-    if (ri >= nRecords) return;
     const cr::BeamRecord& rec = a.records[ri];
     const uint32_t id = __float_as_uint(rec.head[7]);
     if (id >= a.nPaths) return;
@@ -221,6 +218,17 @@ __global__ void __launch_bounds__(256) expand_kernel(cr::TraceArgs a, uint64_t n
         B[1] = make_uint4(__float_as_uint(en.x), __float_as_uint(en.y), __float_as_uint(en.z), __float_as_uint(r));
         B[2] = make_uint4((uint32_t)di, __float_as_uint(off), 0u, 0u);
     }
+}
+
+// A grid dimension holds fewer than 2^32 threads and a launch beyond that runs
+// only a part of them, without an error: past EXPAND_BLOCKS workgroups of four
+// waves (2^22 records) the waves go on to further records.
+constexpr uint32_t EXPAND_BLOCKS = 1u << 20;
+
+__global__ void __launch_bounds__(256) expand_kernel(cr::TraceArgs a, uint64_t nRecords)
+{
+    for (uint64_t ri = (uint64_t)blockIdx.x * 4 + threadIdx.x / 64; ri < nRecords; ri += (uint64_t)gridDim.x * 4)
+        expand_record(a, ri, threadIdx.x & 63u);
 }
 
 // A ray with a direction component exactly 0 keeps that coordinate for every
@@ -528,7 +536,8 @@ hipError_t launch_trace(const TraceArgs& a, int dtype, int layout, hipStream_t s
 hipError_t launch_trace_expand(const TraceArgs& a, uint64_t records, hipStream_t s)
 {
     if (records == 0) return hipSuccess;
-    hipLaunchKernelGGL(expand_kernel, dim3((unsigned)((records + 3) / 4)), dim3(256), 0, s, a, records);
+    const uint64_t blocks = (records + 3) / 4;
+    hipLaunchKernelGGL(expand_kernel, dim3((unsigned)(blocks < EXPAND_BLOCKS ? blocks : EXPAND_BLOCKS)), dim3(256), 0, s, a, records);
     return hipGetLastError();
 }
 
