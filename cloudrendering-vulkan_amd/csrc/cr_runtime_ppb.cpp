@@ -98,6 +98,20 @@ static const uint32_t MAX_BEAMS = 1u << 28;
 static const uint64_t TRACE_PATHS = 1u << 18;            // photon paths per launch of the producer at most
 static const size_t TRACE_KEEP = (size_t)1 << 30;        // bytes of beam records kept between traces at most
 
+namespace {
+// Gives the records of a large trace back, whichever way it ends.
+struct TrimRecords {
+    Ppb* p;
+    ~TrimRecords()
+    {
+        if (p->recordsCap <= TRACE_KEEP) return;
+        hipFree(p->records);
+        p->records = nullptr;
+        p->recordsCap = 0;
+    }
+};
+} // namespace
+
 // Sort, tree and traversal buffers for n beams (grown, never shrunk).
 static cr_status lbvh_buffers(cr_context* ctx, Ppb* p, uint32_t n)
 {
@@ -180,6 +194,7 @@ cr_status cr_ppb_trace_beams(cr_context* ctx, const cr_beam_trace_params* prm, u
     hipSetDevice(ctx->device);
     Ppb* p;
     CR_TRY(ppb_get(ctx, &p));
+    const TrimRecords trim{p};
     const uint32_t P = prm->numPaths;
     const DeviceGrid& g = ctx->grid;
     TraceArgs a;
@@ -230,8 +245,13 @@ cr_status cr_ppb_trace_beams(cr_context* ctx, const cr_beam_trace_params* prm, u
             // more records than there is room for: make room, keep those of
             // the earlier launches and trace these paths again
             BeamRecord* more = nullptr;
-            const size_t bytes = (size_t)(total + total / 2) * sizeof(BeamRecord);
+            size_t bytes = (size_t)(total + total / 2) * sizeof(BeamRecord);
             hipError_t e = hipMalloc((void**)&more, bytes);
+            if (e != hipSuccess) {  // no room for more than these
+                (void)hipGetLastError();
+                bytes = (size_t)total * sizeof(BeamRecord);
+                e = hipMalloc((void**)&more, bytes);
+            }
             if (e != hipSuccess) return fail(ctx, CR_ERR_OUT_OF_MEMORY, std::string("hipMalloc beam records: ") + hipGetErrorString(e));
             if (records) e = hipMemcpyAsync(more, p->records, (size_t)records * sizeof(BeamRecord), hipMemcpyDeviceToDevice, ctx->stream);
             if (e == hipSuccess) e = hipMemcpyAsync(p->recordCount, &records, 8, hipMemcpyHostToDevice, ctx->stream);
@@ -253,10 +273,10 @@ cr_status cr_ppb_trace_beams(cr_context* ctx, const cr_beam_trace_params* prm, u
             sb += hc[i];
         }
         done += n;
+        if (sd > MAX_BEAMS) return fail(ctx, CR_ERR_CAPACITY, "beam data exceeds 2^28 records");
     }
     const uint64_t nb = sb < max_beams ? sb : max_beams;
     const uint64_t nd = sd;
-    if (nd > MAX_BEAMS) return fail(ctx, CR_ERR_CAPACITY, "beam data exceeds 2^28 records");
     CR_TRY(ensure_buffer(ctx, (void**)&p->beams, &p->beamsCap, (size_t)nb * sizeof(cr_photon_beam), "beams"));
     CR_TRY(ensure_buffer(ctx, (void**)&p->data, &p->dataCap, (size_t)nd * sizeof(cr_photon_beam_data), "beam data"));
     CR_TRY(ensure_buffer(ctx, (void**)&p->pathOffsets, &p->pathOffsetsCap, (size_t)done * 16, "path offsets"));
@@ -273,11 +293,6 @@ cr_status cr_ppb_trace_beams(cr_context* ctx, const cr_beam_trace_params* prm, u
     a.maxData = nd;
     CR_HIP(ctx, launch_trace_expand(a, records, ctx->stream), "beam expansion");
     CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "beam expansion");
-    if (p->recordsCap > TRACE_KEEP) {
-        hipFree(p->records);
-        p->records = nullptr;
-        p->recordsCap = 0;
-    }
     p->n = (uint32_t)nb;
     p->nData = (uint32_t)nd;
     p->built = false;

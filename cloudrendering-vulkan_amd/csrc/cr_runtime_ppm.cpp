@@ -65,6 +65,21 @@ static Ppm* ppm_get(cr_context* ctx)
 
 static const uint32_t MAX_DEPOSITS = 1u << 28;
 static const size_t RECORDS_KEEP = (size_t)1 << 30;   // bytes of deposit records kept between traces at most
+
+namespace {
+// Gives the records of a large trace back, whichever way it ends.
+struct TrimRecords {
+    Ppm* p;
+    ~TrimRecords()
+    {
+        if (p->recordsCap <= RECORDS_KEEP) return;
+        hipFree(p->records);
+        p->records = nullptr;
+        p->recordsCap = 0;
+    }
+};
+} // namespace
+
 static const uint64_t MAX_CELLS = 1ull << 27;
 
 extern "C" {
@@ -171,6 +186,7 @@ cr_status cr_ppm_trace(cr_context* ctx, int32_t seed, const cr_ppm_params* prm, 
     if (!ctx->hasPm) return fail(ctx, CR_ERR_STATE, "no photon map properties (cr_set_photon_map)");
     hipSetDevice(ctx->device);
     Ppm* p = ppm_get(ctx);
+    const TrimRecords trim{p};
     p->valid = false;
     const uint32_t P = prm->numPaths;
     const uint64_t nCells = (uint64_t)ctx->pm.voxelCount[0] * ctx->pm.voxelCount[1] * ctx->pm.voxelCount[2];
@@ -202,6 +218,7 @@ cr_status cr_ppm_trace(cr_context* ctx, int32_t seed, const cr_ppm_params* prm, 
     a.lanes = 8;
     while (a.lanes < 64u && a.lanes * 512u < P) a.lanes *= 2u;
     unsigned long long chunks = 0;
+    uint64_t n = 0;  // deposits
     // chunks to have room for: half as many as paths, or what an earlier trace needed
     uint64_t room = P / 2u + 64u;
     if (p->recordsCap / sizeof(PpmRecord) > (uint64_t)P * PPM_FIRST)
@@ -219,16 +236,15 @@ cr_status cr_ppm_trace(cr_context* ctx, int32_t seed, const cr_ppm_params* prm, 
         CR_HIP(ctx, hipMemcpyAsync(counts.data(), p->pathCounts, (size_t)P * 4, hipMemcpyDeviceToHost, s), "copy counts");
         CR_HIP(ctx, hipMemcpyAsync(&chunks, p->chunkCount, 8, hipMemcpyDeviceToHost, s), "copy chunk count");
         CR_HIP(ctx, hipStreamSynchronize(s), "sync");
-        if (chunks <= room) break;
-        // more deposits than there is room for: make room and trace again
-        if (chunks > MAX_DEPOSITS) return fail(ctx, CR_ERR_CAPACITY, "more than 2^28 photon deposits in one trace");
-        room = chunks;
-    }
-    uint64_t n = 0;
-    for (uint32_t i = 0; i < P; i++) {
-        offsets[i] = (uint32_t)n;
-        n += counts[i];
+        n = 0;
+        for (uint32_t i = 0; i < P; i++) {
+            offsets[i] = (uint32_t)n;
+            n += counts[i];
+        }
+        // (the counts are whole even where the records did not fit)
         if (n > MAX_DEPOSITS) return fail(ctx, CR_ERR_CAPACITY, "more than 2^28 photon deposits in one trace");
+        if (chunks <= room) break;
+        room = chunks;  // more deposits than there is room for: make room and trace again
     }
     const uint32_t nd = (uint32_t)n;
     CR_TRY(ensure_buffer(ctx, (void**)&p->arrivals, &p->arrivalsCap, (size_t)nCells * 4, "cell arrivals"));
@@ -255,11 +271,6 @@ cr_status cr_ppm_trace(cr_context* ctx, int32_t seed, const cr_ppm_params* prm, 
                "cell runs");
     }
     CR_HIP(ctx, hipStreamSynchronize(s), "sync");
-    if (p->recordsCap > RECORDS_KEEP) {
-        hipFree(p->records);
-        p->records = nullptr;
-        p->recordsCap = 0;
-    }
     p->nDeposits = nd;
     p->nCells = (uint32_t)nCells;
     p->valid = true;
