@@ -7,6 +7,7 @@
 
 #include "../../include/cr/abi.h"
 #include "cr_device.h"
+#include "pt_schedule.h"
 
 namespace cr {
 
@@ -94,7 +95,6 @@ struct BatchArgs {
 // kern_pt.hip: a render of a.nFrames frames; launches whose work items hold
 // at most PT_FEW_FRAMES frames use the instantiation with gated pixel claims
 // (kern_pt_few.hip), which is faster when an item carries little work.
-constexpr uint32_t PT_FEW_FRAMES = 16;
 // Atomics on one cache line are carried out one by one, some 14 ns each: the
 // parts' queue words lie 256 bytes apart.
 constexpr uint32_t PT_QUEUE_STRIDE = 64, PT_QUEUE_WORDS = 8 * PT_QUEUE_STRIDE;
@@ -103,28 +103,6 @@ constexpr uint32_t PT_QUEUE_STRIDE = 64, PT_QUEUE_WORDS = 8 * PT_QUEUE_STRIDE;
 // (In one copy the 4096 waves of a launch waited 280 us for each other at its
 // end: 512x512 at 1 spp 1.28 ms against 1.01.)
 constexpr uint32_t COUNTER_SLOTS = 64, COUNTER_STRIDE = 32, COUNTER_WORDS = COUNTER_SLOTS * COUNTER_STRIDE;
-// Work items of a chunked pass: at least this many per resident lane while
-// there are samples to make them of, each of at most PT_FEW_FRAMES samples.
-// Frames per work item of a chunked pass: at least PT_ITEMS_PER_LANE items per
-// resident lane while there are samples to make them of, each of at most
-// `most` samples.  Renders: chunks of 4 measured best where samples abound (a
-// 16-job batch: 125 ms with chunks of up to 16, 101 with 8, 85 with 4, 95 with
-// 1; 512x512 at 128 spp: 26.0, -, 20.6, 23.4), and 8 items per lane where they
-// do not (256x256 at 64 spp: 3.18 ms; with 4 items 3.47, with 32 3.32).
-// Record passes, whose samples are short, pay for the set-up of more items
-// (1080p at 32 spp, the whole learned render: 27.7 ms with 16, 29.0 with 4).
-constexpr uint64_t PT_ITEMS_PER_LANE = 8;
-constexpr uint32_t PT_CHUNK_RENDER = 4, PT_CHUNK_RECORD = 16;
-static_assert(PT_CHUNK_RENDER <= PT_FEW_FRAMES && PT_CHUNK_RECORD <= PT_FEW_FRAMES, "chunked items are few-frame items");
-inline uint32_t pt_chunk(uint64_t pixels, uint32_t samples, uint64_t lanes, uint32_t most)
-{
-    const uint64_t c = pixels * samples / (PT_ITEMS_PER_LANE * lanes);
-    return (uint32_t)(c < 1 ? 1 : (c > most ? most : c));
-}
-// Samples stored by one chunked launch at most (4 GiB); more go in several
-// launches, each of which ends on its longest paths (16-job batch: 88.6 ms
-// with 1 GiB).
-constexpr uint64_t PT_SAMPLE_BUDGET = 1ull << 28;
 hipError_t launch_pt(const PTArgs& a, int dtype, int layout, int grid_blocks, hipStream_t s);
 int pt_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee, uint32_t chunk);
 // The tile list of a render (lists: pt_list_words(a) words; the list ends where

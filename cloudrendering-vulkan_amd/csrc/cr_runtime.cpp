@@ -827,7 +827,7 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
         b.nFrames = std::min(group, n_frames - f0);
         b.frames = a.frames + 2 * (size_t)f0;
         b.chunk = b.nFrames;
-        if (a.samples) set_chunk(b, pt_chunk(px, b.nFrames, lanes, PT_CHUNK_RENDER));
+        if (a.samples) set_chunk(b, pt_chunk(px, b.nFrames, lanes, PT_ITEMS_RENDER, PT_CHUNK_RENDER));
         int blocks = ctx->numCUs * pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, b.chunk);
         const uint32_t needed = (b.totalIdx + 255u) / 256u;
         if ((uint32_t)blocks > needed) blocks = (int)needed;

@@ -184,7 +184,7 @@ cr_status build_groups(cr_context* ctx, Batch* b, const std::vector<uint32_t>& w
             PTArgs a;
             fill_job_args(a, j.grid, j.sv, j.svDims, j.cam, j.cloud, j.params, j.svp, j.ext, j.dFrames + 2 * (size_t)f0,
                           take, images ? (*images)[k] : j.image, j.W, j.H, tile_log2(tuning.tileWidth));
-            if (store && fits && take > 1) set_chunk(a, pt_chunk(budget, 1, lanes, PT_CHUNK_RENDER));
+            if (store && fits && take > 1) set_chunk(a, pt_chunk(budget, 1, lanes, PT_ITEMS_RENDER, PT_CHUNK_RENDER));
             if ((uint64_t)g.total + a.totalIdx >= (1ull << 31)) close();
             a.base = g.total;
             a.blendBase = g.blendBlocks;

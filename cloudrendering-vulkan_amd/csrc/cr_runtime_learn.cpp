@@ -196,14 +196,11 @@ cr_status check_render_state(cr_context* ctx)
     return CR_OK;
 }
 
-int pass_blocks(cr_context* ctx, int continuation, uint32_t work)
+// Workgroups of a record (or continuation) pass the chip holds at a time.
+int pass_resident(cr_context* ctx, int continuation)
 {
-    const int per_cu = pt_learn_blocks_per_cu(ctx->grid.dtype, ctx->grid.layout, ctx->ext.trackingMode, ctx->ext.neeMode,
-                                              continuation);
-    int blocks = ctx->numCUs * per_cu;
-    const uint32_t needed = (work + 255u) / 256u;
-    if ((uint32_t)blocks > needed) blocks = (int)needed;
-    return blocks > 0 ? blocks : 1;
+    return ctx->numCUs * pt_learn_blocks_per_cu(ctx->grid.dtype, ctx->grid.layout, ctx->ext.trackingMode, ctx->ext.neeMode,
+                                                continuation);
 }
 
 // Record pass of n_frames frames into L->records; returns the record count.
@@ -215,11 +212,13 @@ cr_status record_pass(cr_context* ctx, Learn* L, const cr_push_constants* frames
     CR_TRY(ensure_buffer(ctx, (void**)&L->records, &L->recordsCap, n * 32, "records"));
     PTArgs a;
     CR_TRY(fill_pt_args(ctx, a, n_frames));
-    set_chunk(a, pt_chunk((uint64_t)ctx->W * (uint64_t)ctx->H, n_frames, (uint64_t)pass_blocks(ctx, 0, ~0u) * 256u, PT_CHUNK_RECORD));
+    const int resident = pass_resident(ctx, 0);
+    set_chunk(a, pt_chunk((uint64_t)ctx->W * (uint64_t)ctx->H, n_frames, (uint64_t)resident * 256u, PT_ITEMS_RECORD,
+                         PT_CHUNK_RECORD));
     a.records = L->records;
     a.counters = nullptr;
     CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
-    CR_HIP(ctx, launch_pt_record(a, ctx->grid.dtype, ctx->grid.layout, pass_blocks(ctx, 0, a.totalIdx), ctx->stream),
+    CR_HIP(ctx, launch_pt_record(a, ctx->grid.dtype, ctx->grid.layout, pt_blocks(a.totalIdx, resident), ctx->stream),
            "record pass");
     *n_out = n;
     return CR_OK;
@@ -252,7 +251,7 @@ cr_status continue_pass(cr_context* ctx, const float* pts, uint32_t m, uint32_t 
         a.chunk = a.samples ? 1u : a.spp;
         a.totalIdx = m * ((a.spp + a.chunk - 1u) / a.chunk);
         CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
-        CR_HIP(ctx, launch_pt_continue(a, ctx->grid.dtype, ctx->grid.layout, pass_blocks(ctx, 1, a.totalIdx), ctx->stream),
+        CR_HIP(ctx, launch_pt_continue(a, ctx->grid.dtype, ctx->grid.layout, pt_blocks(a.totalIdx, pass_resident(ctx, 1)), ctx->stream),
                "continuation pass");
         if (a.samples) CR_HIP(ctx, launch_pt_sum(a, spp, ctx->stream), "continuation sums");
     }
