@@ -29,6 +29,34 @@ cr_status hip_fail(cr_context* ctx, hipError_t e, const char* what)
     return fail(ctx, CR_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+bool release_scratch(cr_context* ctx)
+{
+    bool any = false;
+    if (ctx->ptSamples) {
+        hipFree(ctx->ptSamples);  // waits for the kernels that use it
+        ctx->ptSamples = nullptr;
+        ctx->ptSamplesCap = 0;
+        any = true;
+    }
+    any = batch_release_samples(ctx) || any;
+    any = ppb_release_records(ctx) || any;
+    return ppm_release_records(ctx) || any;
+}
+
+hipError_t device_alloc(cr_context* ctx, void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        if (release_scratch(ctx)) e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 cr_status ensure_buffer(cr_context* ctx, void** p, size_t* cap, size_t bytes, const char* what)
 {
     if (*cap >= bytes && *p) return CR_OK;
@@ -38,9 +66,8 @@ cr_status ensure_buffer(cr_context* ctx, void** p, size_t* cap, size_t bytes, co
         *cap = 0;
     }
     if (bytes == 0) return CR_OK;
-    hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = device_alloc(ctx, p, bytes);
     if (e != hipSuccess) {
-        *p = nullptr;
         return fail(ctx, CR_ERR_OUT_OF_MEMORY, std::string("hipMalloc ") + what + " (" + std::to_string(bytes) + " B): " +
                                                    hipGetErrorString(e));
     }
@@ -199,9 +226,8 @@ cr_status grid_alloc(cr_context* ctx, int32_t nx, int32_t ny, int32_t nz, int dt
         g.bytes = 0;
     }
     if (!g.data) {
-        hipError_t e = hipMalloc(&g.data, bytes);
+        hipError_t e = device_alloc(ctx, &g.data, bytes);
         if (e != hipSuccess) {
-            g.data = nullptr;
             return fail(ctx, CR_ERR_OUT_OF_MEMORY, std::string("hipMalloc grid: ") + hipGetErrorString(e));
         }
         g.bytes = bytes;
@@ -233,8 +259,8 @@ cr_status majorants_build(cr_context* ctx, DeviceGrid& g, int mb)
         g.skip = nullptr;
     }
     if (!g.majorants) {
-        hipError_t e = hipMalloc((void**)&g.majorants, n * sizeof(float));
-        if (e == hipSuccess) e = hipMalloc((void**)&g.skip, 2 * n * sizeof(float));
+        hipError_t e = device_alloc(ctx, (void**)&g.majorants, n * sizeof(float));
+        if (e == hipSuccess) e = device_alloc(ctx, (void**)&g.skip, 2 * n * sizeof(float));
         if (e != hipSuccess) {
             if (g.majorants) hipFree(g.majorants);
             g.majorants = nullptr;
@@ -246,8 +272,13 @@ cr_status majorants_build(cr_context* ctx, DeviceGrid& g, int mb)
     CR_HIP(ctx, launch_majorants(g.data, g.dtype, g.layout, g.nx, g.ny, g.nz, g.nbx, g.nby, mb, g.majorants, mx, my, mz,
                                  ctx->stream), "majorant kernel");
     uint8_t* tmp = nullptr;
-    CR_HIP(ctx, hipMallocAsync((void**)&tmp, 2 * n, ctx->stream), "skip scratch");
-    hipError_t e = launch_skip_grid(g.majorants, mx, my, mz, ctx->cloud.densityScaling, ctx->cloud.baseScaling, g.skip, tmp,
+    hipError_t e = hipMallocAsync((void**)&tmp, 2 * n, ctx->stream);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        if (release_scratch(ctx)) e = hipMallocAsync((void**)&tmp, 2 * n, ctx->stream);
+    }
+    CR_HIP(ctx, e, "skip scratch");
+    e = launch_skip_grid(g.majorants, mx, my, mz, ctx->cloud.densityScaling, ctx->cloud.baseScaling, g.skip, tmp,
                                     ctx->stream);
     hipError_t e2 = hipFreeAsync(tmp, ctx->stream);
     CR_HIP(ctx, e, "skip grid");
@@ -311,7 +342,7 @@ cr_status cr_grid_upload(cr_context* ctx, const cr_grid_header* hdr, const void*
     size_t n = (size_t)hdr->sizeX * hdr->sizeY * hdr->sizeZ;
     size_t srcBytes = n * (src_dtype == CR_DTYPE_F16 ? 2 : 4);
     void* staging = nullptr;
-    CR_HIP(ctx, hipMalloc(&staging, srcBytes), "hipMalloc staging");
+    CR_HIP(ctx, device_alloc(ctx, &staging, srcBytes), "hipMalloc staging");
     hipError_t e = hipMemcpyAsync(staging, data, srcBytes, hipMemcpyHostToDevice, ctx->stream);
     cr_status st = CR_OK;
     if (e != hipSuccess) st = hip_fail(ctx, e, "upload");
@@ -354,7 +385,7 @@ cr_status cr_grid_download(cr_context* ctx, float* out)
     DeviceGrid& g = ctx->grid;
     size_t n = (size_t)g.nx * g.ny * g.nz;
     float* tmp = nullptr;
-    CR_HIP(ctx, hipMalloc((void**)&tmp, n * 4), "hipMalloc");
+    CR_HIP(ctx, device_alloc(ctx, (void**)&tmp, n * 4), "hipMalloc");
     hipError_t e = launch_grid_to_f32(g.data, g.dtype, g.layout, tmp, g.nx, g.ny, g.nz, g.nbx, g.nby, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, n * 4, hipMemcpyDeviceToHost, ctx->stream);
     hipError_t e2 = hipStreamSynchronize(ctx->stream);
@@ -395,7 +426,7 @@ cr_status cr_math_probe(cr_context* ctx, int op, const float* in, uint32_t n, fl
     if (n == 0) return CR_OK;
     if (!in || !out) return fail(ctx, CR_ERR_INVALID_ARGUMENT, "null array");
     float* d = nullptr;
-    hipError_t e = hipMalloc(&d, (size_t)n * 8);
+    hipError_t e = device_alloc(ctx, (void**)&d, (size_t)n * 8);
     if (e != hipSuccess) return hip_fail(ctx, e, "probe buffer");
     e = hipMemcpyAsync(d, in, (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = launch_math_probe(op, d, n, d + n, ctx->stream);
@@ -726,21 +757,19 @@ void set_chunk(PTArgs& a, uint32_t chunk)
     a.totalIdx *= chunks;
 }
 
-// Scratch for `count` stored samples; false (and nothing allocated) when the
-// device has no room for it, where the caller renders without storing them.
-bool sample_buffer(float4** p, size_t* cap, uint64_t count)
+uint64_t sample_buffer(float4** p, size_t* cap, uint64_t want, uint64_t least)
 {
-    if (*p && *cap >= count) return true;
+    if (*p && *cap >= want) return want;
+    const uint64_t had = *cap;
     if (*p) hipFree(*p);
     *p = nullptr;
-    *cap = 0;
-    if (hipMalloc((void**)p, count * sizeof(float4)) != hipSuccess) {
+    *cap = (size_t)pt_sample_room(want, least, had, [&](uint64_t n) {
+        if (hipMalloc((void**)p, n * sizeof(float4)) == hipSuccess) return true;
         (void)hipGetLastError();
         *p = nullptr;
         return false;
-    }
-    *cap = count;
-    return true;
+    });
+    return *cap;
 }
 
 cr_status read_counters(cr_context* ctx, const unsigned long long* slots, unsigned long long* out, uint32_t n)
@@ -792,13 +821,15 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
                            (uint64_t)pt_blocks_per_cu(g.dtype, g.layout, ctx->ext.trackingMode, ctx->ext.neeMode, 1);
     uint32_t group = n_frames;  // frames per launch
     if (n_frames > 1) {
-        group = (uint32_t)std::min<uint64_t>(n_frames, std::max<uint64_t>(1, PT_SAMPLE_BUDGET / px));
-        if (sample_buffer(&ctx->ptSamples, &ctx->ptSamplesCap, px * group)) a.samples = ctx->ptSamples;
-        else group = n_frames;
-    }
-    if (n_frames > 1) {
         st = ensure_buffer(ctx, (void**)&ctx->tileList, &ctx->tileListCap, (size_t)pt_list_words(a) * 4, "tile list");
         if (st != CR_OK) return st;
+        const uint64_t most = std::min<uint64_t>(n_frames, std::max<uint64_t>(1, PT_SAMPLE_BUDGET / px));
+        const uint64_t room = sample_buffer(&ctx->ptSamples, &ctx->ptSamplesCap, px * most,
+                                            px * std::min<uint64_t>(most, PT_LEAST_STORED));
+        if (room) {
+            a.samples = ctx->ptSamples;
+            group = (uint32_t)(room / px);
+        }
     }
     if (ctx->ptEventsUsed >= 1024) {
         st = fold_pt_events(ctx);

@@ -79,7 +79,8 @@ struct cr_context {
     int ptBlocksOverride = 0;
     uint32_t* tileList = nullptr;   // tile schedule of the last render
     size_t tileListCap = 0;
-    // samples of a chunked render or continuation pass (at most PT_SAMPLE_BUDGET)
+    // samples of a chunked render or continuation pass (at most PT_SAMPLE_BUDGET,
+    // or one frame); optional scratch, as are the batch's and the traces' records
     float4* ptSamples = nullptr;
     size_t ptSamplesCap = 0;
     uint32_t ptTileLog2W = 3;                  // 8x8 pixel tiles
@@ -104,6 +105,10 @@ struct cr_context {
 namespace cr {
 cr_status fail(cr_context* ctx, cr_status code, const std::string& msg);
 cr_status hip_fail(cr_context* ctx, hipError_t e, const char* what);
+// hipMalloc for what a call cannot do without: when the device has no room, the
+// context's optional scratch (samples, trace records) is given up and it is
+// tried again.  Leaves no HIP error behind.
+hipError_t device_alloc(cr_context* ctx, void** p, size_t bytes);
 cr_status ensure_buffer(cr_context* ctx, void** p, size_t* cap, size_t bytes, const char* what);
 hipError_t zero_async(void* p, size_t bytes, hipStream_t s);
 // The first n statistics counters, summed over their COUNTER_SLOTS copies (synchronises the stream).
@@ -115,7 +120,15 @@ void fill_job_args(PTArgs& a, const DeviceGrid& g, const float* sv, const uint32
                    const cr_shadow_volume_properties& svp, const cr_render_ext& ext, const int32_t* frames,
                    uint32_t n_frames, float* image, int W, int H, uint32_t tileLog2W);
 void set_chunk(PTArgs& a, uint32_t chunk);
-bool sample_buffer(float4** p, size_t* cap, uint64_t count);
+// Room for samples: `want` of them, or fewer if the device has none for so many, at
+// least `least`; 0 (and nothing allocated) when not even those fit, and the caller
+// renders without storing them.  Holds until the context's next device_alloc.
+uint64_t sample_buffer(float4** p, size_t* cap, uint64_t want, uint64_t least);
+// The optional scratch of each part, freed unless in use; whether any was.
+bool release_scratch(cr_context* ctx);
+bool batch_release_samples(cr_context* ctx);
+bool ppb_release_records(cr_context* ctx);
+bool ppm_release_records(cr_context* ctx);
 cr_status fold_pt_events(cr_context* ctx);
 cr_status majorants_build(cr_context* ctx, DeviceGrid& g, int mb);
 void ppb_free(cr_context* ctx);

@@ -75,6 +75,7 @@ struct Batch {
     size_t scratchCap = 0;
     float4* dSamples = nullptr;     // a launch group's samples
     size_t samplesCap = 0;
+    bool samplesBusy = false;       // between laying out the groups and their launches
     std::vector<Group> groups;
     bool tableDirty = true, graphDirty = true;
     hipGraph_t graph = nullptr;
@@ -158,8 +159,11 @@ cr_status build_groups(cr_context* ctx, Batch* b, const std::vector<uint32_t>& w
     };
     for (size_t k = 0; k < which.size(); k++)
         all += (uint64_t)b->jobs[which[k]].W * (uint64_t)b->jobs[which[k]].H * frames_of(k);
-    const uint64_t budget = std::min(all, PT_SAMPLE_BUDGET);
-    const bool store = sample_buffer(&b->dSamples, &b->samplesCap, budget);
+    uint64_t budget = std::min(all, PT_SAMPLE_BUDGET), largest = 1;
+    for (uint32_t k : which) largest = std::max(largest, (uint64_t)b->jobs[k].W * (uint64_t)b->jobs[k].H);
+    const uint64_t room = sample_buffer(&b->dSamples, &b->samplesCap, budget, std::min(budget, largest * PT_LEAST_STORED));
+    const bool store = room != 0;
+    if (store) budget = room;
     const uint64_t lanes = (uint64_t)ctx->numCUs * tuning.blockThreads *
                            (uint64_t)blocks_per_cu(b, tuning, (uint32_t)which.size());
     Group g;
@@ -248,6 +252,13 @@ cr_status upload_table(cr_context* ctx, PTArgs** dst, size_t* cap, const std::ve
     return CR_OK;
 }
 
+// Keeps the samples the groups' tables point to until they are launched.
+struct SamplesBusy {
+    Batch* b;
+    explicit SamplesBusy(Batch* batch) : b(batch) { b->samplesBusy = true; }
+    ~SamplesBusy() { b->samplesBusy = false; }
+};
+
 // One trial: `which` jobs, each with 1/TRIAL_FRAME_DIV of its frames (so the
 // trial has the real mix of long and short pixels), into the scratch images;
 // returns the best of `reps` timed launches (after one untimed one).
@@ -264,6 +275,7 @@ cr_status trial(cr_context* ctx, Batch* b, const std::vector<uint32_t>& which, c
     }
     std::vector<PTArgs> table;
     std::vector<Group> groups;
+    const SamplesBusy busy(b);
     cr_status st = build_groups(ctx, b, which, t, &images, TRIAL_FRAME_DIV, &table, &groups);
     if (st == CR_OK) st = upload_table(ctx, &b->dTuneTable, &b->tuneTableCap, table, nullptr);
     if (st != CR_OK) return st;
@@ -331,6 +343,17 @@ void batch_free(cr_context* ctx)
     delete b;
     ctx->batch = nullptr;
 }
+
+bool batch_release_samples(cr_context* ctx)
+{
+    Batch* b = ctx->batch;
+    if (!b || !b->dSamples || b->samplesBusy) return false;
+    hipFree(b->dSamples);
+    b->dSamples = nullptr;
+    b->samplesCap = 0;
+    b->tableDirty = true;
+    return true;
+}
 } // namespace cr
 
 extern "C" {
@@ -365,13 +388,13 @@ cr_status cr_batch_add(cr_context* ctx, const cr_push_constants* frames, uint32_
     j.W = ctx->W;
     j.H = ctx->H;
     const size_t px = (size_t)j.W * j.H;
-    CR_HIP(ctx, hipMalloc((void**)&j.image, px * 16), "hipMalloc job image");
+    CR_HIP(ctx, device_alloc(ctx, (void**)&j.image, px * 16), "hipMalloc job image");
     std::vector<int32_t> fr(2 * (size_t)n_frames);
     for (uint32_t i = 0; i < n_frames; i++) {
         fr[2 * i] = frames[i].seed;
         fr[2 * i + 1] = (int32_t)frames[i].frameCount;
     }
-    hipError_t e = hipMalloc((void**)&j.dFrames, fr.size() * 4);
+    hipError_t e = device_alloc(ctx, (void**)&j.dFrames, fr.size() * 4);
     if (e == hipSuccess) e = hipMemcpyAsync(j.dFrames, fr.data(), fr.size() * 4, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = zero_async(j.image, px * 16, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -453,7 +476,7 @@ cr_status cr_batch_set_frames(cr_context* ctx, uint32_t job, const cr_push_const
     CR_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
     if (fr.size() * 4 > j.framesCap) {
         int32_t* p = nullptr;
-        CR_HIP(ctx, hipMalloc((void**)&p, fr.size() * 4), "hipMalloc frames");
+        CR_HIP(ctx, device_alloc(ctx, (void**)&p, fr.size() * 4), "hipMalloc frames");
         hipFree(j.dFrames);
         j.dFrames = p;
         j.framesCap = fr.size() * 4;
@@ -511,6 +534,7 @@ cr_status cr_batch_render(cr_context* ctx)
         std::vector<Group> groups;
         const float4* samples = b->dSamples;
         bool moved = false;
+        const SamplesBusy busy(b);
         cr_status st = build_groups(ctx, b, table_order(b), b->tuning, nullptr, 0, &table, &groups);
         if (st == CR_OK) st = upload_table(ctx, &b->dTable, &b->tableCap, table, &moved);
         if (st != CR_OK) return st;

@@ -241,9 +241,13 @@ cr_status continue_pass(cr_context* ctx, const float* pts, uint32_t m, uint32_t 
     a.counters = nullptr;
     uint32_t group = spp;
     if (spp > 1) {
-        group = (uint32_t)std::min<uint64_t>(spp, std::max<uint64_t>(1, PT_SAMPLE_BUDGET / m));
-        if (sample_buffer(&ctx->ptSamples, &ctx->ptSamplesCap, (uint64_t)m * group)) a.samples = ctx->ptSamples;
-        else group = spp;
+        const uint64_t most = std::min<uint64_t>(spp, std::max<uint64_t>(1, PT_SAMPLE_BUDGET / m));
+        const uint64_t room = sample_buffer(&ctx->ptSamples, &ctx->ptSamplesCap, m * most,
+                                            m * std::min<uint64_t>(most, PT_LEAST_STORED));
+        if (room) {
+            a.samples = ctx->ptSamples;
+            group = (uint32_t)(room / m);
+        }
     }
     for (uint32_t s0 = 0; s0 < spp; s0 += group) {
         a.sample0 = s0;
@@ -310,8 +314,8 @@ cr_status ensure_dataset(cr_context* ctx, Learn* L, uint64_t need)
     cap = std::max<uint64_t>(cap, 1u << 16);
     uint16_t* X = nullptr;
     float* T = nullptr;
-    CR_HIP(ctx, hipMalloc((void**)&X, cap * 448), "hipMalloc data set");
-    hipError_t e = hipMalloc((void**)&T, cap * 12);
+    CR_HIP(ctx, device_alloc(ctx, (void**)&X, cap * 448), "hipMalloc data set");
+    hipError_t e = device_alloc(ctx, (void**)&T, cap * 12);
     if (e != hipSuccess) {
         hipFree(X);
         return hip_fail(ctx, e, "hipMalloc data set");

@@ -40,6 +40,7 @@ struct Ppb {
     size_t overflowCap = 0;
     // beam producer: records of the last trace, per-path counts and offsets
     BeamRecord* records = nullptr;
+    bool tracing = false;           // records in use
     unsigned long long* recordCount = nullptr;
     uint32_t* pathCounts = nullptr;
     uint64_t* pathOffsets = nullptr;
@@ -98,19 +99,31 @@ static const uint32_t MAX_BEAMS = 1u << 28;
 static const uint64_t TRACE_PATHS = 1u << 18;            // photon paths per launch of the producer at most
 static const size_t TRACE_KEEP = (size_t)1 << 30;        // bytes of beam records kept between traces at most
 
+static bool free_records(Ppb* p)
+{
+    if (!p->records) return false;
+    hipFree(p->records);
+    p->records = nullptr;
+    p->recordsCap = 0;
+    return true;
+}
+
 namespace {
-// Gives the records of a large trace back, whichever way it ends.
-struct TrimRecords {
+// A trace's hold on its records; those of a large trace go back, whichever way it ends.
+struct TraceRecords {
     Ppb* p;
-    ~TrimRecords()
+    explicit TraceRecords(Ppb* state) : p(state) { p->tracing = true; }
+    ~TraceRecords()
     {
-        if (p->recordsCap <= TRACE_KEEP) return;
-        hipFree(p->records);
-        p->records = nullptr;
-        p->recordsCap = 0;
+        p->tracing = false;
+        if (p->recordsCap > TRACE_KEEP) free_records(p);
     }
 };
 } // namespace
+
+namespace cr {
+bool ppb_release_records(cr_context* ctx) { return ctx->ppb && !ctx->ppb->tracing && free_records(ctx->ppb); }
+} // namespace cr
 
 // Sort, tree and traversal buffers for n beams (grown, never shrunk).
 static cr_status lbvh_buffers(cr_context* ctx, Ppb* p, uint32_t n)
@@ -194,7 +207,7 @@ cr_status cr_ppb_trace_beams(cr_context* ctx, const cr_beam_trace_params* prm, u
     hipSetDevice(ctx->device);
     Ppb* p;
     CR_TRY(ppb_get(ctx, &p));
-    const TrimRecords trim{p};
+    const TraceRecords hold(p);
     const uint32_t P = prm->numPaths;
     const DeviceGrid& g = ctx->grid;
     TraceArgs a;
@@ -250,7 +263,7 @@ cr_status cr_ppb_trace_beams(cr_context* ctx, const cr_beam_trace_params* prm, u
             if (e != hipSuccess) {  // no room for more than these
                 (void)hipGetLastError();
                 bytes = (size_t)total * sizeof(BeamRecord);
-                e = hipMalloc((void**)&more, bytes);
+                e = device_alloc(ctx, (void**)&more, bytes);
             }
             if (e != hipSuccess) return fail(ctx, CR_ERR_OUT_OF_MEMORY, std::string("hipMalloc beam records: ") + hipGetErrorString(e));
             if (records) e = hipMemcpyAsync(more, p->records, (size_t)records * sizeof(BeamRecord), hipMemcpyDeviceToDevice, ctx->stream);
@@ -392,7 +405,7 @@ cr_status cr_lbvh_download(cr_context* ctx, uint32_t* morton_sorted, uint32_t* p
     if (nodes) {
         cr_tree_node* tmp = nullptr;
         const size_t bytes = (2 * (size_t)n - 1) * sizeof(cr_tree_node);
-        CR_HIP(ctx, hipMalloc((void**)&tmp, bytes), "hipMalloc nodes");
+        CR_HIP(ctx, device_alloc(ctx, (void**)&tmp, bytes), "hipMalloc nodes");
         hipError_t e = launch_treenodes(n, p->meta, p->leafParent, p->lo, p->hi, tmp, s);
         if (e == hipSuccess) e = hipMemcpyAsync(nodes, tmp, bytes, hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);

@@ -24,6 +24,7 @@ struct Ppm {
     uint32_t *pathCounts = nullptr, *pathOffsets = nullptr;
     size_t pathCountsCap = 0, pathOffsetsCap = 0;
     PpmRecord* records = nullptr;   // deposits as the paths left them
+    bool tracing = false;           // records in use
     uint2* chunks = nullptr;
     unsigned long long* chunkCount = nullptr;
     size_t recordsCap = 0, chunksCap = 0, chunkCountCap = 0;
@@ -66,19 +67,31 @@ static Ppm* ppm_get(cr_context* ctx)
 static const uint32_t MAX_DEPOSITS = 1u << 28;
 static const size_t RECORDS_KEEP = (size_t)1 << 30;   // bytes of deposit records kept between traces at most
 
+static bool free_records(Ppm* p)
+{
+    if (!p->records) return false;
+    hipFree(p->records);
+    p->records = nullptr;
+    p->recordsCap = 0;
+    return true;
+}
+
 namespace {
-// Gives the records of a large trace back, whichever way it ends.
-struct TrimRecords {
+// A trace's hold on its records; those of a large trace go back, whichever way it ends.
+struct TraceRecords {
     Ppm* p;
-    ~TrimRecords()
+    explicit TraceRecords(Ppm* state) : p(state) { p->tracing = true; }
+    ~TraceRecords()
     {
-        if (p->recordsCap <= RECORDS_KEEP) return;
-        hipFree(p->records);
-        p->records = nullptr;
-        p->recordsCap = 0;
+        p->tracing = false;
+        if (p->recordsCap > RECORDS_KEEP) free_records(p);
     }
 };
 } // namespace
+
+namespace cr {
+bool ppm_release_records(cr_context* ctx) { return ctx->ppm && !ctx->ppm->tracing && free_records(ctx->ppm); }
+} // namespace cr
 
 static const uint64_t MAX_CELLS = 1ull << 27;
 
@@ -186,7 +199,7 @@ cr_status cr_ppm_trace(cr_context* ctx, int32_t seed, const cr_ppm_params* prm, 
     if (!ctx->hasPm) return fail(ctx, CR_ERR_STATE, "no photon map properties (cr_set_photon_map)");
     hipSetDevice(ctx->device);
     Ppm* p = ppm_get(ctx);
-    const TrimRecords trim{p};
+    const TraceRecords hold(p);
     p->valid = false;
     const uint32_t P = prm->numPaths;
     const uint64_t nCells = (uint64_t)ctx->pm.voxelCount[0] * ctx->pm.voxelCount[1] * ctx->pm.voxelCount[2];

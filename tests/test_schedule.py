@@ -36,3 +36,22 @@ def test_chunks(evaluate):
              (1, 1, 8, 4, 1), (1 << 28, 0xFFFFFFFF, 8, 4, 4)]
     got = evaluate(*(f"pt_chunk({px}, {n}u, {lanes}, {per}, {most})" for px, n, per, most, _ in cases))
     assert got == [w for *_, w in cases]
+
+
+def test_sample_room(evaluate):
+    # a device with room for `free` samples; the attempts made are counted
+    before = """
+static int tries;
+static long long room(unsigned long long want, unsigned long long least, unsigned long long had, unsigned long long free)
+{
+    tries = 0;
+    return (long long)pt_sample_room(want, least, had, [&](uint64_t n) { tries++; return n <= free; });
+}
+"""
+    cases = [((1000, 20, 0, 5000), 1000), ((1000, 20, 0, 1000), 1000), ((1000, 20, 0, 600), 500), ((1000, 20, 0, 30), 20),
+             ((1000, 20, 0, 20), 20), ((1000, 20, 0, 19), 0), ((1000, 1000, 0, 999), 0),
+             # what was held before is tried once it is the next smaller size
+             ((1000, 20, 700, 700), 700), ((1000, 20, 700, 400), 350), ((1000, 20, 300, 300), 300), ((1000, 20, 300, 499), 300),
+             ((1, 1, 0, 0), 0), ((1 << 28, 2, 0, 0), 0)]
+    got = evaluate(*(f"room({w}u, {l}u, {h}u, {f}u)" for (w, l, h, f), _ in cases), before=before)
+    assert got == [v for _, v in cases]
