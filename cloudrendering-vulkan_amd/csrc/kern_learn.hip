@@ -33,10 +33,15 @@ __global__ void __launch_bounds__(256) mip_kernel(const float* src, int32_t sx, 
     dst[(size_t)x + (size_t)dx * ((size_t)y + (size_t)dy * z)] = fdiv(acc, cnt);
 }
 
-// The coarsest mip levels, as many as fit in this many floats (18.4 KB), are
-// copied into LDS by each workgroup: for a 128^3 grid, levels 3-7 (16^3 down
-// to 1^3), whose taps are 135 of a record's 216.
-constexpr uint32_t FEATURE_LDS_FLOATS = 4736;
+// The coarsest mip levels, as many as fit in this many floats (32 KB), are copied
+// into LDS by each workgroup: for a 128^3 grid, levels 3-7 (16^3 down to 1^3),
+// whose taps are 135 of a record's 216.  The kernel's 126 vector registers allow
+// four waves per SIMD, four workgroups per CU, and four times 32 KB fit in its LDS
+// with room to spare; half the size costs grids of 33-38, 65-76, 129-152 and
+// 257-304 voxels a level and helps no other (learned renders at 1080p and 16 spp
+// with 18.5 and 32 KB: 17.8 and 17.3 ms at 36^3, 15.7 and 15.7 at 72^3, 12.5 and
+// 12.5 at 128^3, 12.5 and 12.2 at 144^3, 12.1 and 12.1 at 200^3).
+constexpr uint32_t FEATURE_LDS_FLOATS = 8192;
 
 __device__ __forceinline__ uint32_t mip_floats(const cr::FeatureArgs& a, int k)
 {
