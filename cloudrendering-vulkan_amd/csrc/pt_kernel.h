@@ -201,6 +201,15 @@ __device__ __forceinline__ float2 brick_skip(const cr::PTArgs& a, uint32_t brick
     return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(a.skip) + (brick << 3));
 }
 
+// The generator's state 0 draws nothing but 0, whose flights -log 0 are infinite: a
+// path that starts with it crosses the box without a collision.  No other state
+// ever becomes 0.  With the global majorant such a sample ends where it starts; the
+// brick walk, which counts the bricks it crosses, takes the flight as infinite.
+// (A select on the state in every segment of the global majorant's tracker cost
+// registers: FP32 grids with ratio tracking 96 -> 98 and a wave per SIMD.)
+template <int TRACK>
+__device__ __forceinline__ bool stuck(const Lane& L) { return TRACK != CR_TRACK_BRICK_DDA && L.rng == 0u; }
+
 // Start a tracking segment from L.pos along `dir` (primary or shadow); invd =
 // 1 / dir.  Returns false when the segment misses the box (no RNG draw is made
 // then, as findScatterPoint returns before tracking, PathTracer.comp:321-324).
@@ -211,16 +220,11 @@ __device__ __forceinline__ bool begin_segment(const cr::PTArgs& a, Lane& L, f3 d
     if (!intersect_box_inv(B0(a), B1(a), L.pos, invd, tmin, tmax)) return false;
     f3 exitp = add(L.pos, mul(dir, tmax));
     L.dist = length(sub(L.pos, exitp));
-    // The state 0 draws nothing but 0, whose flights -log 0 are infinite: such a
-    // path leaves every segment.  No other state ever becomes 0, so this is the
-    // one place that has to look (one select per segment).
+    L.t = 0.0f;
     if (TRACK == CR_TRACK_BRICK_DDA) {
-        L.t = 0.0f;
         dda_init(a, L.pos, dir, invd, L);
         const float tau = -crd_log_normal(xs_float(L.rng));
         L.tau = L.rng != 0u ? tau : __builtin_inff();
-    } else {
-        L.t = L.rng != 0u ? 0.0f : __builtin_inff();
     }
     return true;
 }
@@ -744,6 +748,8 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
                 } else if (L.camMiss) {
                     sky = true;
                     missed = true;
+                } else if (stuck<TRACK>(L)) {
+                    sky = true;
                 } else {
                     seg = 1;
                 }
@@ -812,6 +818,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
                         missed = true;
                     } else {
                         L.pos = add(L.pos, mul(L.dir, tmax < tmin ? tmax : tmin));
+                        sky = stuck<TRACK>(L);
                     }
                 }
             }
