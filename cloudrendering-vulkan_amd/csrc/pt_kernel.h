@@ -510,11 +510,13 @@ __device__ __forceinline__ uint32_t part_first(uint32_t part, uint32_t logParts)
 }
 
 // Waves per SIMD the registers are to allow (1: no demand).  Renders of FP32
-// grids with brick tracking take 103 registers unasked and run as well with the
-// 96 that five waves leave each (1080p at 64 spp: 71.3 ms with four waves of
-// either code, 65.9 with five); FP16 grids and the global majorant lose more in
-// the tighter code than the fifth wave brings (1 GiB FP16 grid 326 ms against
-// 404, shadow-volume NEE at 256x256 3.09 against 3.59).
+// grids with brick tracking run in the 96 registers that five waves leave each:
+// with ratio tracking, 103 unasked, 1080p at 64 spp takes 71.3 ms with four waves
+// of either code and 65.9 with five; with shadow-volume NEE and without NEE a few
+// registers may spill (up to 6) and the fifth wave is worth more: 38.1 -> 35.8 and
+// 34.2 -> 30.8 ms, in bricks 38.3 -> 36.4 and 34.6 -> 30.7.  FP16 grids and the
+// global majorant lose more in the tighter code than the fifth wave brings (1 GiB
+// FP16 grid 326 ms against 404, shadow-volume NEE at 256x256 3.09 against 3.59).
 template <typename T, int TRACK, bool BATCH, int KMODE>
 constexpr int min_waves()
 {
