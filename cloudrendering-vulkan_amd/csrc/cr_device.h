@@ -543,12 +543,15 @@ __device__ __forceinline__ f3 sv_norm(const cr_shadow_volume_properties& s, f3 p
     return mk(r[0], r[1], r[2]);
 }
 
+// RESIDUAL: by div3, else by the divide sequence.
+template <bool RESIDUAL = true>
 __device__ __forceinline__ f3 sv_norm(const SvMap& s, f3 p)
 {
     const float v0 = p.x - s.org[0], v1 = p.y - s.org[1], v2 = p.z - s.org[2];
     float num[3];
 #pragma unroll
     for (int i = 0; i < 3; i++) num[i] = ((s.m[i][0] * v0 + s.m[i][1] * v1) + s.m[i][2] * v2) + s.c[i];
+    if (!RESIDUAL) return mk(fdiv(num[0], s.den.d[0]), fdiv(num[1], s.den.d[1]), fdiv(num[2], s.den.d[2]));
     return div3(s.den, mk(num[0], num[1], num[2]));
 }
 

@@ -103,7 +103,8 @@ constexpr uint32_t PT_QUEUE_STRIDE = 64, PT_QUEUE_WORDS = 8 * PT_QUEUE_STRIDE;
 // (In one copy the 4096 waves of a launch waited 280 us for each other at its
 // end: 512x512 at 1 spp 1.28 ms against 1.01.)
 constexpr uint32_t COUNTER_SLOTS = 64, COUNTER_STRIDE = 32, COUNTER_WORDS = COUNTER_SLOTS * COUNTER_STRIDE;
-hipError_t launch_pt(const PTArgs& a, int dtype, int layout, int grid_blocks, hipStream_t s);
+// (whole-pixel launches of at most one workgroup per CU, `cus`, go out as single waves)
+hipError_t launch_pt(const PTArgs& a, int dtype, int layout, int grid_blocks, int cus, hipStream_t s);
 int pt_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee, uint32_t chunk);
 // The tile list of a render (lists: pt_list_words(a) words; the list ends where
 // the nine part starts begin, at pt_list_starts(a)).  The image is cut into

@@ -864,7 +864,7 @@ cr_status cr_pt_render(cr_context* ctx, const cr_push_constants* frames, uint32_
         if ((uint32_t)blocks > needed) blocks = (int)needed;
         if (ctx->ptBlocksOverride > 0) blocks = ctx->ptBlocksOverride;
         if (f0) CR_HIP(ctx, zero_async(ctx->dQueue, PT_QUEUE_WORDS * 4, ctx->stream), "zero queue");
-        CR_HIP(ctx, launch_pt(b, g.dtype, g.layout, blocks, ctx->stream), "path tracer kernel");
+        CR_HIP(ctx, launch_pt(b, g.dtype, g.layout, blocks, ctx->numCUs, ctx->stream), "path tracer kernel");
         if (b.samples) CR_HIP(ctx, launch_pt_blend(b, ctx->stream), "blend kernel");
     }
     CR_HIP(ctx, hipEventRecord(ev.second, ctx->stream), "event");

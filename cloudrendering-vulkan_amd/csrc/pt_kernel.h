@@ -110,11 +110,13 @@ __device__ __forceinline__ float sample_cloud(const cr::PTArgs& a, f3 p)
     return trilinear<T, LAYOUT, PAIRS && sizeof(T) == 4>(g, cloud_norm(a.box, p));
 }
 
+template <bool WHOLE>
 __device__ __forceinline__ float sample_sv(const cr::PTArgs& a, f3 p)
 {
     GridView g;
     g.data = a.sv; g.nx = a.svx; g.ny = a.svy; g.nz = a.svz; g.nbx = 0; g.nby = 0;
-    return trilinear<float, LAYOUT_DENSE, true>(g, sv_norm(a.svMap, p));
+    if (WHOLE) return trilinear<float, LAYOUT_DENSE>(g, sv_norm<false>(a.svMap, p));
+    return trilinear<float, LAYOUT_DENSE, true>(g, sv_norm<true>(a.svMap, p));
 }
 
 // Per lane and axis, for the lane's current segment (written once per segment
@@ -234,8 +236,10 @@ enum : uint32_t { EV_NONE = 0, EV_COLLIDE = 1, EV_EXIT = 2 };
 // One tracking step: at most one density lookup.  Primary mode: delta
 // tracking (PathTracer.comp:335-355); shadow mode: ratio tracking.
 // WHOLE: passes of whole pixels of many frames are bound by the latency of one
-// path's chain, where the divide sequence and eight loads end sooner than uniform
-// branches and selects (68x68 pixels at 53 spp 14.6 ms, 16.1 with the others).
+// path's chain while the image is small, where the divide sequence and eight loads
+// end sooner than uniform branches and selects (shadow-volume NEE, 68x68 pixels at
+// 53 spp 3.8 ms, 4.2 with the others; ratio tracking 12.2 and 13.3; at 256x256 they
+// even out and at 1080p and 64 spp the others gain, 98 to 83 and 98 to 97).
 template <typename T, int LAYOUT, int TRACK, bool WHOLE>
 __device__ __forceinline__ uint32_t track_step(const cr::PTArgs& a, Lane& L, f3 sdir, Counters& c)
 {
@@ -538,6 +542,18 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
         for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
         __syncthreads();
     }
+    // Passes of whole pixels have every argument of the tracker in registers (or
+    // spilled to lanes of one): the compiler would load some of them again in every
+    // step (1080p, 32 spp, FP16 and ratio tracking with the global majorant 128.7 ->
+    // 112.8 ms).
+    constexpr bool WHOLE = KMODE == K_RENDER && !BATCH;
+    cr::PTArgs held = a0;
+    if (WHOLE) {
+        asm volatile("" : "+s"(held.grid));
+        asm volatile("" : "+s"(held.nx));
+        asm volatile("" : "+s"(held.cloud.maxExtinction));
+    }
+    const cr::PTArgs& single = WHOLE ? held : a0;
     uint32_t* const queue = BATCH ? b.queue : a0.queue;
     Lane L;
     Counters c = {0, 0, 0, 0, 0};
@@ -550,17 +566,25 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
     // The work items come in parts, one per XCD (workgroup b runs on XCD b mod 8)
     // or one in all: the waves of an XCD work on the same regions of the image,
     // whose rays share its L2, and go on to the next part when theirs is drained.
-    const uint32_t logParts = BATCH ? b.logParts : a0.logParts;
+    // (Passes of whole pixels take them as one: they have no more than a few items
+    // per wave.)
+    const uint32_t logParts = BATCH ? b.logParts : (WHOLE ? 0u : a0.logParts);
     uint32_t part = blockIdx.x & ((1u << logParts) - 1u), partsLeft = 1u << logParts;
     uint32_t partAt, partEnd;
-    part_range<BATCH, KMODE>(b, part, logParts, partAt, partEnd);
+    if (WHOLE) {
+        partAt = 0u;
+        partEnd = a0.partStart ? a0.partStart[8] * 64u : a0.totalIdx;
+    } else {
+        part_range<BATCH, KMODE>(b, part, logParts, partAt, partEnd);
+    }
     // In renders each wave's first 64 items are set by its number in the part and
     // the queue deals out those after them: the waves of a launch need not wait
     // for each other's atomics (512x512 at 1 spp 1.00 -> 0.93 ms).
     constexpr bool FIRST_SET = renders(KMODE) && !BATCH;
-    const uint32_t first = partAt + (((blockIdx.x >> logParts) * 4u + (threadIdx.x >> 6)) << 6);
+    const uint32_t waves = WHOLE ? blockDim.x >> 6 : 4u;   // of a workgroup
+    const uint32_t first = partAt + (((blockIdx.x >> logParts) * waves + (threadIdx.x >> 6)) << 6);
     bool started = !FIRST_SET;
-    if (FIRST_SET) partAt += part_first(part, logParts);
+    if (FIRST_SET) partAt += WHOLE ? gridDim.x * blockDim.x : part_first(part, logParts);
 
     for (;;) {
         // ---- claim pixels for idle lanes (wave-wide, one atomic per wave)
@@ -580,9 +604,11 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
                 }
                 end = partEnd;
                 if (started && at + n >= end) {
-                    part = (part + 1u) & ((1u << logParts) - 1u);
-                    part_range<BATCH, KMODE>(b, part, logParts, partAt, partEnd);
-                    if (FIRST_SET) partAt += part_first(part, logParts);
+                    if (!WHOLE) {
+                        part = (part + 1u) & ((1u << logParts) - 1u);
+                        part_range<BATCH, KMODE>(b, part, logParts, partAt, partEnd);
+                        if (FIRST_SET) partAt += part_first(part, logParts);
+                    }
                     partsLeft--;
                 }
                 started = true;
@@ -651,14 +677,14 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
         if (__ballot(state != ST_DEAD) == 0ull) break;
         if (state != ST_ACTIVE) continue;
 
-        const cr::PTArgs& a = BATCH ? jobs[L.job] : a0;
+        const cr::PTArgs& a = BATCH ? jobs[L.job] : single;
         const f3 ldir = ld3(a.lightDirection);
         const f3 sdir = neg(ldir);
         const float I = a.params.lightIntensity;
         const float albedo = a.ext.albedo;
         const uint32_t cap = a.ext.bounceCap;
 
-        if (ev == EV_NONE && L.mode != 0xFFu) ev = track_step<T, LAYOUT, TRACK, KMODE == K_RENDER && !BATCH>(a, L, sdir, c);
+        if (ev == EV_NONE && L.mode != 0xFFu) ev = track_step<T, LAYOUT, TRACK, WHOLE>(a, L, sdir, c);
 
         // ---- divergent tail: events that need no lookup are resolved here,
         // possibly several in a row (e.g. a camera ray that misses the box).
@@ -792,7 +818,7 @@ __global__ void __launch_bounds__(256, (min_waves<T, TRACK, BATCH, KMODE>())) pt
                     } else {
                         float Tv;
                         if (NEE == CR_NEE_SHADOW_VOLUME) {
-                            Tv = sample_sv(a, L.pos);
+                            Tv = sample_sv<WHOLE>(a, L.pos);
                             c.svLookups++;
                         } else {
                             Tv = 0.0f;

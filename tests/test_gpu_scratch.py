@@ -74,3 +74,23 @@ def test_samples_make_way(pkg, cfg, S, batch):
     else:
         assert_bitexact(few, render(), "image")
     ctx.close()
+
+
+def test_no_room_for_samples(pkg, cfg, S):
+    """Room for less than two frames: whole pixels, from the list of the tiles."""
+    w = h = 8192
+    frames = cfg.frames(20, first=1)
+    ctx = pkg.Context(0)
+    sc = cfg.c1(width=w, height=h, size=32, sv_axis=32)
+    sc.cam = cfg.camera(w, h, position=(0.0, 0.0, -3.0))
+    sc.setup(ctx)
+    full = Full(3 * GIB // 2)               # two frames of samples are 2 GiB
+    try:
+        ctx.pt_render(frames)
+        whole = ctx.download_image(h, w)
+    finally:
+        full.release()
+    ctx.clear_image()
+    ctx.pt_render(frames)
+    assert_bitexact(whole, ctx.download_image(h, w), "image")
+    ctx.close()
