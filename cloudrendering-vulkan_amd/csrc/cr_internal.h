@@ -94,7 +94,8 @@ struct BatchArgs {
 
 // kern_pt.hip: a render of a.nFrames frames; launches whose work items hold
 // at most PT_FEW_FRAMES frames use the instantiation with gated pixel claims
-// (kern_pt_few.hip), which is faster when an item carries little work.
+// (kern_pt_few.hip), which is faster when an item carries little work, unless
+// the items are whole pixels for no more than a wave per SIMD.
 // Atomics on one cache line are carried out one by one, some 14 ns each: the
 // parts' queue words lie 256 bytes apart.
 constexpr uint32_t PT_QUEUE_STRIDE = 64, PT_QUEUE_WORDS = 8 * PT_QUEUE_STRIDE;
@@ -103,7 +104,7 @@ constexpr uint32_t PT_QUEUE_STRIDE = 64, PT_QUEUE_WORDS = 8 * PT_QUEUE_STRIDE;
 // (In one copy the 4096 waves of a launch waited 280 us for each other at its
 // end: 512x512 at 1 spp 1.28 ms against 1.01.)
 constexpr uint32_t COUNTER_SLOTS = 64, COUNTER_STRIDE = 32, COUNTER_WORDS = COUNTER_SLOTS * COUNTER_STRIDE;
-// (whole-pixel launches of at most one workgroup per CU, `cus`, go out as single waves)
+// cus: the device's CUs.
 hipError_t launch_pt(const PTArgs& a, int dtype, int layout, int grid_blocks, int cus, hipStream_t s);
 int pt_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee, uint32_t chunk);
 // The tile list of a render (lists: pt_list_words(a) words; the list ends where

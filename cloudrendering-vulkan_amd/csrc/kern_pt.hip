@@ -199,19 +199,18 @@ hipError_t launch_pt_sum(const PTArgs& a, uint32_t total, hipStream_t s)
 
 hipError_t launch_pt(const PTArgs& a, int dtype, int layout, int blocks, int cus, hipStream_t s)
 {
-    if (a.chunk <= PT_FEW_FRAMES) return launch_pt_few(a, dtype, layout, blocks, s);
-    BatchArgs none = {};
-    int threads = 256;
     // No more than a wave per SIMD: workgroups of one wave, dealt over the whole
     // chip, where four neighbouring tiles of one workgroup would share a CU (256x256
     // at 64 spp, brick tracking 58.4 -> 55.5 ms, 128x128 at 32 spp with the shadow
     // volume 5.8 -> 5.4; beyond that neighbours sharing a cache are worth more,
-    // 512x512 at 64 spp 16.9 ms against 21.7).
-    if (blocks <= cus) {
-        blocks = (int)std::min<uint32_t>(4u * (uint32_t)blocks, (a.totalIdx + 63u) / 64u);
-        threads = 64;
-    }
-    return launch(pick<false, K_RENDER>(dtype, layout, a.ext.trackingMode, a.ext.neeMode), a, none, blocks, threads, 0, s);
+    // 512x512 at 64 spp 16.9 ms against 21.7), and the kernel of whole pixels however
+    // few their frames (256x256 with the shadow volume, 4 frames 0.94 -> 0.80 ms, one
+    // frame 0.27 -> 0.24).
+    const bool sparse = blocks <= cus && !a.samples;
+    if (a.chunk <= PT_FEW_FRAMES && !sparse) return launch_pt_few(a, dtype, layout, blocks, s);
+    BatchArgs none = {};
+    if (sparse) blocks = (int)std::min<uint32_t>(4u * (uint32_t)blocks, (a.totalIdx + 63u) / 64u);
+    return launch(pick<false, K_RENDER>(dtype, layout, a.ext.trackingMode, a.ext.neeMode), a, none, blocks, sparse ? 64 : 256, 0, s);
 }
 
 int pt_blocks_per_cu(int dtype, int layout, uint32_t tracking, uint32_t nee, uint32_t chunk)

@@ -366,10 +366,9 @@ __device__ __forceinline__ void blend(const cr::PTArgs& a, Lane& L)
 }
 
 // What a launch computes per work item.
-//   K_RENDER   : pixels, frames blended into the image (the reference's pass).
-//   K_RENDER_FEW: the same for launches of a few frames per pixel (the
-//                reference's interactive loop renders one), with claims gated
-//                as in K_RECORD.
+//   K_RENDER   : whole pixels, frames blended into the image (the reference's pass).
+//   K_RENDER_FEW: the same for work items of a few frames (the reference's
+//                interactive loop renders one), with claims gated as in K_RECORD.
 //   K_RECORD   : pixels; each frame's camera path stops at its first real
 //                collision, which is recorded as (position, direction, RNG
 //                state, flag 1), or, for a path that escapes before any
