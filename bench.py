@@ -72,7 +72,7 @@ def log(msg):
 
 
 # the sources that define the path-tracing kernel's code
-PT_SOURCES = ("pt_kernel.h", "cr_device.h", "cr_internal.h", "kern_pt.hip")
+PT_SOURCES = ("pt_kernel.h", "cr_device.h", "cr_internal.h", "pt_schedule.h", "kern_pt.hip")
 LBVH_SOURCES = ("kern_lbvh.hip", "cr_internal_ppb.h", "cr_device.h")
 
 

@@ -359,7 +359,7 @@ constexpr uint32_t STACK_LDS = 24;  //   of them in LDS, deeper ones in scratch 
 // with the tests in the walk, 12.6 with the queues, and 8.5 with 16 instead of
 // 32 lanes to start a stage, four waves per SIMD and 8x8 instead of 16x4
 // pixels per wave (stages at 8, 24, 32 or 48 lanes, queues of 16, and 3 or 5
-// waves are within 3% or slower).
+// waves are within 3% or slower); under other suns such frames take 9.2-11.1.
 constexpr uint32_t FOUND = 8, PASSED = 4;                    // queue lengths (powers of two)
 constexpr uint32_t FOUND_LANES = 16, PASSED_LANES = 16;      // lanes with work that start a stage
 template <typename T, int LAYOUT>
