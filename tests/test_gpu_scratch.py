@@ -17,10 +17,13 @@ class Full:
     def __init__(self, left):
         self.hip = C.CDLL("libamdhip64.so.7")
         self.held = []
-        while self.free() > left + (256 << 20):
+        size = 64 * GIB
+        while self.free() > left + (256 << 20) and size >= 256 << 20:
             p = C.c_void_p()
-            assert self.hip.hipMalloc(C.byref(p), C.c_size_t(min(self.free() - left, 64 * GIB))) == 0
-            self.held.append(p)
+            if self.hip.hipMalloc(C.byref(p), C.c_size_t(min(self.free() - left, size))) == 0:
+                self.held.append(p)
+            else:
+                size //= 2      # no piece of that size is free
 
     def free(self):
         f, t = C.c_size_t(), C.c_size_t()
